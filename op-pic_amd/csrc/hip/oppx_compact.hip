@@ -8,7 +8,8 @@
 //   #holes below index v        = wp[v/64] + popcount(word & low bits)      (wp = word prefix)
 //   rank of live v >= S from top = (N-1-v) - (R - #holes below v)
 // so every live tail record finds its destination hole by a binary search over wp and a
-// select inside one word. Passes: block popcounts -> scan -> word prefix -> tail copy -> finalize.
+// select inside one word. Two launches: the word prefixes inside each block of words and the block counts;
+// then the tail copy, whose blocks scan the block counts themselves and one of which writes the counters.
 
 #include <mutex>
 
@@ -24,13 +25,15 @@ namespace {
 
 constexpr int kB = 256;
 constexpr int kMaxDats = 16;
+constexpr int kMaxComps = 64;   // components one fill launch moves (more take further launches)
+constexpr int kMaxGroups = 4096;  // group prefixes a fill block holds in LDS
+constexpr int kCopyBatch = 8;   // components loaded before any of them is stored
 
-struct DatTable {
+// The dats as single components: base address of each, and which of them have 8-byte elements.
+struct CompTable {
     int n;
-    int64_t stride;
-    void* base[kMaxDats];
-    int dim[kMaxDats];
-    int eb[kMaxDats];
+    uint64_t wide;
+    void* base[kMaxComps];
 };
 
 __device__ __forceinline__ int64_t words_of(int64_t n) { return (n + 63) >> 6; }
@@ -63,98 +66,121 @@ __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* t
     return off + inc - v;
 }
 
-__global__ void __launch_bounds__(kB) hf_block_sums(const uint64_t* __restrict__ bits,
-                                                    const oppx_move_counters* __restrict__ ctr,
-                                                    uint32_t* __restrict__ bsum, int64_t n_max) {
-    const int64_t W = words_of(live_count(ctr, n_max));
-    const int64_t w = (int64_t)blockIdx.x * kB + threadIdx.x;
-    const uint32_t c = (w < W) ? (uint32_t)__popcll(bits[w]) : 0u;
-    uint32_t tot;
-    block_exclusive_scan(c, &tot);
-    if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
-}
-
-// single block of kB threads: exclusive scan of nb block sums in place; total = removed count
-__global__ void __launch_bounds__(kB) hf_scan_blocks(uint32_t* __restrict__ bsum, int64_t nb,
-                                                     oppx_move_counters* __restrict__ ctr) {
-    uint32_t carry = 0;
-    for (int64_t base = 0; base < nb; base += kB) {
-        const int64_t j = base + threadIdx.x;
-        const uint32_t v = (j < nb) ? bsum[j] : 0u;
-        uint32_t tot;
-        const uint32_t ex = block_exclusive_scan(v, &tot);
-        if (j < nb) bsum[j] = carry + ex;
-        carry += tot;
-    }
-    if (threadIdx.x == 0) ctr->removed = (int32_t)carry;
-}
-
-__global__ void __launch_bounds__(kB) hf_word_prefix(const uint64_t* __restrict__ bits,
-                                                     const oppx_move_counters* __restrict__ ctr,
-                                                     const uint32_t* __restrict__ bsum, uint32_t* __restrict__ wp,
-                                                     int64_t n_max) {
-    const int64_t W = words_of(live_count(ctr, n_max));
+// Removals of every bitmap word before it in its block of kB words (wp), of every block (bsum), and the
+// live count (head[0]): the fill reads the count from here, so that it may write the new one while its
+// other blocks still run.
+__global__ void __launch_bounds__(kB) hf_count(const uint64_t* __restrict__ bits,
+                                               const oppx_move_counters* __restrict__ ctr, uint32_t* __restrict__ bsum,
+                                               uint32_t* __restrict__ wp, uint32_t* __restrict__ head, int64_t n_max) {
+    const int64_t N = live_count(ctr, n_max), W = words_of(N);
     const int64_t w = (int64_t)blockIdx.x * kB + threadIdx.x;
     const uint32_t c = (w < W) ? (uint32_t)__popcll(bits[w]) : 0u;
     uint32_t tot;
     const uint32_t ex = block_exclusive_scan(c, &tot);
-    if (w < W) wp[w] = bsum[blockIdx.x] + ex;
+    if (w < W) wp[w] = ex;
+    if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
+    if (blockIdx.x == 0 && threadIdx.x == 0) head[0] = (uint32_t)N;
 }
 
-template <typename T>
-__device__ __forceinline__ void move_record(void* base, int dim, int64_t stride, int64_t from, int64_t to) {
-    T* p = reinterpret_cast<T*>(base);
-    for (int d = 0; d < dim; d++) p[d * stride + to] = p[d * stride + from];
-}
-
-__global__ void __launch_bounds__(kB) hf_fill_tail(const uint64_t* __restrict__ bits,
-                                                   const oppx_move_counters* __restrict__ ctr,
-                                                   const uint32_t* __restrict__ wp, DatTable T, int64_t n_max) {
-    const int64_t N = live_count(ctr, n_max), R = ctr->removed;
-    if (R <= 0 || R > N) return;
-    const int64_t S = N - R, W = words_of(N);
+// Every block scans the block counts into LDS itself (group e: blocks [e * per, (e + 1) * per)), then its
+// threads move the live records of the tail [S, N) to their holes. What bounds this is the chain of
+// dependent reads of one record (its hole's search, then the copy): a scan kernel, a word-prefix kernel and a
+// finalize kernel beside it cost a launch each, 4.5-5 us after a large kernel. Measured (kernel time, a few
+// percent removed), five launches before and these two: 4,000 particles 14.5 and 11.5 us, 1 M 38.9 and 23.7 us,
+// 24 M 64 and 48 us.
+__global__ void __launch_bounds__(kB) hf_fill(const uint64_t* __restrict__ bits, oppx_move_counters* __restrict__ ctr,
+                                              const uint32_t* __restrict__ bsum, const uint32_t* __restrict__ wp,
+                                              const uint32_t* __restrict__ head, CompTable T, int64_t nb, int per,
+                                              int finish) {
+    __shared__ uint32_t s_pre[kMaxGroups];
+    const int64_t N = head[0];
+    const int ng = (int)((nb + per - 1) / per);
+    for (int e = threadIdx.x; e < ng; e += kB) {
+        uint32_t c = 0;
+        for (int64_t b = (int64_t)e * per; b < (int64_t)(e + 1) * per && b < nb; b++) c += bsum[b];
+        s_pre[e] = c;
+    }
+    __syncthreads();
+    const int items = (ng + kB - 1) / kB;  // groups of one thread, consecutive
+    const int e0 = (int)threadIdx.x * items, e1 = e0 + items < ng ? e0 + items : ng;
+    uint32_t mine = 0, total;
+    for (int e = e0; e < e1; e++) mine += s_pre[e];
+    uint32_t run = block_exclusive_scan(mine, &total);
+    for (int e = e0; e < e1; e++) {
+        const uint32_t c = s_pre[e];
+        s_pre[e] = run;
+        run += c;
+    }
+    __syncthreads();
+    const int64_t R = total, S = N - R, W = words_of(N);
+    // removals before word w
+    auto before = [&](int64_t w) {
+        const int64_t b = w / kB;
+        const int e = (int)(b / per);
+        int64_t c = (int64_t)s_pre[e] + wp[w];
+        for (int64_t q = (int64_t)e * per; q < b; q++) c += bsum[q];
+        return c;
+    };
+    const bool some = R > 0 && R <= N;
+    if (finish && blockIdx.x == 0 && threadIdx.x == 0) {
+        ctr->removed = (int32_t)R;
+        if (some) {
+            const int j = (int)(S & 63);
+            const uint64_t lowmask = j ? ((1ull << j) - 1ull) : 0ull;
+            ctr->holes_low = (int32_t)(before(S >> 6) + __popcll(bits[S >> 6] & lowmask));
+            ctr->size = (int32_t)S;
+        } else {
+            ctr->holes_low = 0;
+        }
+    }
+    if (!some) return;
     for (int64_t v = S + (int64_t)blockIdx.x * kB + threadIdx.x; v < N; v += (int64_t)gridDim.x * kB) {
         const uint64_t word = bits[v >> 6];
         const int j = (int)(v & 63);
         if ((word >> j) & 1ull) continue;  // a hole itself
-        const int64_t below = (int64_t)wp[v >> 6] + __popcll(word & ((1ull << j) - 1ull));
-        const int64_t k = (N - 1 - v) - (R - below);
-        // k-th hole: largest word w with wp[w] <= k, then the (k - wp[w])-th set bit of it
-        int64_t lo = 0, hi = W - 1;
+        const int64_t k = (N - 1 - v) - (R - (before(v >> 6) + __popcll(word & ((1ull << j) - 1ull))));
+        // k-th hole: the last group, block and word with at most k removals before it, then the set bit
+        int glo = 0, ghi = ng - 1;
+        while (glo < ghi) {
+            const int mid = (glo + ghi + 1) >> 1;
+            if ((int64_t)s_pre[mid] <= k) glo = mid;
+            else ghi = mid - 1;
+        }
+        int64_t b = (int64_t)glo * per, left = k - (int64_t)s_pre[glo];
+        while (b + 1 < nb && b + 1 < (int64_t)(glo + 1) * per && (int64_t)bsum[b] <= left) left -= bsum[b++];
+        int64_t lo = b * kB, hi = (b + 1) * kB < W ? (b + 1) * kB - 1 : W - 1;
         while (lo < hi) {
             const int64_t mid = (lo + hi + 1) >> 1;
-            if ((int64_t)wp[mid] <= k) lo = mid;
+            if ((int64_t)wp[mid] <= left) lo = mid;
             else hi = mid - 1;
         }
         uint64_t hw = bits[lo];
-        for (int64_t r = k - (int64_t)wp[lo]; r > 0 && hw; r--) hw &= hw - 1ull;
+        for (int64_t r = left - (int64_t)wp[lo]; r > 0 && hw; r--) hw &= hw - 1ull;
         if (hw == 0ull) continue;  // inconsistent bitmap: never write outside [0, S)
         const int64_t h = lo * 64 + (__ffsll((long long)hw) - 1);
         if (h < 0 || h >= S) continue;
-        for (int q = 0; q < T.n; q++) {
-            if (T.eb[q] == 8) move_record<double>(T.base[q], T.dim[q], T.stride, v, h);
-            else move_record<int32_t>(T.base[q], T.dim[q], T.stride, v, h);
+        for (int c0 = 0; c0 < T.n; c0 += kCopyBatch) {
+            uint64_t x[kCopyBatch];
+#pragma unroll
+            for (int u = 0; u < kCopyBatch; u++) {
+                if (c0 + u >= T.n) continue;
+                if ((T.wide >> (c0 + u)) & 1ull) x[u] = reinterpret_cast<const uint64_t*>(T.base[c0 + u])[v];
+                else x[u] = reinterpret_cast<const uint32_t*>(T.base[c0 + u])[v];
+            }
+#pragma unroll
+            for (int u = 0; u < kCopyBatch; u++) {
+                if (c0 + u >= T.n) continue;
+                if ((T.wide >> (c0 + u)) & 1ull) reinterpret_cast<uint64_t*>(T.base[c0 + u])[h] = x[u];
+                else reinterpret_cast<uint32_t*>(T.base[c0 + u])[h] = (uint32_t)x[u];
+            }
         }
     }
-}
-
-__global__ void hf_finalize(const uint64_t* __restrict__ bits, oppx_move_counters* __restrict__ ctr,
-                            const uint32_t* __restrict__ wp, int64_t n_max) {
-    const int64_t N = live_count(ctr, n_max), R = ctr->removed;
-    if (R <= 0 || R > N) {
-        ctr->holes_low = 0;
-        return;
-    }
-    const int64_t S = N - R;
-    const int j = (int)(S & 63);
-    const uint64_t lowmask = j ? ((1ull << j) - 1ull) : 0ull;
-    ctr->holes_low = (int32_t)(wp[S >> 6] + __popcll(bits[S >> 6] & lowmask));
-    ctr->size = (int32_t)S;
 }
 
 struct Scratch {
     uint32_t* bsum;
     uint32_t* wp;
+    uint32_t* head;  // of the 64 spare words
     int64_t nb;
 };
 
@@ -174,33 +200,35 @@ Scratch carve(void* scratch, int64_t n_max) {
     s.nb = nb > 0 ? nb : 1;
     s.bsum = reinterpret_cast<uint32_t*>(scratch);
     s.wp = s.bsum + ((s.nb + 63) / 64) * 64;
+    s.head = s.wp + W;
     return s;
 }
 
 int holefill_impl(int64_t n_max, int64_t stride, oppx_move_counters* counters, const uint64_t* hole_bits,
                   const oppx_dat_desc* dats, int n_dats, void* work, hipStream_t s) {
-    DatTable T{};
-    T.n = n_dats;
-    T.stride = stride;
     for (int q = 0; q < n_dats; q++) {
         OPPX_ARG_CHECK(dats[q].base && dats[q].dim > 0, "oppx_holefill: bad dat descriptor");
         OPPX_ARG_CHECK(dats[q].elem_bytes == 4 || dats[q].elem_bytes == 8, "oppx_holefill: elem_bytes 4 or 8");
-        T.base[q] = dats[q].base;
-        T.dim[q] = dats[q].dim;
-        T.eb[q] = dats[q].elem_bytes;
     }
     // every scratch word a pass reads was written by an earlier pass of the same call: nothing to clear
     Scratch sc = carve(work, n_max);
-    hf_block_sums<<<(unsigned)sc.nb, kB, 0, s>>>(hole_bits, counters, sc.bsum, n_max);
-    OPPX_LAUNCH_CHECK("hf_block_sums");
-    hf_scan_blocks<<<1, kB, 0, s>>>(sc.bsum, sc.nb, counters);
-    OPPX_LAUNCH_CHECK("hf_scan_blocks");
-    hf_word_prefix<<<(unsigned)sc.nb, kB, 0, s>>>(hole_bits, counters, sc.bsum, sc.wp, n_max);
-    OPPX_LAUNCH_CHECK("hf_word_prefix");
-    hf_fill_tail<<<1024, kB, 0, s>>>(hole_bits, counters, sc.wp, T, n_max);
-    OPPX_LAUNCH_CHECK("hf_fill_tail");
-    hf_finalize<<<1, 1, 0, s>>>(hole_bits, counters, sc.wp, n_max);
-    OPPX_LAUNCH_CHECK("hf_finalize");
+    hf_count<<<(unsigned)sc.nb, kB, 0, s>>>(hole_bits, counters, sc.bsum, sc.wp, sc.head, n_max);
+    OPPX_LAUNCH_CHECK("hf_count");
+    const int per = (int)((sc.nb + kMaxGroups - 1) / kMaxGroups);
+    // one block for 8 * kB particles: with a few percent removed, a thread has at most one record to move
+    int64_t g = (n_max + 8 * kB - 1) / (8 * kB);
+    g = g < 1 ? 1 : (g > 1024 ? 1024 : g);
+    CompTable T{};
+    for (int q = 0, d = 0; q < n_dats;) {  // flatten the dats; a full table is launched and started again
+        if (dats[q].elem_bytes == 8) T.wide |= 1ull << T.n;
+        T.base[T.n++] = reinterpret_cast<char*>(dats[q].base) + (size_t)d * (size_t)stride * (size_t)dats[q].elem_bytes;
+        if (++d == dats[q].dim) { d = 0; q++; }
+        if (T.n == kMaxComps || q == n_dats) {
+            hf_fill<<<(unsigned)g, kB, 0, s>>>(hole_bits, counters, sc.bsum, sc.wp, sc.head, T, sc.nb, per, q == n_dats);
+            OPPX_LAUNCH_CHECK("hf_fill");
+            T = CompTable{};
+        }
+    }
     return OPPX_OK;
 }
 
