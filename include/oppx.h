@@ -89,8 +89,7 @@ typedef struct oppx_move_counters {
     int64_t total_hops;        /* kernel evaluations of the pass */
     int32_t faults;            /* particles whose walk hit the hop cap or an invalid cell index */
     int32_t pad;
-    int32_t queue[8];          /* per XCD: next block tile of the persistent walk, or worklist length of
-                                  the two-pass move (reset per launch) */
+    int32_t queue[8];          /* per XCD: next block tile of the persistent walk (reset per launch) */
 } oppx_move_counters;
 
 /* Walks longer than this are stopped and counted in oppx_move_counters.faults (the
@@ -273,7 +272,8 @@ int oppx_tet_aux_build(const double* c_vol, const int32_t* c2c, int64_t n_cells,
 int oppx_fempic_push(int64_t n_max, const oppx_fempic_parts* parts, const oppx_tet_mesh* mesh,
                      double k, double dt, oppx_move_counters* counters, void* stream);
 
-/* Device workspace of the two-pass move (first-hop pass + worklist walk) for n_max particles. */
+/* Device workspace of the two-pass move (first-hop pass + worklist walk) for n_max particles: a record per
+ * first-pass block and the blocks' worklists. Nothing in it has to be set before a call. */
 size_t oppx_fempic_work_bytes(int64_t n_max);
 
 /* opp_particle_move__move_kernel (apps_codegen/app_fempic_cg/hip/move_kernel_loop.hpp:142-407):

@@ -61,7 +61,7 @@ struct StepArgs {
     const oppx_batch_inst* __restrict__ insts;   // batched mode: per-instance overlay, k, dt
     oppx_move_counters* ctr;
     struct StatSlot* slots;  // nullable: per-block statistics spread over kSlots lines, reduced after the pass
-    int32_t* qcount;         // two-pass move: worklist lengths, one per queue
+    int reset;               // first pass: clear the per-move counters (the walk pass adds to them)
     uint64_t* __restrict__ hole_bits;
     int32_t* __restrict__ hops;
     double* __restrict__ charge;
@@ -96,7 +96,7 @@ __device__ __forceinline__ void st_record(double* rec, double x, double y, doubl
     r[2] = f64x2{vy, vz};
 }
 
-// Per-block statistics go to one of kSlots slots (blockIdx modulo kSlots) instead of the single
+// Tile walk: per-block statistics go to one of kSlots slots (blockIdx modulo kSlots) instead of the single
 // counters record: thousands of blocks adding to one address serialise in one L2 channel. The
 // slots are zeroed before the pass and folded into the counters by slots_reduce_kernel after it.
 constexpr int kSlots = 256;
@@ -105,7 +105,17 @@ struct StatSlot {
     int max_hops, removed, faults, pad[3];
 };
 
-__device__ __forceinline__ void block_stats(const StepArgs& P, long long hsum, int hmax, int nrem, int nfault) {
+// Two-pass move: what a block of the first pass hands to the walk pass. Each block stores its own record, so
+// nothing is cleared before the pass and no atomic is needed; the walk pass, which follows anyway, adds the
+// records up. Before, clearing and folding the slots were launches of their own, 4.5 us each after a large kernel.
+struct BlockStat {
+    unsigned long long hops;
+    int max_hops, removed, faults;
+    int pending;  // worklist entries of the block
+};
+
+// The block's totals, valid in thread 0 (ends with the other threads free to leave).
+__device__ __forceinline__ BlockStat block_totals(long long hsum, int hmax, int nrem, int nfault) {
     __shared__ long long s_sum[kMaxBlock / kWave];
     __shared__ int s_max[kMaxBlock / kWave], s_rem[kMaxBlock / kWave], s_flt[kMaxBlock / kWave];
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
@@ -113,37 +123,50 @@ __device__ __forceinline__ void block_stats(const StepArgs& P, long long hsum, i
     const int hm = wave_max_i32(hmax), nr = wave_sum_i32(nrem), nf = wave_sum_i32(nfault);
     if (lane == 0) { s_sum[w] = hs; s_max[w] = hm; s_rem[w] = nr; s_flt[w] = nf; }
     __syncthreads();
+    BlockStat t{0ull, 0, 0, 0, 0};
     if (threadIdx.x == 0) {
-        long long t = 0;
-        int m = 0, r = 0, f = 0;
         for (int q = 0; q < (int)(blockDim.x / kWave); q++) {
-            t += s_sum[q];
-            m = m > s_max[q] ? m : s_max[q];
-            r += s_rem[q];
-            f += s_flt[q];
+            t.hops += (unsigned long long)s_sum[q];
+            t.max_hops = t.max_hops > s_max[q] ? t.max_hops : s_max[q];
+            t.removed += s_rem[q];
+            t.faults += s_flt[q];
         }
+    }
+    return t;
+}
+
+__device__ __forceinline__ void block_stats(const StepArgs& P, long long hsum, int hmax, int nrem, int nfault) {
+    const BlockStat t = block_totals(hsum, hmax, nrem, nfault);
+    if (threadIdx.x == 0) {
         if (P.slots) {
             StatSlot* sl = P.slots + (blockIdx.x % kSlots);
-            if (t) atomicAdd(&sl->hops, (unsigned long long)t);
-            if (m) atomicMax(&sl->max_hops, m);
-            if (r) atomicAdd(&sl->removed, r);
-            if (f) atomicAdd(&sl->faults, f);
+            if (t.hops) atomicAdd(&sl->hops, t.hops);
+            if (t.max_hops) atomicMax(&sl->max_hops, t.max_hops);
+            if (t.removed) atomicAdd(&sl->removed, t.removed);
+            if (t.faults) atomicAdd(&sl->faults, t.faults);
         } else {
-            if (t) atomicAdd((unsigned long long*)&P.ctr->total_hops, (unsigned long long)t);
-            if (m) atomicMax(&P.ctr->max_hops, m);
-            if (r) atomicAdd(&P.ctr->removed, r);
-            if (f) atomicAdd(&P.ctr->faults, f);
+            if (t.hops) atomicAdd((unsigned long long*)&P.ctr->total_hops, t.hops);
+            if (t.max_hops) atomicMax(&P.ctr->max_hops, t.max_hops);
+            if (t.removed) atomicAdd(&P.ctr->removed, t.removed);
+            if (t.faults) atomicAdd(&P.ctr->faults, t.faults);
         }
     }
 }
 
-__global__ void slots_reset_kernel(StatSlot* slots, int32_t* qcount) {
+__device__ __forceinline__ void reset_counters(oppx_move_counters* ctr) {
+    ctr->removed = 0;
+    ctr->holes_low = 0;
+    ctr->max_hops = 0;
+    ctr->total_hops = 0;
+    for (int x = 0; x < kXcds; x++) ctr->queue[x] = 0;
+}
+
+__global__ void slots_reset_kernel(StatSlot* slots) {
     const int t = threadIdx.x;  // kSlots threads
     slots[t].hops = 0ull;
     slots[t].max_hops = 0;
     slots[t].removed = 0;
     slots[t].faults = 0;
-    if (qcount) qcount[t] = 0;
 }
 
 __global__ void slots_reduce_kernel(const StatSlot* slots, oppx_move_counters* ctr) {
@@ -329,9 +352,10 @@ __global__ void __launch_bounds__(kBlock) fempic_pass_kernel(StepArgs P, uint32_
 // ---------------------------------------------------------------------------------------------
 // Two-pass move. The first pass is one lane per particle over the whole set (full occupancy, every
 // load independent across lanes): push, overlay lookup and up to `inline_hops` evaluations of the
-// elemental move kernel. A particle still moving after that is appended to its XCD's worklist
+// elemental move kernel. A particle still moving after that is appended to its block's worklist
 // (wave-aggregated append) with its current cell in p2c; the second pass walks only those, on a
-// resident grid, to completion. Per-particle results are those of the single walk.
+// resident grid, to completion, and adds up the first pass's statistics. Per-particle results are those
+// of the single walk.
 
 enum HopResult { kHopInside = 0, kHopMove = 1, kHopExit = 2, kHopBad = 3 };
 
@@ -451,10 +475,12 @@ union FirstLds {
 };
 static_assert(sizeof(CellCache) <= sizeof(DepositTable), "the cell cache lives inside the deposit table's LDS");
 
-// Worklist of the second pass: one list per XCD, `cap` entries each, {particle, hops so far}.
+// What the first pass leaves for the walk pass: one record per block, and the blocks' worklists, `parts`
+// (the particles of a block) entries {particle, hops so far} each.
 struct WorkList {
+    BlockStat* __restrict__ rec;
     int2* __restrict__ entry;
-    int64_t cap;
+    int parts;
 };
 
 template <int BS, bool PUSH, bool DH, bool DEPOSIT, bool BATCH, bool GATHER>
@@ -464,7 +490,10 @@ __global__ void __launch_bounds__(BS) fempic_first_kernel(StepArgs P, uint32_t n
     // workgroups past the blocks of live particles (the grid is sized by the host's bound) leave at
     // once; the removal-bitmap words past the live count are never read
     const uint32_t nlive = live_blocks(n, BS, nblocks);
+    if (P.reset && blockIdx.x == 0 && threadIdx.x == 0) reset_counters(P.ctr);
     if (blockIdx.x >= nlive) return;
+    __shared__ int s_pending;
+    if (threadIdx.x == 0) s_pending = 0;  // a barrier comes before its first use
     const uint32_t b = xcd_block(blockIdx.x, nlive);
     const int64_t i = (int64_t)b * BS + threadIdx.x;
     const bool live = i < n;
@@ -596,6 +625,7 @@ __global__ void __launch_bounds__(BS) fempic_first_kernel(StepArgs P, uint32_t n
     }
     if constexpr (!CACHE) {
         if (DEPOSIT) table_clear(s_table);
+        __syncthreads();
     }
 
     // direct hop
@@ -667,17 +697,14 @@ __global__ void __launch_bounds__(BS) fempic_first_kernel(StepArgs P, uint32_t n
         if (P.hops && !(live && !skip && !fault)) P.hops[i] = h;
     }
 
-    // hand the still-moving particles to worklist (blockIdx mod kSlots): same XCD, spread counters
+    // hand the still-moving particles to the block's worklist
     const unsigned long long pmask = __ballot(pending);
     if (pmask) {
-        const uint32_t q = blockIdx.x % kSlots;
         int base = 0;
-        if (lane == 0) base = atomicAdd(&P.qcount[q], __popcll(pmask));
+        if (lane == 0) base = atomicAdd(&s_pending, __popcll(pmask));
         base = __shfl(base, 0);
-        if (pending) {
-            const int64_t slot = base + __popcll(pmask & ((1ull << lane) - 1ull));
-            if (slot < W.cap) W.entry[q * W.cap + slot] = make_int2((int)i, h);
-        }
+        if (pending)
+            W.entry[(int64_t)blockIdx.x * BS + base + __popcll(pmask & ((1ull << lane) - 1ull))] = make_int2((int)i, h);
     }
     if (DEPOSIT) {
         __syncthreads();  // table cleared
@@ -695,7 +722,11 @@ __global__ void __launch_bounds__(BS) fempic_first_kernel(StepArgs P, uint32_t n
     const unsigned long long rmask = __ballot(live && removed);
     if (lane == 0) P.hole_bits[i >> 6] = rmask;
     const bool done = live && !skip && !pending;
-    block_stats(P, done ? h : 0, done ? h : 0, (live && removed) ? 1 : 0, fault ? 1 : 0);
+    BlockStat t = block_totals(done ? h : 0, done ? h : 0, (live && removed) ? 1 : 0, fault ? 1 : 0);
+    if (threadIdx.x == 0) {
+        t.pending = s_pending;
+        W.rec[blockIdx.x] = t;
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -767,6 +798,7 @@ __global__ void __launch_bounds__(kQuadBlock) fempic_quad_kernel(StepArgs P, uin
     int64_t n = P.ctr->size;
     n = n < 0 ? 0 : (n > P.n_max ? P.n_max : n);
     const uint32_t nlive = live_blocks(n, kQuadParts, nblocks);
+    if (P.reset && blockIdx.x == 0 && threadIdx.x == 0) reset_counters(P.ctr);
     if (blockIdx.x >= nlive) return;  // no block of live particles left for this workgroup
     const uint32_t b = xcd_block(blockIdx.x, nlive);
     const int r = threadIdx.x & 3;
@@ -796,7 +828,10 @@ __global__ void __launch_bounds__(kQuadBlock) fempic_quad_kernel(StepArgs P, uin
     double l = 0.0;
     __shared__ DepositTable s_table;
     __shared__ uint32_t s_bits[kQuadBlock / kWave];
+    __shared__ int s_pending;
+    if (threadIdx.x == 0) s_pending = 0;
     if (DEPOSIT) table_clear(s_table);
+    __syncthreads();
 
     if (live && !skip && !fault) {
         double kk = P.k, dt = P.dt;
@@ -883,17 +918,14 @@ __global__ void __launch_bounds__(kQuadBlock) fempic_quad_kernel(StepArgs P, uin
     const bool lead = r == 0;
     const unsigned long long pmask = __ballot(pending && lead);
     if (pmask) {
-        const uint32_t q = blockIdx.x % kSlots;
         int base = 0;
-        if (lane == 0) base = atomicAdd(&P.qcount[q], __popcll(pmask));
+        if (lane == 0) base = atomicAdd(&s_pending, __popcll(pmask));
         base = __shfl(base, 0);
-        if (pending && lead) {
-            const int64_t slot = base + __popcll(pmask & ((1ull << lane) - 1ull));
-            if (slot < W.cap) W.entry[q * W.cap + slot] = make_int2((int)i, h);
-        }
+        if (pending && lead)
+            W.entry[(int64_t)blockIdx.x * kQuadParts + base + __popcll(pmask & ((1ull << lane) - 1ull))] =
+                make_int2((int)i, h);
     }
     if (DEPOSIT) {
-        __syncthreads();  // table cleared
         if (live && !skip && !fault && !removed && !pending) {
             const int node = P.c2n[4 * (int64_t)cell + r];
             table_add(s_table, P.charge, node, l);
@@ -910,78 +942,115 @@ __global__ void __launch_bounds__(kQuadBlock) fempic_quad_kernel(StepArgs P, uin
         P.hole_bits[b] = word;
     }
     const bool done = live && !skip && !pending && lead;
-    block_stats(P, done ? h : 0, done ? h : 0, (live && removed && lead) ? 1 : 0, (fault && lead) ? 1 : 0);
+    BlockStat t = block_totals(done ? h : 0, done ? h : 0, (live && removed && lead) ? 1 : 0, (fault && lead) ? 1 : 0);
+    if (threadIdx.x == 0) {
+        t.pending = s_pending;
+        W.rec[blockIdx.x] = t;
+    }
 }
 
+// The walk pass: adds up the first pass's block records and walks its worklists to completion. A block takes
+// `per` first-pass blocks at a time, all of one XCD (first-pass block p ran on XCD p % 8), and walks their
+// entries as one dense list: 256 where the first pass walks (nearly) everything itself and the records are
+// all there is to read, few where it hands over many entries and the grid should spread them.
 template <bool DEPOSIT>
-__global__ void __launch_bounds__(kBlock) fempic_walk_kernel(StepArgs P, WorkList W) {
-    const uint32_t q = blockIdx.x % kSlots;
-    const uint32_t nb_q = gridDim.x / kSlots;  // blocks draining this queue (grid is a multiple of kSlots)
-    const uint32_t k_q = blockIdx.x / kSlots;
-    int64_t m = P.qcount[q];
-    m = m < 0 ? 0 : (m > W.cap ? W.cap : m);
+__global__ void __launch_bounds__(kBlock) fempic_walk_kernel(StepArgs P, WorkList W, uint32_t nblocks, int per) {
+    int64_t n = P.ctr->size;
+    n = n < 0 ? 0 : (n > P.n_max ? P.n_max : n);
+    const uint32_t nlive = live_blocks(n, W.parts, nblocks);
+    const uint32_t x = blockIdx.x % kXcds, mine = nlive > x ? (nlive - x + kXcds - 1) / kXcds : 0;
+    const uint32_t chunks = (mine + per - 1) / per;
     const int64_t S = P.stride;
     __shared__ DepositTable s_table;
-    if (DEPOSIT) table_clear(s_table);
-    __syncthreads();
+    __shared__ int s_off[kBlock], s_wave[kBlock / kWave];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
 
     long long hsum = 0;
     int hmax = 0, nrem = 0, nfault = 0;
-    // block-uniform rounds of kBlock entries; with the deposit, the LDS table is flushed after every
-    // round so that it never fills (a full table sends every further add to a global atomic)
-    for (int64_t base = (int64_t)k_q * kBlock; base < m; base += (int64_t)nb_q * kBlock) {
-        const int64_t e = base + threadIdx.x;
-        if (DEPOSIT && base != (int64_t)k_q * kBlock) {
-            __syncthreads();  // the previous round's adds are in the table
-            table_flush(s_table, P.charge);
-            __syncthreads();
-            table_clear(s_table);
-            __syncthreads();
+    for (uint32_t c = blockIdx.x / kXcds; c < chunks; c += gridDim.x / kXcds) {
+        const uint32_t first = x + kXcds * c * (uint32_t)per;  // first-pass blocks first, first + 8, ...
+        BlockStat t{0ull, 0, 0, 0, 0};
+        if ((int)threadIdx.x < per && c * (uint32_t)per + threadIdx.x < mine) t = W.rec[first + kXcds * threadIdx.x];
+        hsum += (long long)t.hops;
+        hmax = hmax > t.max_hops ? hmax : t.max_hops;
+        nrem += t.removed;
+        nfault += t.faults;
+        if (!__syncthreads_or(t.pending)) continue;  // the usual case: nothing was handed over
+        int inc = t.pending;  // exclusive scan of the worklist lengths over the block
+#pragma unroll
+        for (int d = 1; d < kWave; d <<= 1) {
+            const int v = __shfl_up(inc, d);
+            if (lane >= d) inc += v;
         }
-        if (e >= m) continue;
-        const int2 w = W.entry[q * W.cap + e];
-        const int64_t i = w.x;
-        int h = w.y;
-        int cell = P.p2c[i];
-        const bool rec = P.rec_out != nullptr;  // the first pass left the pushed position in a record
-        const double x = rec ? P.rec_out[6 * i] : P.pos[i];
-        const double y = rec ? P.rec_out[6 * i + 1] : P.pos[S + i];
-        const double z = rec ? P.rec_out[6 * i + 2] : P.pos[2 * S + i];
-        double l0 = 0.0, l1 = 0.0, l2 = 0.0, l3 = 0.0;
-        bool removed = false, fault = !((unsigned)cell < (unsigned)P.n_cells);
-        while (!fault) {
-            const int r = hop_eval(P, x, y, z, cell, l0, l1, l2, l3);
-            h++;
-            if (r == kHopInside) break;
-            if (r == kHopExit) { removed = true; break; }
-            if (r == kHopBad || h >= OPPX_MAX_HOPS) fault = true;
+        if (lane == kWave - 1) s_wave[wave] = inc;
+        __syncthreads();
+        int off = 0, total = 0;
+        for (int q = 0; q < kBlock / kWave; q++) {
+            if (q < wave) off += s_wave[q];
+            total += s_wave[q];
         }
-        if (!fault) {
-            P.lc[i] = l0; P.lc[S + i] = l1; P.lc[2 * S + i] = l2; P.lc[3 * S + i] = l3;
-            P.p2c[i] = removed ? kMaxCell : cell;
-            if (removed) {
-                atomicOr((unsigned long long*)&P.hole_bits[i >> 6], 1ull << (i & 63));
-                nrem++;
-            } else if (DEPOSIT) {
-                const int4 c = *reinterpret_cast<const int4*>(P.c2n + 4 * (int64_t)cell);
-                table_add(s_table, P.charge, c.x, l0);
-                table_add(s_table, P.charge, c.y, l1);
-                table_add(s_table, P.charge, c.z, l2);
-                table_add(s_table, P.charge, c.w, l3);
+        s_off[threadIdx.x] = off + inc - t.pending;
+        // block-uniform rounds of kBlock entries; with the deposit, the LDS table is flushed after every
+        // round so that it never fills (a full table sends every further add to a global atomic)
+        for (int base = 0; base < total; base += kBlock) {
+            if (DEPOSIT) table_clear(s_table);
+            __syncthreads();  // table cleared, offsets written
+            const int e = base + (int)threadIdx.x;
+            if (e < total) {
+                int lo = 0, hi = per - 1;  // the last worklist that begins at or before entry e
+                while (lo < hi) {
+                    const int mid = (lo + hi + 1) >> 1;
+                    if (s_off[mid] <= e) lo = mid;
+                    else hi = mid - 1;
+                }
+                const int2 w = W.entry[(int64_t)(first + kXcds * (uint32_t)lo) * W.parts + (e - s_off[lo])];
+                const int64_t i = w.x;
+                int h = w.y;
+                int cell = P.p2c[i];
+                const bool rec = P.rec_out != nullptr;  // the first pass left the pushed position in a record
+                const double px = rec ? P.rec_out[6 * i] : P.pos[i];
+                const double py = rec ? P.rec_out[6 * i + 1] : P.pos[S + i];
+                const double pz = rec ? P.rec_out[6 * i + 2] : P.pos[2 * S + i];
+                double l0 = 0.0, l1 = 0.0, l2 = 0.0, l3 = 0.0;
+                bool removed = false, fault = !((unsigned)cell < (unsigned)P.n_cells);
+                while (!fault) {
+                    const int r = hop_eval(P, px, py, pz, cell, l0, l1, l2, l3);
+                    h++;
+                    if (r == kHopInside) break;
+                    if (r == kHopExit) { removed = true; break; }
+                    if (r == kHopBad || h >= OPPX_MAX_HOPS) fault = true;
+                }
+                if (!fault) {
+                    P.lc[i] = l0; P.lc[S + i] = l1; P.lc[2 * S + i] = l2; P.lc[3 * S + i] = l3;
+                    P.p2c[i] = removed ? kMaxCell : cell;
+                    if (removed) {
+                        atomicOr((unsigned long long*)&P.hole_bits[i >> 6], 1ull << (i & 63));
+                        nrem++;
+                    } else if (DEPOSIT) {
+                        const int4 m = *reinterpret_cast<const int4*>(P.c2n + 4 * (int64_t)cell);
+                        table_add(s_table, P.charge, m.x, l0);
+                        table_add(s_table, P.charge, m.y, l1);
+                        table_add(s_table, P.charge, m.z, l2);
+                        table_add(s_table, P.charge, m.w, l3);
+                    }
+                } else {
+                    nfault++;
+                }
+                if (P.hops) P.hops[i] = h;
+                hsum += h;
+                hmax = hmax > h ? hmax : h;
             }
-        } else {
-            nfault++;
+            __syncthreads();  // the round's adds are in the table; its entries' offsets are read
+            if (DEPOSIT) {
+                table_flush(s_table, P.charge);
+                __syncthreads();
+            }
         }
-        if (P.hops) P.hops[i] = h;
-        hsum += h;
-        hmax = hmax > h ? hmax : h;
     }
-    __syncthreads();
-    if (DEPOSIT) table_flush(s_table, P.charge);
     block_stats(P, hsum, hmax, nrem, nfault);
 }
 
-// Zero the per-XCD worklist / queue counters before a launch that uses them.
+// Zero the per-XCD queue counters before a launch that uses them.
 __global__ void reset_queue_kernel(oppx_move_counters* ctr) {
     if (threadIdx.x < kXcds) ctr->queue[threadIdx.x] = 0;
 }
@@ -1209,13 +1278,7 @@ __global__ void __launch_bounds__(kBlock) fempic_tile_kernel(StepArgs P, uint32_
 }
 
 // Per-move reset of the counters (a kernel, not a memset, so the step can be graph-captured).
-__global__ void reset_counters_kernel(oppx_move_counters* ctr) {
-    ctr->removed = 0;
-    ctr->holes_low = 0;
-    ctr->max_hops = 0;
-    ctr->total_hops = 0;
-    for (int x = 0; x < kXcds; x++) ctr->queue[x] = 0;
-}
+__global__ void reset_counters_kernel(oppx_move_counters* ctr) { reset_counters(ctr); }
 
 // Start of a fused step: zero the deposit target and the per-step counters in one launch.
 __global__ void step_begin_kernel(oppx_move_counters* __restrict__ ctr, double* __restrict__ charge, int64_t n_nodes) {
@@ -1318,25 +1381,25 @@ void launch_tile(const StepArgs& P, int64_t n_max, hipStream_t s) {
     kern<<<g, kBlock, 0, s>>>(P, nbt);
 }
 
-// Work buffer of the move: worklist lengths [kSlots] int32, statistics slots [kSlots], then kSlots
-// worklists of work_cap(n_max) {particle, hops} entries.
-constexpr size_t kWorkHeader = kSlots * sizeof(int32_t) + kSlots * sizeof(StatSlot);
+// Work buffer of the move. Tile walk: statistics slots [kSlots]. Two-pass move: one record per block of the
+// first pass (64, 256 or 1024 particles), then the blocks' worklists.
+constexpr size_t kSlotBytes = kSlots * sizeof(StatSlot);
 
-int64_t work_cap(int64_t n_max) {  // per queue, for either first-pass block size
-    const int64_t a = ((n_max + kBlock - 1) / kBlock / kSlots + 1) * kBlock;
-    const int64_t b = ((n_max + kMaxBlock - 1) / kMaxBlock / kSlots + 1) * kMaxBlock;
-    return a > b ? a : b;
+size_t record_bytes(int64_t n_max) {
+    const int64_t blocks = n_max > 0 ? (n_max + kQuadParts - 1) / kQuadParts : 0;
+    return ((size_t)blocks * sizeof(BlockStat) + 255) & ~(size_t)255;
 }
 
-size_t work_need(int64_t n_max) { return kWorkHeader + (size_t)kSlots * (size_t)work_cap(n_max) * sizeof(int2); }
+size_t work_need(int64_t n_max) {
+    const size_t two = record_bytes(n_max) + (size_t)(n_max + kMaxBlock) * sizeof(int2);
+    return two > kSlotBytes ? two : kSlotBytes;
+}
 
 // Point P's statistics at the slots of the work buffer (when it holds them) and zero them.
-bool attach_slots(StepArgs& P, void* work, size_t work_bytes, hipStream_t s) {
-    if (!work || work_bytes < kWorkHeader) return false;
-    P.qcount = reinterpret_cast<int32_t*>(work);
-    P.slots = reinterpret_cast<StatSlot*>(reinterpret_cast<char*>(work) + kSlots * sizeof(int32_t));
-    slots_reset_kernel<<<1, kSlots, 0, s>>>(P.slots, P.qcount);
-    return true;
+void attach_slots(StepArgs& P, void* work, size_t work_bytes, hipStream_t s) {
+    if (!work || work_bytes < kSlotBytes) return;
+    P.slots = reinterpret_cast<StatSlot*>(work);
+    slots_reset_kernel<<<1, kSlots, 0, s>>>(P.slots);
 }
 
 void fold_slots(const StepArgs& P, hipStream_t s) {
@@ -1347,22 +1410,32 @@ void fold_slots(const StepArgs& P, hipStream_t s) {
 // tuning asks for it; returns false when the caller should use the cooperative tile walk instead.
 template <bool PUSH, bool DH, bool DEPOSIT, bool BATCH, bool GATHER = false>
 bool launch_two_pass(const StepArgs& P, int64_t n_max, void* work, size_t work_bytes, hipStream_t s) {
-    if (!P.slots || g_tuning.inline_hops < 1 || work_bytes < work_need(n_max)) return false;
-    WorkList W{reinterpret_cast<int2*>(reinterpret_cast<char*>(work) + kWorkHeader), work_cap(n_max)};
+    if (!work || g_tuning.inline_hops < 1 || work_bytes < work_need(n_max)) return false;
+    WorkList W{reinterpret_cast<BlockStat*>(work),
+               reinterpret_cast<int2*>(reinterpret_cast<char*>(work) + record_bytes(n_max)), kBlock};
+    unsigned g;
     if (g_tuning.lanes == 4) {
-        const unsigned g = grid_for(n_max, kQuadParts);
+        W.parts = kQuadParts;
+        g = grid_for(n_max, kQuadParts);
         fempic_quad_kernel<PUSH, DH, DEPOSIT, BATCH, GATHER><<<g, kQuadBlock, 0, s>>>(P, g, g_tuning.inline_hops, W);
     } else if (g_tuning.first_block == kMaxBlock) {
-        const unsigned g = grid_for(n_max, kMaxBlock);
+        W.parts = kMaxBlock;
+        g = grid_for(n_max, kMaxBlock);
         fempic_first_kernel<kMaxBlock, PUSH, DH, DEPOSIT, BATCH, GATHER><<<g, kMaxBlock, 0, s>>>(P, g, g_tuning.inline_hops, W);
     } else {
-        const unsigned g = grid_for(n_max, kBlock);
+        g = grid_for(n_max, kBlock);
         fempic_first_kernel<kBlock, PUSH, DH, DEPOSIT, BATCH, GATHER><<<g, kBlock, 0, s>>>(P, g, g_tuning.inline_hops, W);
     }
+    // A first pass that walks 16 evaluations itself hands over next to nothing: 256 records a walk block, at most
+    // 256 blocks (each adds to the one counters record). Below that the walk spreads over the resident grid.
+    const bool rare = g_tuning.inline_hops >= 16;
+    const int per = rare ? kBlock : 8;
     auto walk = fempic_walk_kernel<DEPOSIT>;
-    unsigned wg = resident_blocks(reinterpret_cast<const void*>(walk), kBlock);
-    wg = wg < (unsigned)kSlots ? (unsigned)kSlots : (wg / kSlots) * kSlots;
-    walk<<<wg, kBlock, 0, s>>>(P, W);
+    const unsigned cap = rare ? 256u : resident_blocks(reinterpret_cast<const void*>(walk), kBlock);
+    unsigned wg = ((g + kXcds - 1) / kXcds + per - 1) / per * kXcds;  // every chunk of every XCD
+    if (wg > cap) wg = cap / kXcds * kXcds;
+    if (wg < (unsigned)kXcds) wg = kXcds;
+    walk<<<wg, kBlock, 0, s>>>(P, W, g, per);
     return true;
 }
 
@@ -1420,7 +1493,6 @@ int step_rec(StepArgs& P, const char* who, int64_t n_max, const int32_t* perm, c
     P.hops = hops;
     P.charge = node_charge;
     P.rec_out = rec_out;
-    attach_slots(P, work, work_bytes, s);
     if (perm) {
         P.perm = perm;
         P.src_rec = src_rec;
@@ -1437,7 +1509,6 @@ int step_rec(StepArgs& P, const char* who, int64_t n_max, const int32_t* perm, c
         if (perm) launch_rec<false, false, true>(P, node_charge != nullptr, n_max, work, work_bytes, s);
         else launch_rec<false, false, false>(P, node_charge != nullptr, n_max, work, work_bytes, s);
     }
-    fold_slots(P, s);
     OPPX_LAUNCH_CHECK(who);
     return OPPX_OK;
 }
@@ -1480,17 +1551,24 @@ int oppx_fempic_move(int64_t n_max, const oppx_fempic_parts* parts, const oppx_t
     OPPX_ARG_CHECK(n_max >= 0 && n_max <= parts->stride, "oppx_fempic_move: n_max beyond capacity");
     OPPX_ARG_CHECK(hole_bits != nullptr, "oppx_fempic_move: hole_bits required");
     hipStream_t s = as_stream(stream);
-    reset_counters_kernel<<<1, 1, 0, s>>>(counters);
-    OPPX_LAUNCH_CHECK("reset_counters");
-    if (n_max == 0) return OPPX_OK;
+    if (n_max == 0) {
+        reset_counters_kernel<<<1, 1, 0, s>>>(counters);
+        OPPX_LAUNCH_CHECK("reset_counters");
+        return OPPX_OK;
+    }
     P.n_max = n_max;
     P.hole_bits = hole_bits;
     P.hops = hops;
-    attach_slots(P, work, work_bytes, s);
+    P.reset = 1;  // the first pass clears the counters, which only the walk pass adds to
     const bool two = dh ? launch_two_pass<false, true, false, false>(P, n_max, work, work_bytes, s)
                         : launch_two_pass<false, false, false, false>(P, n_max, work, work_bytes, s);
-    if (!two) launch_pass<false, true, false>(P, dh != nullptr, true, n_max, s);
-    fold_slots(P, s);
+    if (!two) {
+        reset_counters_kernel<<<1, 1, 0, s>>>(counters);
+        OPPX_LAUNCH_CHECK("reset_counters");
+        attach_slots(P, work, work_bytes, s);
+        launch_pass<false, true, false>(P, dh != nullptr, true, n_max, s);
+        fold_slots(P, s);
+    }
     OPPX_LAUNCH_CHECK("fempic_move");
     return OPPX_OK;
 }
@@ -1527,12 +1605,12 @@ int oppx_fempic_step_fused(int64_t n_max, const oppx_fempic_parts* parts, const 
     P.hole_bits = hole_bits;
     P.hops = hops;
     P.charge = node_charge;
-    attach_slots(P, work, work_bytes, s);
     bool two;
     if (dh) two = node_charge ? launch_two_pass<true, true, true, false>(P, n_max, work, work_bytes, s)
                               : launch_two_pass<true, true, false, false>(P, n_max, work, work_bytes, s);
     else two = node_charge ? launch_two_pass<true, false, true, false>(P, n_max, work, work_bytes, s)
                            : launch_two_pass<true, false, false, false>(P, n_max, work, work_bytes, s);
+    if (!two) attach_slots(P, work, work_bytes, s);
     if (two) {
     } else if (g_tuning.split == 1 && dh != nullptr) {
         // two passes: coalesced push + overlay relocation, then the cooperative walk (+ deposit)
@@ -1580,7 +1658,6 @@ int oppx_fempic_step_fused_gather(int64_t n_max, const int32_t* perm, const oppx
     P.src_vel = src->vel;
     P.src_lc = src->lc;
     P.src_p2c = src->p2c;
-    attach_slots(P, work, work_bytes, s);
     if (dh) {
         if (node_charge) launch_two_pass<true, true, true, false, true>(P, n_max, work, work_bytes, s);
         else launch_two_pass<true, true, false, false, true>(P, n_max, work, work_bytes, s);
@@ -1588,7 +1665,6 @@ int oppx_fempic_step_fused_gather(int64_t n_max, const int32_t* perm, const oppx
         if (node_charge) launch_two_pass<true, false, true, false, true>(P, n_max, work, work_bytes, s);
         else launch_two_pass<true, false, false, false, true>(P, n_max, work, work_bytes, s);
     }
-    fold_slots(P, s);
     OPPX_LAUNCH_CHECK("fempic_step_fused_gather");
     return OPPX_OK;
 }
@@ -1655,14 +1731,14 @@ int oppx_fempic_batch_step_fused(int64_t n_max, const oppx_fempic_parts* parts, 
     P.insts = insts;
     P.n_insts = n_insts;
     hipStream_t s = as_stream(stream);
-    attach_slots(P, work, work_bytes, s);
     const bool two = node_charge ? launch_two_pass<true, true, true, true>(P, n_max, work, work_bytes, s)
                                  : launch_two_pass<true, true, false, true>(P, n_max, work, work_bytes, s);
     if (!two) {
+        attach_slots(P, work, work_bytes, s);
         if (node_charge) launch_tile<true, true, true, true, false, true>(P, n_max, s);
         else launch_tile<true, true, false, true, false, true>(P, n_max, s);
+        fold_slots(P, s);
     }
-    fold_slots(P, s);
     OPPX_LAUNCH_CHECK("fempic_batch_step_fused");
     return OPPX_OK;
 }
