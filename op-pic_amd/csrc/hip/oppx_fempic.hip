@@ -1316,7 +1316,10 @@ __global__ void __launch_bounds__(kBlock) gather_records_kernel(int64_t n_max, i
                                                                 double* __restrict__ vel, int32_t* __restrict__ faults) {
     int64_t n = ctr->size;
     n = n < 0 ? 0 : (n > n_max ? n_max : n);
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
+    const XcdTiles X((n + kBlock - 1) / kBlock);  // a permuted record's lines in one L2
+    for (int64_t t = X.first; t < X.end; t += X.step) {
+        const int64_t i = t * kBlock + threadIdx.x;
+        if (i >= n) break;
         const int64_t src = perm ? (int64_t)perm[i] : i;
         if (!((uint64_t)src < (uint64_t)stride)) {  // a corrupt permutation entry: report, touch nothing
             atomicAdd(faults, 1);
@@ -1705,7 +1708,7 @@ int oppx_gather_records(int64_t n_max, int64_t stride, oppx_move_counters* count
     OPPX_ARG_CHECK(n_max >= 0 && stride >= n_max, "oppx_gather_records: need 0 <= n_max <= stride");
     if (n_max == 0) return OPPX_OK;
     unsigned g = grid_for(n_max, kBlock);
-    if (g > 8192) g = 8192;
+    g = xcd_grid(g > 8192 ? 8192 : g);
     gather_records_kernel<<<g, kBlock, 0, as_stream(stream)>>>(n_max, stride, counters, perm, rec, pos, vel,
                                                               &counters->faults);
     OPPX_LAUNCH_CHECK("gather_records");

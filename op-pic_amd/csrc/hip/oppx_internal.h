@@ -75,6 +75,21 @@ __device__ __forceinline__ uint32_t live_blocks(int64_t n, int64_t per_block, ui
     return l < (int64_t)nblocks ? (uint32_t)l : nblocks;
 }
 
+// The tiles a block of a striding grid takes: each XCD one contiguous eighth of the tiles, its blocks strided
+// inside it. The grid is a multiple of kXcds (xcd_grid).
+struct XcdTiles {
+    int64_t first, end, step;
+    __device__ __forceinline__ explicit XcdTiles(int64_t tiles) {
+        const uint32_t x = blockIdx.x % kXcds;
+        const int64_t q = tiles / kXcds, r = tiles % kXcds;
+        const int64_t begin = x * q + (x < r ? x : r);
+        first = begin + blockIdx.x / kXcds;
+        end = begin + q + (x < r ? 1 : 0);
+        step = gridDim.x / kXcds;
+    }
+};
+inline unsigned xcd_grid(unsigned blocks) { return (blocks + kXcds - 1) / kXcds * kXcds; }
+
 __device__ __forceinline__ int wave_sum_i32(int v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);

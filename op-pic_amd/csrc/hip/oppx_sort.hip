@@ -9,12 +9,18 @@
 // Each pass sorts by one 8-bit digit. A tile is 256 * sort_items consecutive elements (tuning), each
 // wave of its block a contiguous part of them; ranks come from wave-level digit matching (8 ballots
 // give the lanes holding the same digit) against the wave's own digit counts, so equal digits keep
-// their index order and no LDS atomic is contended by nearly sorted keys. Per-tile digit counts (a
-// histogram pass that needs no ranks) are scanned digit-major across the tiles to give every
-// (digit, tile) its output offset. Every kernel reads the live count on the device: the histogram and
-// scatter grids (sized by the capacity, capped at a few times the resident blocks) stride over the
-// live tiles only, the counts are laid out with the live tile count as row stride, and the scan
-// covers only those rows.
+// their index order and no LDS atomic is contended by nearly sorted keys. A pass is three launches: per-tile
+// digit counts (they need no ranks), one block per digit that scans its row of counts across the tiles, and
+// the scatter, whose blocks scan the 256 row totals themselves to give every (digit, tile) its output
+// offset. Every kernel reads the live count on the device: the histogram and scatter grids (sized by the
+// capacity, capped at a few times the resident blocks) stride over the live tiles only, the counts are laid
+// out with the live tile count as row stride, and the row scan covers only those. Histogram, scatter and gather
+// blocks take their tiles XCD by XCD, a contiguous eighth each (XcdTiles, xcd_block): the runs that neighbouring
+// tiles write, and the lines that neighbouring records are gathered from, then meet in one L2. Measured, sort of
+// two-steps-old particles: 24 M lazy 587 -> 523 us, their gather 1,880 -> 1,640 us; 1 M gather 81 -> 56 us;
+// 3 M 257 -> 219 us. The first row scan leaves
+// the live count and the removed count in the scratch; the later launches read them there, so that the last
+// one can write the counters while its other blocks still run.
 
 #include "oppx_internal.h"
 
@@ -22,13 +28,13 @@ namespace oppx {
 namespace {
 
 constexpr int kB = 256;
-constexpr int kItems = 16;           // elements per thread of the scan kernels
+constexpr int kItems = 16;           // elements per thread of the row scan
 constexpr int kElems = kB * kItems;
 constexpr int kMinSortItems = 4;     // smallest radix block (elements per thread) the scratch is sized for
 constexpr int kBins = 256;
 constexpr int kMaxDats = 16;
-constexpr int kRemSlots = 256;  // removed-particle counters (block id modulo kRemSlots)
 constexpr unsigned kGridMult = 4;  // grids that stride over live work: this many times the resident blocks
+constexpr unsigned kMaxHistGrid = 8192;  // blocks of a histogram launch at most (one removed count each)
 
 struct GatherTable {
     int n;
@@ -39,9 +45,24 @@ struct GatherTable {
     int eb[kMaxDats];
 };
 
-__device__ __forceinline__ int64_t live_n(const oppx_move_counters* ctr, int64_t n_max) {
-    const int64_t n = ctr->size;
+// live count behind `live` (the counters' size, or its copy in the scratch), clamped to the host's bound
+__device__ __forceinline__ int64_t live_n(const int32_t* live, int64_t n_max) {
+    const int64_t n = *live;
     return n < 0 ? 0 : (n > n_max ? n_max : n);
+}
+
+// What a sort does to the counters, by one thread of its last launch. state: live count, removed count.
+struct Finish {
+    oppx_move_counters* ctr;  // null: not the last launch
+    const int32_t* state;
+    int drop;
+};
+
+__device__ __forceinline__ void finish_sort(const Finish& F) {
+    if (!F.ctr || blockIdx.x != 0 || threadIdx.x != 0) return;
+    F.ctr->removed = F.state[1];
+    F.ctr->holes_low = 0;
+    if (F.drop) F.ctr->size = F.state[0] - F.state[1];
 }
 
 // lanes of the wave (among `active`) holding the same 8-bit digit as this lane
@@ -67,17 +88,18 @@ __device__ __forceinline__ uint32_t cell_key(int32_t c, uint32_t n_cells) {
 // once (nearly sorted keys), any other wave adds per lane.
 template <int ITEMS, bool FIRST>
 __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(8))) sort_hist(const uint32_t* __restrict__ keys, const int32_t* __restrict__ p2c,
-                                                uint32_t n_cells, const oppx_move_counters* ctr, int64_t n_max,
+                                                uint32_t n_cells, const int32_t* __restrict__ live, int64_t n_max,
                                                 int shift, uint32_t* __restrict__ hist,
-                                                unsigned long long* __restrict__ n_removed) {
+                                                uint32_t* __restrict__ rem_block) {
     __shared__ uint32_t s_h[kBins];
-    const int64_t n = live_n(ctr, n_max);
+    const int64_t n = live_n(live, n_max);
     const int lane = threadIdx.x & (kWave - 1);
     // the grid strides over the tiles below the live count; tile t's count of digit d goes to
     // hist[d * tiles + t], so the scan covers the live tiles only
     const int64_t tiles = (n + kB * ITEMS - 1) / (kB * ITEMS);
-    unsigned long long removed = 0;
-    for (int64_t t = blockIdx.x; t < tiles; t += gridDim.x) {
+    uint32_t removed = 0;  // of the wave
+    const XcdTiles X(tiles);
+    for (int64_t t = X.first; t < X.end; t += X.step) {
         s_h[threadIdx.x] = 0;  // each thread clears the word it wrote out last tile
         __syncthreads();
         const int64_t base = t * (kB * ITEMS);
@@ -91,7 +113,7 @@ __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(8))) so
         for (int r = 0; r < ITEMS; r++) {
             const bool ok = base + r * kB + threadIdx.x < n;
             const uint32_t k = key[r];
-            if (FIRST) removed += (unsigned long long)__popcll(__ballot(ok && k == n_cells));
+            if (FIRST) removed += (uint32_t)__popcll(__ballot(ok && k == n_cells));
             const uint32_t d = (k >> shift) & 0xFFu;
             const unsigned long long act = __ballot(ok);
             if (act == 0ull) continue;  // uniform over the wave
@@ -106,9 +128,17 @@ __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(8))) so
         __syncthreads();
         hist[(int64_t)threadIdx.x * tiles + t] = s_h[threadIdx.x];  // digit-major rows of the live tiles
     }
-    // per-wave removed counts land on one of kRemSlots counters (block id modulo kRemSlots): one
-    // shared counter would serialise every wave's atomic in one L2 channel
-    if (FIRST && lane == 0 && removed) atomicAdd(n_removed + (blockIdx.x % kRemSlots), removed);
+    // the block's removed particles: a word of its own, which nothing has to clear beforehand
+    if (FIRST) {
+        __shared__ uint32_t s_rem[kB / kWave];
+        if (lane == 0) s_rem[threadIdx.x / kWave] = removed;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            uint32_t r = 0;
+            for (int w = 0; w < kB / kWave; w++) r += s_rem[w];
+            rem_block[blockIdx.x] = r;
+        }
+    }
 }
 
 // ---- one digit pass over a tile of 256 * ITEMS consecutive elements ----
@@ -124,7 +154,8 @@ template <int ITEMS>
 struct TileLds {
     uint32_t run[kBins];               // the tile's elements of each digit, then the digit's start in the tile
     uint32_t wave[kB / kWave][kBins];  // per-wave digit counts, then their exclusive prefix over the waves
-    uint32_t dst[kBins];               // global offset of each digit's run
+    uint32_t base[kBins];              // global offset of each digit
+    uint32_t dst[kBins];               // global offset of each digit's run of the tile
     uint32_t tot[kB / kWave];          // wave totals of the digit-start scan
     uint32_t key[kB * ITEMS], val[kB * ITEMS];
 };
@@ -236,22 +267,33 @@ __device__ __forceinline__ void tile_write(TileLds<ITEMS>& L, int tid, const uin
     }
 }
 
-// Scatter of one digit pass with the (digit, block) offsets from the scanned per-block histograms.
+__device__ __forceinline__ uint32_t block_scan_excl(uint32_t v, uint32_t* total);
+
+// Scatter of one digit pass: a tile's run of digit d goes to the elements of smaller digits (the scanned row
+// totals) plus those of d in earlier tiles (the scanned row). Every block scans the 256 totals itself, which
+// costs it one read of 1 KB; before, scanning digits and tiles as one array took three launches a pass.
 // Four waves per SIMD: the occupancy the 16-key tile's LDS allows (four 39 KB blocks per CU), reached
 // without spilling.
 template <int ITEMS, bool LAST, bool FIRST>
 __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(4)))
 sort_scatter(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin, const int32_t* __restrict__ p2c,
-             uint32_t n_cells, const oppx_move_counters* ctr, int64_t n_max, int shift,
-             const uint32_t* __restrict__ offs, uint32_t* __restrict__ kout,
-             uint32_t* __restrict__ vout, int32_t* __restrict__ p2c_out) {
+             uint32_t n_cells, const int32_t* __restrict__ live, int64_t n_max, int shift,
+             const uint32_t* __restrict__ offs, const uint32_t* __restrict__ row_total, uint32_t* __restrict__ kout,
+             uint32_t* __restrict__ vout, int32_t* __restrict__ p2c_out, Finish F) {
     __shared__ TileLds<ITEMS> L;
-    const int64_t n = live_n(ctr, n_max);
+    const int64_t n = live_n(live, n_max);
+    {
+        uint32_t all;
+        const uint32_t b = block_scan_excl(row_total[threadIdx.x], &all);
+        L.base[threadIdx.x] = b;
+    }
+    finish_sort(F);
     // the grid (at most the blocks that fit the chip at once) strides over the tiles that hold live
     // elements: a tile past the live count is never dispatched, where each such block would still have
     // had to be given its LDS (40 KB) before it could leave
     const int64_t tiles = (n + kB * ITEMS - 1) / (kB * ITEMS);
-    for (int64_t t = blockIdx.x; t < tiles; t += gridDim.x) {
+    const XcdTiles X(tiles);
+    for (int64_t t = X.first; t < X.end; t += X.step) {
         const int64_t base = t * (kB * ITEMS);
         const int m = (int)((n - base) < kB * ITEMS ? (n - base) : kB * ITEMS);  // elements of the tile
         // the thread index, opaque to the compiler inside each tile: the per-element indexes and LDS
@@ -259,7 +301,7 @@ sort_scatter(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
         int tid = (int)threadIdx.x;
         asm volatile("" : "+v"(tid));
         for (int q = 0; q < kB / kWave; q++) L.wave[q][tid] = 0;
-        L.dst[tid] = offs[(int64_t)tid * tiles + t];
+        L.dst[tid] = L.base[tid] + offs[(uint32_t)tid * (uint32_t)tiles + (uint32_t)t];  // < 2^31 counts (n below 2^32)
         uint32_t key[ITEMS], val[ITEMS], rank[ITEMS];
         tile_load<ITEMS, FIRST>(kin, vin, p2c, n_cells, base, m, tid, key, val);
         __syncthreads();
@@ -270,7 +312,6 @@ sort_scatter(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
     }
 }
 
-// ---- exclusive scan of a uint32 array (chunks of kElems) ----
 __device__ __forceinline__ uint32_t block_scan_excl(uint32_t v, uint32_t* total) {
     __shared__ uint32_t s_w[kB / kWave];
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
@@ -292,72 +333,58 @@ __device__ __forceinline__ uint32_t block_scan_excl(uint32_t v, uint32_t* total)
     return off + inc - v;
 }
 
-// Entries of the digit counts of the live tiles (kBins rows of live tiles of per_tile elements).
-__device__ __forceinline__ int64_t live_hist_n(const oppx_move_counters* ctr, int64_t n_max, int64_t per_tile) {
-    return (int64_t)kBins * ((live_n(ctr, n_max) + per_tile - 1) / per_tile);
-}
-
-// The scan of the live digit counts: blocks of chunks past them leave at once.
-__global__ void __launch_bounds__(kB) scan_reduce(const uint32_t* __restrict__ a, const oppx_move_counters* ctr,
-                                                  int64_t n_max, int64_t per_tile, uint32_t* __restrict__ sums) {
-    const int64_t n = live_hist_n(ctr, n_max, per_tile);
-    if ((int64_t)blockIdx.x * kElems >= n) return;
-    uint32_t s = 0;
-    for (int r = 0; r < kItems; r++) {  // the chunk's total: any order, so consecutive threads on consecutive words
-        const int64_t i = (int64_t)blockIdx.x * kElems + (int64_t)r * kB + threadIdx.x;
-        if (i < n) s += a[i];
-    }
-    uint32_t tot;
-    block_scan_excl(s, &tot);
-    if (threadIdx.x == 0) sums[blockIdx.x] = tot;
-}
-
-__global__ void __launch_bounds__(kB) scan_sums(uint32_t* __restrict__ sums, const oppx_move_counters* ctr,
-                                                int64_t n_max, int64_t per_tile) {
-    const int64_t nb = (live_hist_n(ctr, n_max, per_tile) + kElems - 1) / kElems;
-    uint32_t carry = 0;
-    for (int64_t base = 0; base < nb; base += kB) {
-        const int64_t j = base + threadIdx.x;
-        const uint32_t v = (j < nb) ? sums[j] : 0u;
-        uint32_t tot;
-        const uint32_t ex = block_scan_excl(v, &tot);
-        if (j < nb) sums[j] = carry + ex;
-        carry += tot;
-    }
-}
-
-__global__ void __launch_bounds__(kB) scan_apply(uint32_t* __restrict__ a, const oppx_move_counters* ctr,
-                                                 int64_t n_max, int64_t per_tile, const uint32_t* __restrict__ sums) {
-    // The chunk passes through LDS so that global loads and stores are coalesced while each thread scans
-    // kItems consecutive words; word e sits at e + e / kItems (thread t's words from 17 t on: distinct
-    // banks across the wave).
+// Block d < kBins: exclusive scan of digit d's counts over the live tiles, in place, and the digit's total. A
+// chunk of kElems counts at a time passes through LDS so that global loads and stores are coalesced while each
+// thread scans kItems consecutive words; word e sits at e + e / kItems (thread t's words from 17 t on: distinct
+// banks across the wave). One more block in the first pass (rem_block given): the sum of the histogram blocks'
+// removed counts, and the live count, for the later launches.
+__global__ void __launch_bounds__(kB) sort_rows(uint32_t* __restrict__ hist, const int32_t* __restrict__ live,
+                                                int64_t n_max, int64_t per_tile, uint32_t* __restrict__ row_total,
+                                                const uint32_t* __restrict__ rem_block, unsigned rem_blocks,
+                                                int32_t* __restrict__ state) {
     __shared__ uint32_t s_a[kElems + kElems / kItems];
-    const int64_t n = live_hist_n(ctr, n_max, per_tile);
-    const int64_t base = (int64_t)blockIdx.x * kElems;
-    if (base >= n) return;
-    for (int r = 0; r < kItems; r++) {
-        const int e = r * kB + threadIdx.x;
-        s_a[e + e / kItems] = base + e < n ? a[base + e] : 0u;
+    const int64_t n = live_n(live, n_max);
+    if (blockIdx.x == kBins) {
+        uint32_t r = 0, tot;
+        for (unsigned q = threadIdx.x; q < rem_blocks; q += kB) r += rem_block[q];
+        block_scan_excl(r, &tot);
+        if (threadIdx.x == 0) {
+            state[0] = (int32_t)n;
+            state[1] = (int32_t)tot;
+        }
+        return;
     }
-    __syncthreads();
-    const int t0 = threadIdx.x * (kItems + 1);
-    uint32_t loc[kItems];
-    uint32_t s = 0;
-    for (int r = 0; r < kItems; r++) {
-        loc[r] = s_a[t0 + r];
-        s += loc[r];
+    const int64_t tiles = (n + per_tile - 1) / per_tile;
+    uint32_t* __restrict__ a = hist + (int64_t)blockIdx.x * tiles;
+    uint32_t carry = 0;
+    for (int64_t base = 0; base < tiles; base += kElems) {
+        for (int r = 0; r < kItems; r++) {
+            const int e = r * kB + threadIdx.x;
+            s_a[e + e / kItems] = base + e < tiles ? a[base + e] : 0u;
+        }
+        __syncthreads();
+        const int t0 = threadIdx.x * (kItems + 1);
+        uint32_t loc[kItems];
+        uint32_t sum = 0;
+        for (int r = 0; r < kItems; r++) {
+            loc[r] = s_a[t0 + r];
+            sum += loc[r];
+        }
+        uint32_t tot;
+        uint32_t run = carry + block_scan_excl(sum, &tot);
+        for (int r = 0; r < kItems; r++) {
+            s_a[t0 + r] = run;
+            run += loc[r];
+        }
+        __syncthreads();
+        for (int r = 0; r < kItems; r++) {
+            const int e = r * kB + threadIdx.x;
+            if (base + e < tiles) a[base + e] = s_a[e + e / kItems];
+        }
+        carry += tot;
+        __syncthreads();  // the chunk is stored before the next one is loaded
     }
-    uint32_t tot;
-    uint32_t run = sums[blockIdx.x] + block_scan_excl(s, &tot);
-    for (int r = 0; r < kItems; r++) {
-        s_a[t0 + r] = run;
-        run += loc[r];
-    }
-    __syncthreads();
-    for (int r = 0; r < kItems; r++) {
-        const int e = r * kB + threadIdx.x;
-        if (base + e < n) a[base + e] = s_a[e + e / kItems];
-    }
+    if (threadIdx.x == 0) row_total[blockIdx.x] = carry;
 }
 
 template <typename T>
@@ -367,10 +394,14 @@ __device__ __forceinline__ void gather_rec(const void* in, void* out, int dim, i
     for (int q = 0; q < dim; q++) d[q * stride + to] = s[q * stride + from];
 }
 
-__global__ void __launch_bounds__(kB) sort_gather(const uint32_t* __restrict__ perm, const oppx_move_counters* ctr,
-                                                  int64_t n_max, GatherTable T, int32_t* __restrict__ perm_out) {
-    const int64_t n = live_n(ctr, n_max);
-    const int64_t j = (int64_t)blockIdx.x * kB + threadIdx.x;
+__global__ void __launch_bounds__(kB) sort_gather(const uint32_t* __restrict__ perm, const int32_t* __restrict__ live,
+                                                  int64_t n_max, GatherTable T, int32_t* __restrict__ perm_out, Finish F) {
+    const int64_t n = live_n(live, n_max);
+    finish_sort(F);
+    // each XCD takes one contiguous eighth: a permuted line is then read into one L2 instead of eight
+    const uint32_t nlive = live_blocks(n, kB, gridDim.x);
+    if (blockIdx.x >= nlive) return;
+    const int64_t j = (int64_t)xcd_block(blockIdx.x, nlive) * kB + threadIdx.x;
     if (j >= n) return;
     const int64_t from = perm[j];
     if (from >= T.stride) return;  // never read outside the dats
@@ -380,13 +411,12 @@ __global__ void __launch_bounds__(kB) sort_gather(const uint32_t* __restrict__ p
     }
     if (perm_out) perm_out[j] = (int32_t)from;
 }
-__global__ void zero_u64(unsigned long long* p) { p[threadIdx.x] = 0ull; }  // kRemSlots threads
 
 __global__ void lower_bound_kernel(const int32_t* __restrict__ p2c, const oppx_move_counters* ctr, int64_t n_max,
                                    const int32_t* __restrict__ keys, int64_t k, int64_t* __restrict__ out) {
     const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= k) return;
-    const int64_t n = live_n(ctr, n_max);
+    const int64_t n = live_n(&ctr->size, n_max);
     const int32_t key = keys[j];
     int64_t lo = 0, hi = n;  // first index with p2c >= key in [lo, hi]
     while (lo < hi) {
@@ -397,19 +427,17 @@ __global__ void lower_bound_kernel(const int32_t* __restrict__ p2c, const oppx_m
     out[j] = lo;
 }
 
-__global__ void sort_finalize(oppx_move_counters* ctr, int64_t n_max, const unsigned long long* n_removed, int drop) {
-    const int64_t n = live_n(ctr, n_max);
-    int64_t r = 0;
-    for (int q = 0; q < kRemSlots; q++) r += (int64_t)n_removed[q];
-    ctr->removed = (int32_t)r;
+// the counters after a sort of a set that can hold no particle (n_max 0)
+__global__ void sort_empty(oppx_move_counters* ctr, int drop) {
+    ctr->removed = 0;
     ctr->holes_low = 0;
-    if (drop) ctr->size = (int32_t)(n - r);
+    if (drop) ctr->size = 0;
 }
 
 struct SortScratch {
-    uint32_t *ka, *va, *kb, *vb, *hist, *sums;
-    unsigned long long* n_removed;
-    int64_t nblocks, hist_n, scan_blocks;
+    uint32_t *ka, *va, *kb, *vb, *hist, *row_total, *rem_block;
+    int32_t* state;
+    int64_t nblocks;
 };
 
 // int32 words of the histogram region: per-block histograms at the smallest radix block
@@ -425,8 +453,6 @@ SortScratch carve(void* base, int64_t n_max, int items) {
     const int64_t per_block = (int64_t)kB * items;
     s.nblocks = (n_max + per_block - 1) / per_block;
     if (s.nblocks < 1) s.nblocks = 1;
-    s.hist_n = s.nblocks * kBins;
-    s.scan_blocks = (s.hist_n + kElems - 1) / kElems;
     char* p = reinterpret_cast<char*>(base);
     const size_t arr = align256((size_t)(n_max > 0 ? n_max : 1) * sizeof(uint32_t));
     s.ka = reinterpret_cast<uint32_t*>(p); p += arr;
@@ -434,17 +460,15 @@ SortScratch carve(void* base, int64_t n_max, int items) {
     s.kb = reinterpret_cast<uint32_t*>(p); p += arr;
     s.vb = reinterpret_cast<uint32_t*>(p); p += arr;
     s.hist = reinterpret_cast<uint32_t*>(p); p += align256((size_t)hist_words(n_max) * sizeof(uint32_t));
-    s.sums = reinterpret_cast<uint32_t*>(p); p += align256((size_t)s.scan_blocks * sizeof(uint32_t));
-    s.n_removed = reinterpret_cast<unsigned long long*>(p);
+    s.row_total = reinterpret_cast<uint32_t*>(p); p += kBins * sizeof(uint32_t);
+    s.state = reinterpret_cast<int32_t*>(p); p += 256;
+    s.rem_block = reinterpret_cast<uint32_t*>(p);
     return s;
 }
 
 size_t scratch_need(int64_t n_max) {
-    const int64_t per_block = (int64_t)kB * kMinSortItems;  // the largest histogram any sort_items needs
-    const int64_t nb = n_max > 0 ? (n_max + per_block - 1) / per_block : 1;
-    const int64_t scan_blocks = (nb * kBins + kElems - 1) / kElems;
     return 4 * align256((size_t)(n_max > 0 ? n_max : 1) * 4) + align256((size_t)hist_words(n_max) * 4) +
-           align256((size_t)scan_blocks * 4) + kRemSlots * sizeof(unsigned long long);
+           kBins * sizeof(uint32_t) + 256 + kMaxHistGrid * sizeof(uint32_t);
 }
 
 }  // namespace
@@ -493,40 +517,47 @@ int oppx_sort_by_cell(int64_t n_max, int64_t stride, oppx_move_counters* counter
     int bits = 1;
     while (bits < 32 && ((int64_t)1 << bits) <= n_cells) bits++;  // keys are in [0, n_cells]
     const int passes = (bits + 7) / 8;
-    zero_u64<<<1, kRemSlots, 0, s>>>(sc.n_removed);  // a kernel, not a memset node, so the sort can be captured
-    OPPX_LAUNCH_CHECK("sort_reset");
-    if (n_max > 0) {
+    if (n_max == 0) {
+        sort_empty<<<1, 1, 0, s>>>(counters, drop_removed);
+        OPPX_LAUNCH_CHECK("sort_empty");
+    } else {
         uint32_t *kin = sc.ka, *vin = sc.va, *kout = sc.kb, *vout = sc.vb;
         const uint32_t kc = (uint32_t)n_cells;
         // no dat left to gather: the last digit pass writes the permutation straight into perm_out
         const bool direct = T.n == 0 && perm_out != nullptr;
+        const bool gather = !direct && (T.n > 0 || perm_out);
+        const Finish no_finish{nullptr, nullptr, 0}, finish{counters, sc.state, drop_removed};
         for (int pass = 0; pass < passes; pass++) {
             const int shift = 8 * pass;
             const bool first = pass == 0;
             const bool last = pass == passes - 1;  // the keys of the last pass are not needed
             uint32_t* vdst = (last && direct) ? reinterpret_cast<uint32_t*>(perm_out) : vout;
             {
-#define OPPX_HIST(I, F)                                                                              \
-    sort_hist<I, F><<<stride_grid(reinterpret_cast<const void*>(sort_hist<I, F>), kB, sc.nblocks, kGridMult), kB, 0, \
-                      s>>>(kin, p2c, kc, counters, n_max, shift, sc.hist, sc.n_removed)
+                // the first pass's histogram and row scan read the counters, the later launches the scratch copy
+                const int32_t* live = first ? &counters->size : sc.state;
+                unsigned hist_grid = 1;
+#define OPPX_HIST(I, F)                                                                                              \
+    do {                                                                                                             \
+        hist_grid = stride_grid(reinterpret_cast<const void*>(sort_hist<I, F>), kB, sc.nblocks, kGridMult);          \
+        hist_grid = xcd_grid(hist_grid < kMaxHistGrid ? hist_grid : kMaxHistGrid);                                   \
+        sort_hist<I, F><<<hist_grid, kB, 0, s>>>(kin, p2c, kc, live, n_max, shift, sc.hist, sc.rem_block);           \
+    } while (0)
                 if (items == 4) { if (first) OPPX_HIST(4, true); else OPPX_HIST(4, false); }
                 else if (items == 8) { if (first) OPPX_HIST(8, true); else OPPX_HIST(8, false); }
                 else if (items == 16) { if (first) OPPX_HIST(16, true); else OPPX_HIST(16, false); }
                 else { if (first) OPPX_HIST(32, true); else OPPX_HIST(32, false); }
 #undef OPPX_HIST
                 OPPX_LAUNCH_CHECK("sort_hist");
-                const int64_t per_tile = (int64_t)kB * items;
-                scan_reduce<<<(unsigned)sc.scan_blocks, kB, 0, s>>>(sc.hist, counters, n_max, per_tile, sc.sums);
-                scan_sums<<<1, kB, 0, s>>>(sc.sums, counters, n_max, per_tile);
-                scan_apply<<<(unsigned)sc.scan_blocks, kB, 0, s>>>(sc.hist, counters, n_max, per_tile, sc.sums);
-                OPPX_LAUNCH_CHECK("sort_scan");
+                sort_rows<<<kBins + (first ? 1 : 0), kB, 0, s>>>(sc.hist, live, n_max, (int64_t)kB * items, sc.row_total,
+                                                                 sc.rem_block, hist_grid, sc.state);
+                OPPX_LAUNCH_CHECK("sort_rows");
 #define OPPX_SCATTER(I, LST, F)                                                                      \
     do {                                                                                              \
         auto kern = sort_scatter<I, LST, F>;                                                          \
         const unsigned res = resident_blocks(reinterpret_cast<const void*>(kern), kB);               \
-        const unsigned g = (int64_t)res < sc.nblocks ? res : (unsigned)sc.nblocks;                    \
-        kern<<<g, kB, 0, s>>>(kin, vin, p2c, kc, counters, n_max, shift, sc.hist, kout, vdst,            \
-                              p2c_out);                                                              \
+        const unsigned g = xcd_grid((int64_t)res < sc.nblocks ? res : (unsigned)sc.nblocks);           \
+        kern<<<g, kB, 0, s>>>(kin, vin, p2c, kc, sc.state, n_max, shift, sc.hist, sc.row_total, kout, vdst, \
+                              p2c_out, last && !gather ? finish : no_finish);                        \
     } while (0)
 #define OPPX_SCATTER_LF(I)                                                     \
     do {                                                                       \
@@ -544,13 +575,11 @@ int oppx_sort_by_cell(int64_t n_max, int64_t stride, oppx_move_counters* counter
             uint32_t* t = kin; kin = kout; kout = t;
             t = vin; vin = vout; vout = t;
         }
-        if (!direct && (T.n > 0 || perm_out)) {
-            sort_gather<<<grid_for(n_max, kB), kB, 0, s>>>(vin, counters, n_max, T, perm_out);
+        if (gather) {
+            sort_gather<<<grid_for(n_max, kB), kB, 0, s>>>(vin, sc.state, n_max, T, perm_out, finish);
             OPPX_LAUNCH_CHECK("sort_gather");
         }
     }
-    sort_finalize<<<1, 1, 0, s>>>(counters, n_max, sc.n_removed, drop_removed);
-    OPPX_LAUNCH_CHECK("sort_finalize");
     return OPPX_OK;
 }
 
@@ -574,7 +603,8 @@ int oppx_gather_dats(int64_t n_max, int64_t stride, const oppx_move_counters* co
     }
     if (n_max == 0) return OPPX_OK;
     sort_gather<<<grid_for(n_max, kB), kB, 0, as_stream(stream)>>>(reinterpret_cast<const uint32_t*>(perm),
-                                                                   counters, n_max, T, nullptr);
+                                                                   &counters->size, n_max, T, nullptr,
+                                                                   Finish{nullptr, nullptr, 0});
     OPPX_LAUNCH_CHECK("gather_dats");
     return OPPX_OK;
 }
