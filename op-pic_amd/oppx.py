@@ -245,6 +245,13 @@ def check(rc: int, what: str = ""):
         raise OppxError(f"{what} failed (rc={rc}): {msg}")
 
 
+def raw_stream(dev) -> int:
+    """torch's current stream on `dev` as the hipStream_t the C-ABI takes. The raw handle is asked for directly:
+    torch.cuda.current_stream() makes a Stream object of it, 3 us a call, several calls a step."""
+    import torch
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if dev.index is None else dev.index)
+
+
 def _ptr(a: np.ndarray):
     return a.ctypes.data_as(c_void_p)
 
@@ -486,7 +493,7 @@ class FempicDevice:
         if n and not ((p2c >= 0).all() and (p2c < nc).all()):
             raise ValueError("initial p2c entries out of [0, n_cells)")
         self.nc, self.nn = nc, nn
-        self._mesh_host = dict(n_cells=nc, n_nodes=nn, c2n=mesh["c2n"])
+        self._rows = {}  # the mesh's node rows, built at the first FP32 deposit and shared with every clone
         self.det = t(mesh["c_det"].reshape(-1), torch.float64)
         self.c_vol = t(mesh["c_vol"], torch.float64)
         self.c2c = t(mesh["c2c"].reshape(-1), torch.int32)
@@ -532,7 +539,7 @@ class FempicDevice:
         self.staged = False   # positions/velocities live in a 48-byte record buffer (pass_fused(stage=True))
 
     def stream(self):
-        return self.torch.cuda.current_stream(self.dev).cuda_stream
+        return raw_stream(self.dev)
 
     # attributes a clone gets afresh (the rest, the read-only mesh tensors and host metadata, it shares)
     _PER_INSTANCE = ("pos", "vel", "lc", "p2c", "counters", "hole_bits", "work", "scratch", "charge", "hops", "_swap",
@@ -548,11 +555,14 @@ class FempicDevice:
         g.__dict__.update({k: v for k, v in self.__dict__.items() if k not in self._PER_INSTANCE})
         g.pos, g.vel, g.lc, g.p2c = (t.clone() for t in (self.pos, self.vel, self.lc, self.p2c))
         g.counters = self.counters.clone()
-        for name in ("hole_bits", "work", "scratch", "charge", "hops"):
+        for name in ("hole_bits", "charge", "hops"):
             setattr(g, name, torch.zeros_like(getattr(self, name)))
-        if hasattr(self, "node_start"):  # the FP32 deposit's node rows are shared, its outputs are not
-            for name in ("cell_partials", "charge_f32", "dep_scratch"):
-                setattr(g, name, torch.zeros_like(getattr(self, name)))
+        for name in ("work", "scratch"):  # workspaces: nothing in them has to be set
+            setattr(g, name, torch.empty_like(getattr(self, name)))
+        if hasattr(self, "charge_f32"):  # the FP32 deposit's node rows are shared, its outputs are not
+            g.charge_f32 = torch.zeros_like(self.charge_f32)
+            for name in ("cell_partials", "dep_scratch"):
+                setattr(g, name, torch.empty_like(getattr(self, name)))
         g.pending = g.staged = False
         g._rebind()
         return g
@@ -585,9 +595,41 @@ class FempicDevice:
         if not hasattr(self, "_swap"):
             self._swap = [torch.empty_like(t) for t in (self.pos, self.vel, self.lc, self.p2c)]
             self.sort_scratch_bytes = int(lib().oppx_sort_scratch_bytes(self.cap))
-            self.sort_scratch = torch.zeros(self.sort_scratch_bytes, dtype=torch.uint8, device=self.dev)
-            self.perm = torch.zeros(self.cap, dtype=torch.int32, device=self.dev)
+            self.sort_scratch = torch.empty(self.sort_scratch_bytes, dtype=torch.uint8, device=self.dev)
+            self.perm = torch.empty(self.cap, dtype=torch.int32, device=self.dev)
         return self._swap
+
+    def _node_rows(self):
+        """(node_start, node_ref) of the FP32 deposit, as node_cell_csr gives them: node_ref lists the entries
+        4 c + k of c2n by node, ascending inside a node, which is the permutation of a stable sort of c2n by node,
+        and node_start[v] is the number of entries below v in the sorted c2n. Built on the device, once per mesh
+        (the host builder and its upload took a millisecond of every clone's first deposit at 50,000 nodes); the
+        build ends with a synchronisation, so every stream may read the rows afterwards."""
+        torch = self.torch
+        here = self.stream()
+        if "rows" not in self._rows:
+            L, n, s = lib(), 4 * self.nc, here
+            if n >= MAX_CELL_INDEX:
+                raise ValueError("4 n_cells beyond 32-bit row entries")
+            i32 = lambda k: torch.empty(k, dtype=torch.int32, device=self.dev)
+            live, ref, nodes = torch.zeros(COUNTER_WORDS, dtype=torch.int32, device=self.dev), i32(n), i32(n)
+            live[:1].fill_(n)
+            scratch = torch.empty(int(L.oppx_sort_scratch_bytes(n)), dtype=torch.uint8, device=self.dev)
+            check(L.oppx_sort_by_cell(n, n, live.data_ptr(), self.nn, self.c2n.data_ptr(),
+                                      self._descs([self.c2n], ("p2c",)), self._descs([nodes], ("p2c",)), 1,
+                                      ref.data_ptr(), 0, scratch.data_ptr(), scratch.numel(), s), "node_rows sort")
+            keys = torch.arange(self.nn + 1, dtype=torch.int32, device=self.dev)
+            start = torch.empty(self.nn + 1, dtype=torch.int64, device=self.dev)
+            check(L.oppx_lower_bound(n, live.data_ptr(), nodes.data_ptr(), keys.data_ptr(), self.nn + 1,
+                                     start.data_ptr(), s), "node_rows starts")
+            start = start.to(torch.int32)
+            torch.cuda.current_stream(self.dev).synchronize()
+            self._rows["rows"] = (start, ref, here)
+        start, ref, home = self._rows["rows"]
+        if here != home:  # the rows must outlive this stream's use of them
+            for t in (start, ref):
+                t.record_stream(torch.cuda.current_stream(self.dev))
+        return start, ref
 
     _DAT_SHAPES = {"pos": (3, 8), "vel": (3, 8), "lc": (4, 8), "p2c": (1, 4)}
 
@@ -675,14 +717,12 @@ class FempicDevice:
         else:
             self.materialize()
             p2c, lc = self.p2c, self.lc
-        if not hasattr(self, "node_start"):
-            st, ref = node_cell_csr(self._mesh_host)
-            self.node_start = torch.from_numpy(st).to(self.dev)
-            self.node_ref = torch.from_numpy(ref).to(self.dev)
-            self.cell_partials = torch.zeros(4 * self.nc, dtype=torch.float32, device=self.dev)
+        self.node_start, self.node_ref = self._node_rows()
+        if not hasattr(self, "charge_f32"):
+            self.cell_partials = torch.empty(4 * self.nc, dtype=torch.float32, device=self.dev)
             self.charge_f32 = torch.zeros(self.nn, dtype=torch.float32, device=self.dev)
             self.dep_bytes = int(lib().oppx_fempic_deposit_scratch_bytes(self.cap))
-            self.dep_scratch = torch.zeros(self.dep_bytes, dtype=torch.uint8, device=self.dev)
+            self.dep_scratch = torch.empty(self.dep_bytes, dtype=torch.uint8, device=self.dev)
         tail = (self.nc, self.node_start.data_ptr(), None, self.node_ref.data_ptr(), self.nn,
                 self.cell_partials.data_ptr(), None, self.charge_f32.data_ptr(), self.dep_scratch.data_ptr(),
                 self.dep_bytes, self.stream())
@@ -1029,7 +1069,7 @@ class NesoDevice:
         self.hops = torch.zeros(cap, dtype=torch.int32, device=self.dev)
 
     def stream(self):
-        return self.torch.cuda.current_stream(self.dev).cuda_stream
+        return raw_stream(self.dev)
 
     def step(self, dt, record_hops=False, do_update=True):
         flags = (1 if do_update else 0) | 2

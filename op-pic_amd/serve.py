@@ -186,7 +186,7 @@ class FempicArena:
         self.cap, self.size = P, 0
 
     def stream(self):
-        return self.torch.cuda.current_stream(self.dev).cuda_stream
+        return oppx.raw_stream(self.dev)
 
     def _t(self, a, dt):
         return self.torch.from_numpy(np.ascontiguousarray(a)).to(self.dev, dtype=dt)
