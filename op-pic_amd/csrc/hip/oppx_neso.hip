@@ -12,7 +12,11 @@
 namespace oppx {
 namespace {
 
-constexpr int kBlock = 256;
+// Threads per block. Every block adds to the one counters record at its end, and adds to one address from several
+// XCDs take some 10-20 ns each, one after the other: 2,048 blocks of 256 threads spent 20-40 us on that. Blocks of
+// 1024 make it 512: 1.5 M particles on the grid 61 -> 31 us, gathered 89 -> 64 us, 0.1 M gathered 18 -> 12.5 us.
+constexpr int kBlock = 1024;
+constexpr int kVerifyBlock = 256;
 
 struct NesoArgs {
     int64_t n_cells;
@@ -41,12 +45,17 @@ __device__ __forceinline__ double periodic_update(double p, double v, double dt,
     return fma(-ext, trunc(t / ext), t);
 }
 
+// The halves of a quad record as one load each; records are 8-byte aligned, no more.
+typedef double QuadHalf __attribute__((ext_vector_type(2), aligned(8)));
+typedef int QuadNb __attribute__((ext_vector_type(4), aligned(8)));
+
 // Particle state as one grid-stride iteration loads it.
 struct NesoPart {
     double x, y, vx, vy;
-    int cell, mx, my;
+    int cell;
 };
 
+// (The first evaluation sets the directions: the ones the particle comes with are not read.)
 __device__ __forceinline__ NesoPart neso_load(const NesoArgs& P, int flags, int64_t i) {
     const int64_t S = P.stride;
     NesoPart q;
@@ -57,120 +66,126 @@ __device__ __forceinline__ NesoPart neso_load(const NesoArgs& P, int flags, int6
         q.vx = __builtin_nontemporal_load(P.vel + i);
         q.vy = __builtin_nontemporal_load(P.vel + S + i);
     }
-    q.cell = kMaxCell;
-    q.mx = q.my = 0;
-    if (flags & OPPX_NESO_MOVE) {
-        q.cell = __builtin_nontemporal_load(P.p2c + i);
-        q.mx = __builtin_nontemporal_load(P.mdir + i);
-        q.my = __builtin_nontemporal_load(P.mdir + S + i);
-    }
+    q.cell = (flags & OPPX_NESO_MOVE) ? __builtin_nontemporal_load(P.p2c + i) : kMaxCell;
     return q;
 }
 
-// update_pos_kernel then move_kernel for particle i; returns the evaluations made.
+// A particle between the evaluations of its walk.
+struct NesoWalk {
+    double x, y;
+    int cell, mx, my, ix, iy, h;
+    bool on, fault;
+};
+
+// update_pos_kernel for particle i, and where its walk begins (on: it has one).
 template <bool GRID>
-__device__ __forceinline__ int neso_particle(const NesoArgs& P, int flags, int64_t i, NesoPart q, bool& fault) {
-    const int64_t S = P.stride;
-    int h = 0;
-    double x = q.x, y = q.y;
+__device__ __forceinline__ NesoWalk neso_begin(const NesoArgs& P, int flags, int64_t i, const NesoPart& q) {
+    NesoWalk w{q.x, q.y, q.cell, 0, 0, 0, 0, 0, false, false};
     if (flags & OPPX_NESO_UPDATE) {
-        x = periodic_update(x, q.vx, P.dt, P.ext_x);
-        y = periodic_update(y, q.vy, P.dt, P.ext_y);
-        __builtin_nontemporal_store(x, P.pos + i);
-        __builtin_nontemporal_store(y, P.pos + S + i);
+        w.x = periodic_update(w.x, q.vx, P.dt, P.ext_x);
+        w.y = periodic_update(w.y, q.vy, P.dt, P.ext_y);
+        __builtin_nontemporal_store(w.x, P.pos + i);
+        __builtin_nontemporal_store(w.y, P.pos + P.stride + i);
     }
-    int cell = q.cell;
-    if (cell == kMaxCell) return 0;
-    if (!((unsigned)cell < (unsigned)P.n_cells)) {
-        fault = true;
-        return 0;
-    }
-    int mx = q.mx, my = q.my;
-    const double cw = P.cw;
-    int ix = 0, iy = 0;
-    if (GRID) {
+    if (w.cell == kMaxCell) return w;
+    w.fault = !((unsigned)w.cell < (unsigned)P.n_cells);
+    w.on = !w.fault;
+    if (GRID && w.on) {
         // cell = ix + nx * iy: the quotient from one FP64 product, then corrected by one step
         // (the product's error stays below one for cells under 2^31)
-        iy = (int)((double)cell * P.inv_gnx);
-        ix = cell - iy * P.gnx;
-        if (ix < 0) { iy--; ix += P.gnx; }
-        else if (ix >= P.gnx) { iy++; ix -= P.gnx; }
+        w.iy = (int)((double)w.cell * P.inv_gnx);
+        w.ix = w.cell - w.iy * P.gnx;
+        if (w.ix < 0) { w.iy--; w.ix += P.gnx; }
+        else if (w.ix >= P.gnx) { w.iy++; w.ix -= P.gnx; }
     }
-    for (;;) {
-        double llx, lly;
-        int4 nb = make_int4(0, 0, 0, 0);
-        if (GRID) {
-            llx = (double)ix * cw;
-            lly = (double)iy * cw;
-        } else {
-            const oppx_quad_cell c = P.cells[cell];
-            llx = c.llx;
-            lly = c.lly;
-            nb = make_int4(c.c2c[0], c.c2c[1], c.c2c[2], c.c2c[3]);
-        }
-        const double dx = x - llx, dy = y - lly;
-        h++;
-        if (h == 1) {
-            const bool xp = ((dx > cw) && (P.ext_x > 2 * dx - cw)) || ((dx < 0) && (P.ext_x < cw - 2 * dx));
-            const bool yp = ((dy > cw) && (P.ext_y > 2 * dy - cw)) || ((dy < 0) && (P.ext_y < cw - 2 * dy));
-            mx = xp ? 1 : -1;
-            my = yp ? 1 : -1;
-        }
-        int next = 0;
-        bool hop = false;
-        if ((dx >= 0.0) && (dx <= cw)) mx = 0;
-        else if (mx > 0) { next = nb.y; hop = true; if (GRID) ix = grid_wrap(ix + 1, P.gnx); }
-        else if (mx < 0) { next = nb.x; hop = true; if (GRID) ix = grid_wrap(ix - 1, P.gnx); }
-        if (!hop) {
-            if ((dy >= 0.0) && (dy <= cw)) my = 0;
-            else if (my > 0) { next = nb.w; hop = true; if (GRID) iy = grid_wrap(iy + 1, P.gny); }
-            else if (my < 0) { next = nb.z; hop = true; if (GRID) iy = grid_wrap(iy - 1, P.gny); }
-        }
-        if (!hop) break;  // MOVE_DONE
-        if (GRID) next = ix + P.gnx * iy;
-        if (!((unsigned)next < (unsigned)P.n_cells) || h >= OPPX_MAX_HOPS) {
-            fault = true;
-            break;
-        }
-        cell = next;
-    }
-    __builtin_nontemporal_store(mx, P.mdir + i);
-    __builtin_nontemporal_store(my, P.mdir + S + i);
-    if (!fault) __builtin_nontemporal_store(cell, P.p2c + i);
-    return h;
+    return w;
 }
 
-// Resident grid, grid-stride over the particles, kNesoPerLane particles per lane per iteration (all
-// loaded before any is walked, so each lane keeps that many particles' loads in flight); the
-// per-block statistics then reach the counters from a few thousand blocks instead of one block per
-// 256 particles (same-address atomics serialise).
-constexpr int kNesoPerLane = 4;
+// One evaluation of move_kernel with the cell's corner (llx, lly) and neighbours nb (not read with GRID).
+template <bool GRID>
+__device__ __forceinline__ void neso_eval(const NesoArgs& P, NesoWalk& w, double llx, double lly, int4 nb) {
+    const double cw = P.cw;
+    const double dx = w.x - llx, dy = w.y - lly;
+    w.h++;
+    if (w.h == 1) {
+        const bool xp = ((dx > cw) && (P.ext_x > 2 * dx - cw)) || ((dx < 0) && (P.ext_x < cw - 2 * dx));
+        const bool yp = ((dy > cw) && (P.ext_y > 2 * dy - cw)) || ((dy < 0) && (P.ext_y < cw - 2 * dy));
+        w.mx = xp ? 1 : -1;
+        w.my = yp ? 1 : -1;
+    }
+    int next = 0;
+    bool hop = false;
+    if ((dx >= 0.0) && (dx <= cw)) w.mx = 0;
+    else if (w.mx > 0) { next = nb.y; hop = true; if (GRID) w.ix = grid_wrap(w.ix + 1, P.gnx); }
+    else if (w.mx < 0) { next = nb.x; hop = true; if (GRID) w.ix = grid_wrap(w.ix - 1, P.gnx); }
+    if (!hop) {
+        if ((dy >= 0.0) && (dy <= cw)) w.my = 0;
+        else if (w.my > 0) { next = nb.w; hop = true; if (GRID) w.iy = grid_wrap(w.iy + 1, P.gny); }
+        else if (w.my < 0) { next = nb.z; hop = true; if (GRID) w.iy = grid_wrap(w.iy - 1, P.gny); }
+    }
+    if (!hop) {  // MOVE_DONE
+        w.on = false;
+        return;
+    }
+    if (GRID) next = w.ix + P.gnx * w.iy;
+    if (!((unsigned)next < (unsigned)P.n_cells) || w.h >= OPPX_MAX_HOPS) {
+        w.fault = true;
+        w.on = false;
+        return;
+    }
+    w.cell = next;
+}
 
+__device__ __forceinline__ void neso_end(const NesoArgs& P, int64_t i, const NesoWalk& w) {
+    if (w.h == 0) return;  // no walk: removed, or a cell out of range
+    __builtin_nontemporal_store(w.mx, P.mdir + i);
+    __builtin_nontemporal_store(w.my, P.mdir + P.stride + i);
+    if (!w.fault) __builtin_nontemporal_store(w.cell, P.p2c + i);
+}
+
+// Resident grid, grid-stride over the particles, PER particles per lane per iteration, all loaded before any is
+// walked, so each lane keeps that many particles' loads in flight. Two where the walk computes its records (50
+// VGPRs, two blocks per CU; four take 76 and one block: 32 M particles 549 and 685 us), one where it gathers them:
+// there the waves in flight are what hides a walk's chain of dependent reads (16 M particles on 1024 x 1024 cells
+// 1,021 us; two walks a lane advancing together 1,149, four 1,379).
 template <bool GRID>
 __global__ void __launch_bounds__(kBlock) neso_step_kernel(NesoArgs P, int flags) {
+    constexpr int PER = GRID ? 2 : 1;
     int64_t n = P.ctr->size;
     n = n < 0 ? 0 : (n > P.n_max ? P.n_max : n);
     long long hsum = 0;
     int hmax = 0, nfault = 0;
     const int64_t stride = (int64_t)gridDim.x * kBlock;
-    for (int64_t i0 = (int64_t)blockIdx.x * kBlock + threadIdx.x; i0 < n; i0 += kNesoPerLane * stride) {
-        NesoPart part[kNesoPerLane];
+    for (int64_t i0 = (int64_t)blockIdx.x * kBlock + threadIdx.x; i0 < n; i0 += PER * stride) {
+        NesoPart part[PER];
 #pragma unroll
-        for (int u = 0; u < kNesoPerLane; u++) {
+        for (int u = 0; u < PER; u++) {
             const int64_t i = i0 + u * stride;
             part[u] = i < n ? neso_load(P, flags, i) : NesoPart{};
         }
 #pragma unroll
-        for (int u = 0; u < kNesoPerLane; u++) {
+        for (int u = 0; u < PER; u++) {
             const int64_t i = i0 + u * stride;
-            if (i < n) {
-                bool f = false;
-                const int h = neso_particle<GRID>(P, flags, i, part[u], f);
-                if (P.hops && (flags & OPPX_NESO_MOVE)) P.hops[i] = h;
-                hsum += h;
-                hmax = hmax > h ? hmax : h;
-                nfault += f ? 1 : 0;
+            if (i >= n) continue;
+            NesoWalk w = neso_begin<GRID>(P, flags, i, part[u]);
+            while (w.on) {
+                if (GRID) {
+                    neso_eval<true>(P, w, (double)w.ix * P.cw, (double)w.iy * P.cw, int4{});
+                } else {
+                    const QuadHalf ll = *reinterpret_cast<const QuadHalf*>(P.cells + w.cell);
+                    const QuadNb n4 = *reinterpret_cast<const QuadNb*>(P.cells[w.cell].c2c);
+                    int4 nb = make_int4(n4.x, n4.y, n4.z, n4.w);
+                    // both halves of the record at once: left to itself the compiler reads the one neighbour it
+                    // needs after the corner has arrived, a second trip in the chain (64 -> 76 us above)
+                    asm volatile("" : "+v"(nb.x), "+v"(nb.y), "+v"(nb.z), "+v"(nb.w));
+                    neso_eval<false>(P, w, ll.x, ll.y, nb);
+                }
             }
+            neso_end(P, i, w);
+            if (P.hops && (flags & OPPX_NESO_MOVE)) P.hops[i] = w.h;
+            hsum += w.h;
+            hmax = hmax > w.h ? hmax : w.h;
+            nfault += w.fault ? 1 : 0;
         }
     }
     __shared__ long long s_sum[kBlock / kWave];
@@ -185,6 +200,7 @@ __global__ void __launch_bounds__(kBlock) neso_step_kernel(NesoArgs P, int flags
         int m = 0, f = 0;
         for (int q = 0; q < kBlock / kWave; q++) { t += s_sum[q]; m = m > s_max[q] ? m : s_max[q]; f += s_flt[q]; }
         if (t) atomicAdd((unsigned long long*)&P.ctr->total_hops, (unsigned long long)t);
+        // the maximum only grows: a block whose own does not pass what it reads has nothing to add
         if (m) atomicMax(&P.ctr->max_hops, m);
         if (f) atomicAdd(&P.ctr->faults, f);
     }
@@ -277,7 +293,7 @@ int neso_step_impl(int64_t n_max, const oppx_neso_parts* parts, const oppx_quad_
 // (ix, iy) = (g mod nx, g div nx), or when a coordinate lies outside [ll, ll + cell_width] with
 // ll = ix * cell_width (a product then a sum: the reference build forms them apart, no FMA). Block
 // sums of the count are added to *count.
-__global__ void __launch_bounds__(kBlock) neso_verify_kernel(int64_t n_max, int64_t stride, const double* __restrict__ pos,
+__global__ void __launch_bounds__(kVerifyBlock) neso_verify_kernel(int64_t n_max, int64_t stride, const double* __restrict__ pos,
                                                              const int32_t* __restrict__ p2c,
                                                              const int32_t* __restrict__ c_gbl_idx, int64_t n_cells,
                                                              int nx, double cw, const oppx_move_counters* __restrict__ ctr,
@@ -285,7 +301,7 @@ __global__ void __launch_bounds__(kBlock) neso_verify_kernel(int64_t n_max, int6
     int64_t n = ctr->size;
     n = n < 0 ? 0 : (n > n_max ? n_max : n);
     int bad = 0, flt = 0;
-    for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kBlock) {
+    for (int64_t i = (int64_t)blockIdx.x * kVerifyBlock + threadIdx.x; i < n; i += (int64_t)gridDim.x * kVerifyBlock) {
         const int c = p2c[i];
         if (!((unsigned)c < (unsigned)n_cells)) {  // the reference would read outside c_idx
             flt++;
@@ -305,7 +321,7 @@ __global__ void __launch_bounds__(kBlock) neso_verify_kernel(int64_t n_max, int6
         const double lly = (double)iy * cw, y = pos[stride + i];
         if (y < lly || y > lly + cw) bad++;
     }
-    __shared__ int s_bad[kBlock / kWave], s_flt[kBlock / kWave];
+    __shared__ int s_bad[kVerifyBlock / kWave], s_flt[kVerifyBlock / kWave];
     bad = wave_sum_i32(bad);
     flt = wave_sum_i32(flt);
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
@@ -313,7 +329,7 @@ __global__ void __launch_bounds__(kBlock) neso_verify_kernel(int64_t n_max, int6
     __syncthreads();
     if (threadIdx.x == 0) {
         int b = 0, f = 0;
-        for (int q = 0; q < kBlock / kWave; q++) { b += s_bad[q]; f += s_flt[q]; }
+        for (int q = 0; q < kVerifyBlock / kWave; q++) { b += s_bad[q]; f += s_flt[q]; }
         if (b) atomicAdd(count, b);
         if (f && faults) atomicAdd(faults, f);
     }
@@ -369,9 +385,9 @@ int oppx_neso_verify(int64_t n_max, int64_t stride, const double* pos, const int
     OPPX_ARG_CHECK(nx > 0 && n_cells > 0 && n_cells < kMaxCell, "oppx_neso_verify: nx or n_cells out of range");
     if (n_max == 0) return OPPX_OK;
     OPPX_ARG_CHECK(pos && p2c && c_gbl_idx, "oppx_neso_verify: null array");
-    unsigned g = grid_for(n_max, kBlock);
+    unsigned g = grid_for(n_max, kVerifyBlock);
     if (g > 4096) g = 4096;
-    neso_verify_kernel<<<g, kBlock, 0, as_stream(stream)>>>(n_max, stride, pos, p2c, c_gbl_idx, n_cells, nx, cell_width,
+    neso_verify_kernel<<<g, kVerifyBlock, 0, as_stream(stream)>>>(n_max, stride, pos, p2c, c_gbl_idx, n_cells, nx, cell_width,
                                                             counters, count, &counters->faults);
     OPPX_LAUNCH_CHECK("neso_verify");
     return OPPX_OK;
