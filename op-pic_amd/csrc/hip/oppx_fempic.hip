@@ -10,8 +10,6 @@
 // c_det + a 32 B aux record per hop). Blocks are remapped so each XCD walks one contiguous
 // eighth of the particle range.
 
-#include <type_traits>
-
 #include "oppx_internal.h"
 
 namespace oppx {
@@ -86,15 +84,8 @@ template <typename T>
 __device__ __forceinline__ T ld_stream(const T* p) { return __builtin_nontemporal_load(p); }
 template <typename T>
 __device__ __forceinline__ void st_stream(T* p, T v) { __builtin_nontemporal_store(v, p); }
-// a 48-byte position/velocity record {x, y, z, vx, vy, vz} as three 16-byte stores; ordinary (cached)
-// stores, so that L2 merges a wave's three partial-line writes into whole lines before they leave
+
 typedef double f64x2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ void st_record(double* rec, double x, double y, double z, double vx, double vy, double vz) {
-    f64x2* r = reinterpret_cast<f64x2*>(rec);
-    r[0] = f64x2{x, y};
-    r[1] = f64x2{z, vx};
-    r[2] = f64x2{vy, vz};
-}
 
 // Tile walk: per-block statistics go to one of kSlots slots (blockIdx modulo kSlots) instead of the single
 // counters record: thousands of blocks adding to one address serialise in one L2 channel. The
@@ -361,33 +352,19 @@ enum HopResult { kHopInside = 0, kHopMove = 1, kHopExit = 2, kHopBad = 3 };
 
 // One evaluation of apps/app_fempic/kernels.h:106-161 at `cell`: inside -> kHopInside; otherwise
 // cell becomes the face neighbour of the most negative weight (first index wins ties), or
-// kMaxCell when that face is on the boundary. In two steps, the cell's records (its 128 B c_det line
-// and 32 B aux record) and the evaluation, so that the records can also come from LDS.
-struct HopRec {
-    double2 a[8];  // c_det: alpha, beta ; gamma, delta of vertices 0..3
-    double4 au;    // {c2, c2c[0..1], c2c[2..3], pad}
-};
-
-__device__ __forceinline__ void hop_load(const StepArgs& P, int cell, HopRec& R) {
-    const double2* __restrict__ d = reinterpret_cast<const double2*>(P.det + 16 * (int64_t)cell);
-#pragma unroll
-    for (int q = 0; q < 8; q++) R.a[q] = d[q];
-    R.au = *reinterpret_cast<const double4*>(P.aux + cell);
+// kMaxCell when that face is on the boundary. In two steps, the four weights and what follows from them, so
+// that the cell's records (its 128 B c_det line and 32 B aux record {c2, c2c[0..1], c2c[2..3], pad}) can come
+// from global memory or from LDS.
+__device__ __forceinline__ double hop_weight(double c2, double2 ab, double2 gd, double x, double y, double z) {
+    return c2 * fma(-gd.y, z, fma(gd.x, y, fma(-ab.y, x, ab.x)));  // alpha, beta ; gamma, delta of one vertex
 }
 
-__device__ __forceinline__ int hop_calc(const StepArgs& P, const HopRec& R, double x, double y, double z, int& cell,
-                                        double& l0, double& l1, double& l2, double& l3) {
-    const double2 a0 = R.a[0], a1 = R.a[1], a2 = R.a[2], a3 = R.a[3], a4 = R.a[4], a5 = R.a[5], a6 = R.a[6],
-                  a7 = R.a[7];
-    const double c2 = R.au.x;
-    l0 = c2 * fma(-a1.y, z, fma(a1.x, y, fma(-a0.y, x, a0.x)));
-    l1 = c2 * fma(-a3.y, z, fma(a3.x, y, fma(-a2.y, x, a2.x)));
-    l2 = c2 * fma(-a5.y, z, fma(a5.x, y, fma(-a4.y, x, a4.x)));
-    l3 = c2 * fma(-a7.y, z, fma(a7.x, y, fma(-a6.y, x, a6.x)));
+__device__ __forceinline__ int hop_choose(const StepArgs& P, double c2c01, double c2c23, int& cell, double l0, double l1,
+                                          double l2, double l3) {
     if ((l0 > -1e-10) && ((l0 - 1.0) < 1e-10) && (l1 > -1e-10) && ((l1 - 1.0) < 1e-10) && (l2 > -1e-10) &&
         ((l2 - 1.0) < 1e-10) && (l3 > -1e-10) && ((l3 - 1.0) < 1e-10))
         return kHopInside;
-    const int2 n01 = __builtin_bit_cast(int2, R.au.y), n23 = __builtin_bit_cast(int2, R.au.z);
+    const int2 n01 = __builtin_bit_cast(int2, c2c01), n23 = __builtin_bit_cast(int2, c2c23);
     int nb = n01.x;
     double ml = l0;
     if (l1 < ml) { ml = l1; nb = n01.y; }
@@ -404,9 +381,14 @@ __device__ __forceinline__ int hop_calc(const StepArgs& P, const HopRec& R, doub
 
 __device__ __forceinline__ int hop_eval(const StepArgs& P, double x, double y, double z, int& cell, double& l0,
                                         double& l1, double& l2, double& l3) {
-    HopRec R;
-    hop_load(P, cell, R);
-    return hop_calc(P, R, x, y, z, cell, l0, l1, l2, l3);
+    const double2* __restrict__ d = reinterpret_cast<const double2*>(P.det + 16 * (int64_t)cell);
+    const double2 a0 = d[0], a1 = d[1], a2 = d[2], a3 = d[3], a4 = d[4], a5 = d[5], a6 = d[6], a7 = d[7];
+    const double4 au = *reinterpret_cast<const double4*>(P.aux + cell);
+    l0 = hop_weight(au.x, a0, a1, x, y, z);
+    l1 = hop_weight(au.x, a2, a3, x, y, z);
+    l2 = hop_weight(au.x, a4, a5, x, y, z);
+    l3 = hop_weight(au.x, a6, a7, x, y, z);
+    return hop_choose(P, au.y, au.z, cell, l0, l1, l2, l3);
 }
 
 // How an evaluation's result ends a walk of the first pass (h evaluations so far): kWalkOn (still moving),
@@ -419,61 +401,93 @@ __device__ __forceinline__ int walk_state(int r, int h, int inline_hops) {
     return h >= inline_hops ? kWalkHandOff : kWalkOn;
 }
 
-// Cell records shared by a block's walks. Sorted particles cluster in a few cells, and a wave's
-// record loads are bound by the addresses the vector memory unit processes (one per lane per 16-byte
-// load), so in the first kCacheRounds evaluations each distinct cell of the block is fetched once,
-// 160 bytes by ten lanes, into LDS, and every lane of that cell reads it from there. A lane whose cell
-// finds no slot (kCacheProbe probes) loads its own records. One round of 64 slots (10.5 KB, inside the
-// deposit table's LDS) measured best: a second round's barriers cost more than its loads save.
-constexpr int kCacheBits = 6;
-constexpr int kCacheSlots = 1 << kCacheBits;
-constexpr int kCacheProbe = 16;
-constexpr int kCacheRounds = 1;
-struct CellCache {
-    int key[kCacheSlots];
-    double2 rec[kCacheSlots][10];  // c_det (8 pairs), aux (2 pairs)
+// The first pass's walks, wave by wave: the lanes still moving need 160 bytes of cell records each, and loading
+// them lane by lane (ten 16-byte loads at 64 unrelated lines each) kept the vector memory unit's addresser busy
+// nine tenths of the pass. Here the wave's lanes fetch the records together, straight into LDS
+// (global_load_lds, 16 bytes a lane): eight lanes take one 128-byte c_det line and two lanes one aux record, so one
+// instruction brings 8 lines, or 32 aux records, whole, and needs no registers for them. Only as many records as there
+// are lanes still moving are fetched, and neighbouring lanes in one cell share one (without an overlay, a sorted
+// wave starts in a handful of cells). The buffer holds 32 records: with the 21 KB of a block seven blocks fit a
+// CU; a wave with more goes twice. In LDS the 16-byte chunk q of record r sits at q ^ (r & 7), so that lanes
+// reading the same chunk of consecutive records meet different banks. The weights are computed one vertex at a time
+// and the particle index is recomputed after the push (an opaque copy), which keeps the kernel at 72 registers and
+// seven waves per SIMD without spills; five waves (natural, 95 registers) were slower than the lane-wise loads.
+// Measured, 24 M particles in 3 M tets (a pass over sorted, one- and two-steps-old particles): 1,551 / 1,771 / 2,063 us
+// with lane-wise loads behind a block cache of the first evaluation's cells, 1,433 / 1,575 / 1,859 us so (without
+// the deposit 1,346 / 1,491 / 1,608 and 1,190 / 1,283 / 1,388), and 1,868 -> 1,739 us through a sort's permutation;
+// 3 M: 195 / 219 / 236 -> 181 / 199 / 218 us. 24 or 16 records at eight waves (64 registers, 4-6 spilled): 1,750 /
+// 1,875 / 2,154 us and more.
+constexpr int kCoopRecs = 32;
+struct CoopBuf {
+    double2 det[kCoopRecs * 8];
+    double2 aux[kCoopRecs * 2];
+    int cell[kCoopRecs];
 };
 
-__device__ __forceinline__ int cache_insert(CellCache& C, int cell) {
-    uint32_t h = ((uint32_t)cell * 2654435761u) >> (32 - kCacheBits);
-    for (int p = 0; p < kCacheProbe; p++) {
-        const int k = C.key[h];
-        if (k == cell) return (int)h;
-        if (k == -1) {
-            const int prev = atomicCAS(&C.key[h], -1, cell);
-            if (prev == -1 || prev == cell) return (int)h;
-        }
-        h = (h + 1) & (kCacheSlots - 1);
-    }
-    return -1;
+// 16 bytes per lane from `src` (the lane's own) to dst + 16 * lane (dst wave-uniform), asynchronously.
+__device__ __forceinline__ void load_to_lds(const void* src, void* dst) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                     (__attribute__((address_space(3))) void*)dst, 16, 0, 0);
 }
 
-__device__ __forceinline__ void cache_fill(const StepArgs& P, CellCache& C) {
-    for (int c = threadIdx.x; c < kCacheSlots * 10; c += blockDim.x) {
-        const int sl = c / 10, q = c - 10 * sl;
-        const int key = C.key[sl];
-        if (key >= 0) {
-            const double2* src = q < 8 ? reinterpret_cast<const double2*>(P.det + 16 * (int64_t)key) + q
-                                       : reinterpret_cast<const double2*>(P.aux + key) + (q - 8);
-            C.rec[sl][q] = *src;
-        }
-    }
-}
-
-__device__ __forceinline__ void cache_read(const CellCache& C, int sl, HopRec& R) {
+// Walks the wave's moving lanes until each has ended, or has made inline_hops evaluations.
+__device__ __forceinline__ void coop_walk(const StepArgs& P, CoopBuf& C, bool moving, int lane, double x, double y, double z,
+                                          int& cell, double& l0, double& l1, double& l2, double& l3, int& h, int& walk,
+                                          int inline_hops) {
+    static_assert(kCoopRecs % 8 == 0 && kCoopRecs <= 32, "an aux load brings 32 records");
+    unsigned long long m;
+    while ((m = __ballot(moving)) != 0ull) {
+        const int prev = __shfl_up(cell, 1);
+        const bool lead = moving && (lane == 0 || !((m >> (lane - 1)) & 1ull) || prev != cell);
+        const unsigned long long leads = __ballot(lead);
+        const int rank = __popcll(leads & ((2ull << lane) - 1ull)) - 1;  // the record of a moving lane
+        const int total = __popcll(leads);
+        for (int base = 0; base < total; base += kCoopRecs) {
+            const int cnt = total - base < kCoopRecs ? total - base : kCoopRecs;
+            const int r = rank - base;
+            const bool mine = ((m >> lane) & 1ull) && r >= 0 && r < cnt;
+            if (mine && lead) C.cell[r] = cell;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
 #pragma unroll
-    for (int q = 0; q < 8; q++) R.a[q] = C.rec[sl][q];
-    const double2 u0 = C.rec[sl][8], u1 = C.rec[sl][9];
-    R.au = double4{u0.x, u0.y, u1.x, u1.y};
+            for (int q = 0; q < kCoopRecs / 8; q++) {
+                const int rec = q * 8 + (lane >> 3);
+                if (rec < cnt)
+                    load_to_lds(P.det + 16 * (int64_t)C.cell[rec] + 2 * ((lane & 7) ^ (rec & 7)), &C.det[q * 64]);
+            }
+            if ((lane >> 1) < cnt)
+                load_to_lds(reinterpret_cast<const double*>(P.aux + C.cell[lane >> 1]) + 2 * (lane & 1), C.aux);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the records are in LDS
+            if (mine) {
+                const double2 a0 = C.aux[2 * r];
+                const char* row = reinterpret_cast<const char*>(C.det + 8 * r);
+                const int sw = (r & 7) << 4;
+                double l[4];
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const double2 ab = *reinterpret_cast<const double2*>(row + ((32 * v) ^ sw));
+                    const double2 gd = *reinterpret_cast<const double2*>(row + ((32 * v + 16) ^ sw));
+                    l[v] = hop_weight(a0.x, ab, gd, x, y, z);
+                    __builtin_amdgcn_sched_barrier(0);  // one vertex's coefficients in registers at a time
+                }
+                l0 = l[0]; l1 = l[1]; l2 = l[2]; l3 = l[3];
+                const int res = hop_choose(P, a0.y, C.aux[2 * r + 1].x, cell, l0, l1, l2, l3);
+                h++;
+                walk = walk_state(res, h, inline_hops);
+                moving = walk == kWalkOn;
+            }
+            // every value read above has been used, so the next batch may overwrite the buffer
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
+    }
 }
 
-// LDS of a 256-thread first-pass block: the record staging, the cell cache and the deposit table in turn
-// (side by side, 22.8 KB instead of 12 KB, the pass measured 1-3% slower).
+// LDS of a first-pass block: the record staging, the waves' fetch buffers and the deposit table in turn.
+template <int BS>
 union FirstLds {
     DepositTable dep;
-    CellCache cache;
+    double2 stage[3 * BS];
+    CoopBuf coop[BS / kWave];
 };
-static_assert(sizeof(CellCache) <= sizeof(DepositTable), "the cell cache lives inside the deposit table's LDS");
 
 // What the first pass leaves for the walk pass: one record per block, and the blocks' worklists, `parts`
 // (the particles of a block) entries {particle, hops so far} each.
@@ -484,7 +498,7 @@ struct WorkList {
 };
 
 template <int BS, bool PUSH, bool DH, bool DEPOSIT, bool BATCH, bool GATHER>
-__global__ void __launch_bounds__(BS) fempic_first_kernel(StepArgs P, uint32_t nblocks, int inline_hops, WorkList W) {
+__global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(7))) fempic_first_kernel(StepArgs P, uint32_t nblocks, int inline_hops, WorkList W) {
     int64_t n = P.ctr->size;
     n = n < 0 ? 0 : (n > P.n_max ? P.n_max : n);
     // workgroups past the blocks of live particles (the grid is sized by the host's bound) leave at
@@ -495,7 +509,7 @@ __global__ void __launch_bounds__(BS) fempic_first_kernel(StepArgs P, uint32_t n
     __shared__ int s_pending;
     if (threadIdx.x == 0) s_pending = 0;  // a barrier comes before its first use
     const uint32_t b = xcd_block(blockIdx.x, nlive);
-    const int64_t i = (int64_t)b * BS + threadIdx.x;
+    int64_t i = (int64_t)b * BS + threadIdx.x;
     const bool live = i < n;
     const int64_t S = P.stride;
     const int lane = threadIdx.x & (kWave - 1);
@@ -505,15 +519,16 @@ __global__ void __launch_bounds__(BS) fempic_first_kernel(StepArgs P, uint32_t n
     // streamed particle loads are non-temporal; loads through a permutation are ordinary cached
     // loads, so the neighbours of a gathered word still find its line in L2
     auto ld = [](const auto* p) { return GATHER ? *p : ld_stream(p); };
-    int64_t src = i;
+    uint32_t from = (uint32_t)i;
     bool fault = false;
     if (GATHER && live) {
-        src = P.perm[i];
-        if (!((uint64_t)src < (uint64_t)S)) {  // a corrupt permutation entry: report, touch nothing
+        from = (uint32_t)P.perm[i];
+        if (!((uint64_t)from < (uint64_t)S)) {  // a corrupt permutation entry: report, touch nothing
             fault = true;
-            src = i;
+            from = (uint32_t)i;
         }
     }
+    int64_t src = from;
 
     // the sort may have written the sorted p2c into the target already (src_p2c null): read in place
     const bool p2c_in_place = GATHER && P.src_p2c == nullptr;
@@ -525,10 +540,8 @@ __global__ void __launch_bounds__(BS) fempic_first_kernel(StepArgs P, uint32_t n
     bool removed = false, pending = false, pushed = false, p2c_done = false, lc_done = false;
     int h = 0;
     double l0 = 0.0, l1 = 0.0, l2 = 0.0, l3 = 0.0;
-    constexpr bool CACHE = BS == kBlock;
-    using Lds = std::conditional_t<CACHE, FirstLds, DepositTable>;
-    __shared__ Lds s_lds;
-    DepositTable& s_table = *reinterpret_cast<DepositTable*>(&s_lds);
+    __shared__ FirstLds<BS> s_lds;
+    DepositTable& s_table = s_lds.dep;
 
     // push: the particle's new position and velocity (or, for a particle this pass does not push, the
     // ones it carries over)
@@ -598,34 +611,35 @@ __global__ void __launch_bounds__(BS) fempic_first_kernel(StepArgs P, uint32_t n
             }
         }
     }
-    // records out (block-uniform): every live particle's {x, y, z, vx, vy, vz}. With 256-thread blocks the
-    // wave's 64 records pass through LDS (the deposit table's storage, not yet in use) so that each of
-    // the three 16-byte stores of a lane lands next to its neighbours' (1 KB contiguous per instruction)
+    // records out (block-uniform): every live particle's {x, y, z, vx, vy, vz}. The wave's 64 records pass through
+    // LDS so that each of the three 16-byte stores of a lane lands next to its neighbours' (1 KB contiguous per
+    // instruction)
     if (P.rec_out) {
-        if constexpr (BS * 48 <= (int)sizeof(Lds)) {
-            const int wave = threadIdx.x / kWave;
-            f64x2* slice = reinterpret_cast<f64x2*>(&s_lds) + wave * (3 * kWave);
-            if (live) {
-                slice[3 * lane] = f64x2{x, y};
-                slice[3 * lane + 1] = f64x2{z, vx};
-                slice[3 * lane + 2] = f64x2{vy, vz};
-            }
-            __syncthreads();
-            const int64_t base = (int64_t)b * BS + wave * kWave;  // first particle of the wave
-            const int64_t nw = n - base;                          // live particles of the wave
-            f64x2* dst = reinterpret_cast<f64x2*>(P.rec_out + 6 * base);
-            for (int k = 0; k < 3; k++) {
-                const int q = k * kWave + lane;  // pair q of the wave's 192: record q / 3
-                if (q / 3 < nw) __builtin_nontemporal_store(slice[q], dst + q);
-            }
-            __syncthreads();
-        } else if (live) {
-            st_record(P.rec_out + 6 * i, x, y, z, vx, vy, vz);
+        const int wave = threadIdx.x / kWave;
+        f64x2* slice = reinterpret_cast<f64x2*>(s_lds.stage) + wave * (3 * kWave);
+        if (live) {
+            slice[3 * lane] = f64x2{x, y};
+            slice[3 * lane + 1] = f64x2{z, vx};
+            slice[3 * lane + 2] = f64x2{vy, vz};
+        }
+        __syncthreads();
+        const int64_t base = (int64_t)b * BS + wave * kWave;  // first particle of the wave
+        const int64_t nw = n - base;                          // live particles of the wave
+        f64x2* dst = reinterpret_cast<f64x2*>(P.rec_out + 6 * base);
+        for (int k = 0; k < 3; k++) {
+            const int q = k * kWave + lane;  // pair q of the wave's 192: record q / 3
+            if (q / 3 < nw) __builtin_nontemporal_store(slice[q], dst + q);
         }
     }
-    if constexpr (!CACHE) {
-        if (DEPOSIT) table_clear(s_table);
-        __syncthreads();
+    __syncthreads();  // the staging's readers are done, and s_pending is set
+    {   // the indexes, opaque: addresses formed above are not kept in registers across the walk
+        uint32_t at = (uint32_t)i;
+        asm volatile("" : "+v"(at));
+        i = at;
+        if (GATHER) {
+            asm volatile("" : "+v"(from));
+            src = from;
+        }
     }
 
     // direct hop
@@ -639,43 +653,13 @@ __global__ void __launch_bounds__(BS) fempic_first_kernel(StepArgs P, uint32_t n
         }
         moving = !removed && !fault;
     }
-    // walk: the block's first evaluations through the cell cache (every thread takes part in its barriers),
-    // then each lane on its own
-    if constexpr (CACHE) {
-        CellCache& C = s_lds.cache;
-        for (int round = 0; round < kCacheRounds; round++) {
-            __syncthreads();  // the LDS's last users (record staging, the previous round's readers) are done
-            for (int q = threadIdx.x; q < kCacheSlots; q += BS) C.key[q] = -1;
-            if (!__syncthreads_or(moving)) break;  // a barrier (the keys are clear), the same on every thread
-            const int sl = moving ? cache_insert(C, cell) : -1;
-            __syncthreads();
-            cache_fill(P, C);
-            __syncthreads();
-            if (moving) {
-                HopRec R;
-                if (sl >= 0) cache_read(C, sl, R);
-                else hop_load(P, cell, R);
-                const int r = hop_calc(P, R, x, y, z, cell, l0, l1, l2, l3);
-                h++;
-                walk = walk_state(r, h, inline_hops);
-                moving = walk == kWalkOn;
-            }
-        }
-    }
-    while (moving) {
-        const int r = hop_eval(P, x, y, z, cell, l0, l1, l2, l3);
-        h++;
-        walk = walk_state(r, h, inline_hops);
-        moving = walk == kWalkOn;
-    }
+    coop_walk(P, s_lds.coop[threadIdx.x / kWave], moving, lane, x, y, z, cell, l0, l1, l2, l3, h, walk, inline_hops);
     removed = removed || walk == kWalkOut;
     fault = fault || walk == kWalkBad;
     pending = walk == kWalkHandOff;
-    if constexpr (CACHE) {
-        if (DEPOSIT) {
-            __syncthreads();  // the cache's readers are done with the LDS
-            table_clear(s_table);
-        }
+    if (DEPOSIT) {
+        __syncthreads();  // every wave is done with its fetch buffer
+        table_clear(s_table);
     }
     if (go) {
         if (!fault) {
