@@ -27,6 +27,7 @@ struct DhView {
 
 struct StepArgs {
     int64_t n_cells;
+    int64_t n_nodes;
     const double* __restrict__ det;
     const oppx_tet_aux* __restrict__ aux;
     const int32_t* __restrict__ c2n;
@@ -102,8 +103,9 @@ struct StatSlot {
 struct BlockStat {
     unsigned long long hops;
     int max_hops, removed, faults;
-    int pending;  // worklist entries of the block
+    int pending;  // worklist entries of the block; kScattered: none, and the walk pass deposits its particles
 };
+constexpr int kScattered = -1;
 
 // The block's totals, valid in thread 0 (ends with the other threads free to leave).
 __device__ __forceinline__ BlockStat block_totals(long long hsum, int hmax, int nrem, int nfault) {
@@ -240,24 +242,31 @@ __device__ __forceinline__ void table_clear(DepositTable& T) {
     }
 }
 
-__device__ __forceinline__ void table_add(DepositTable& T, double* __restrict__ charge, int node, double v) {
-    uint32_t h = ((((uint32_t)node / kLine) * 2654435761u) >> 26) * kLine + (uint32_t)node % kLine;
+__device__ __forceinline__ uint32_t table_slot(int node) {
+    return ((((uint32_t)node / kLine) * 2654435761u) >> 26) * kLine + (uint32_t)node % kLine;
+}
+
+enum TableAdd { kOldEntry = 0, kNewEntry = 1, kNoEntry = 2 };  // kNoEntry: the value went to global memory
+
+__device__ __forceinline__ int table_add(DepositTable& T, double* __restrict__ charge, int node, double v) {
+    uint32_t h = table_slot(node);
     for (int p = 0; p < kProbe; p++) {
         const int k = T.key[h];
         if (k == node) {
             atomicAdd(&T.val[h], v);
-            return;
+            return kOldEntry;
         }
         if (k == -1) {
             const int prev = atomicCAS(&T.key[h], -1, node);
             if (prev == -1 || prev == node) {
                 atomicAdd(&T.val[h], v);
-                return;
+                return prev == -1 ? kNewEntry : kOldEntry;
             }
         }
         h = (h + kProbeStep) & (kTable - 1);
     }
     atomicAdd(charge + node, v);
+    return kNoEntry;
 }
 
 __device__ __forceinline__ void table_flush(DepositTable& T, double* __restrict__ charge) {
@@ -509,7 +518,7 @@ struct WorkList {
     int parts;
 };
 
-template <int BS, bool PUSH, bool DH, bool DEPOSIT, bool BATCH, bool GATHER>
+template <int BS, bool PUSH, bool DH, bool DEPOSIT, bool BATCH, bool GATHER, bool DENSE>
 __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(7))) fempic_first_kernel(StepArgs P, uint32_t nblocks, int inline_hops, WorkList W) {
     int64_t n = P.ctr->size;
     n = n < 0 ? 0 : (n > P.n_max ? P.n_max : n);
@@ -519,7 +528,9 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(7))) fe
     if (P.reset && blockIdx.x == 0 && threadIdx.x == 0) reset_counters(P.ctr);
     if (blockIdx.x >= nlive) return;
     __shared__ int s_pending;
-    if (threadIdx.x == 0) s_pending = 0;  // a barrier comes before its first use
+    __shared__ unsigned s_order;  // deposits << 12 + new first nodes; from kKeep on: the table stays
+    constexpr unsigned kKeep = 1u << 28;
+    if (threadIdx.x == 0) s_pending = s_order = 0;  // a barrier comes before their first use
     const uint32_t b = xcd_block(blockIdx.x, nlive);
     int64_t i = (int64_t)b * BS + threadIdx.x;
     const bool live = i < n;
@@ -702,17 +713,34 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(7))) fe
         if (pending)
             W.entry[(int64_t)blockIdx.x * BS + base + __popcll(pmask & ((1ull << lane) - 1ull))] = make_int2((int)i, h);
     }
+    bool scattered = false;  // of the block
     if (DEPOSIT) {
+        const bool give = live && !skip && !fault && !removed && !pending;
         __syncthreads();  // table cleared
-        if (live && !skip && !fault && !removed && !pending) {
-            const int4 m = *reinterpret_cast<const int4*>(P.c2n + 4 * (int64_t)cell);
-            table_add(s_table, P.charge, m.x, l0);
-            table_add(s_table, P.charge, m.y, l1);
-            table_add(s_table, P.charge, m.z, l2);
-            table_add(s_table, P.charge, m.w, l3);
+        int4 m = make_int4(0, 0, 0, 0);
+        if (give) m = *reinterpret_cast<const int4*>(P.c2n + 4 * (int64_t)cell);
+        if constexpr (DENSE) {
+            // Particles in no order: nearly every one of them brings a first node that no other has. The block then
+            // forgets its table and leaves its deposit to the walk pass -- unless something has left the table
+            // already, or the walk pass could not tell which particles deposit.
+            const int first = give ? table_add(s_table, P.charge, m.x, l0) : kOldEntry;
+            const int gives = __popcll(__ballot(give)), news = __popcll(__ballot(first == kNewEntry));
+            const bool keep = __ballot(fault || pending || first == kNoEntry) != 0ull;
+            if (lane == 0) atomicAdd(&s_order, keep ? kKeep : ((unsigned)gives << 12) + (unsigned)news);
+            __syncthreads();
+            const unsigned order = s_order, all = order >> 12;
+            scattered = order < kKeep && all >= 64 && 4 * (order & 0xFFFu) > 3 * all;
         }
-        __syncthreads();
-        table_flush(s_table, P.charge);
+        if (!scattered) {
+            if (give) {
+                if (!DENSE) table_add(s_table, P.charge, m.x, l0);
+                table_add(s_table, P.charge, m.y, l1);
+                table_add(s_table, P.charge, m.z, l2);
+                table_add(s_table, P.charge, m.w, l3);
+            }
+            __syncthreads();
+            table_flush(s_table, P.charge);
+        }
     }
     // removal bitmap: one word per wave, written for every word the grid covers
     const unsigned long long rmask = __ballot(live && removed);
@@ -720,7 +748,7 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(7))) fe
     const bool done = live && !skip && !pending;
     BlockStat t = block_totals(done ? h : 0, done ? h : 0, (live && removed) ? 1 : 0, fault ? 1 : 0);
     if (threadIdx.x == 0) {
-        t.pending = s_pending;
+        t.pending = scattered ? kScattered : s_pending;
         W.rec[blockIdx.x] = t;
     }
 }
@@ -949,8 +977,16 @@ __global__ void __launch_bounds__(kQuadBlock) fempic_quad_kernel(StepArgs P, uin
 // `per` first-pass blocks at a time, all of one XCD (first-pass block p ran on XCD p % 8), and walks their
 // entries as one dense list: 256 where the first pass walks (nearly) everything itself and the records are
 // all there is to read, few where it hands over many entries and the grid should spread them.
-template <bool DEPOSIT>
-__global__ void __launch_bounds__(kBlock) fempic_walk_kernel(StepArgs P, WorkList W, uint32_t nblocks, int per) {
+// DENSE: it also deposits the particles of the first-pass blocks that found theirs scattered. A block then holds the
+// whole charge array in LDS, adds to it there, and adds it to the global one at its end, consecutive lanes to
+// consecutive nodes. Scattered adds to global memory go at 20 a nanosecond over the chip, such a sweep at 100, and LDS
+// takes 16,384 scattered adds a CU in 8 us: 1 M particles in no order on 9,261 nodes,
+// a fused pass 234 -> 114 us; 6 M on 15,625: 1,046 -> 632 us; 1 M in cell order (no block scattered) 70 -> 73 us.
+template <bool DEPOSIT, bool DENSE>
+__global__ void __launch_bounds__(DENSE ? kMaxBlock : kBlock) fempic_walk_kernel(StepArgs P, WorkList W, uint32_t nblocks,
+                                                                                 int per) {
+    constexpr int BT = DENSE ? kMaxBlock : kBlock;
+    extern __shared__ double s_dense[];
     int64_t n = P.ctr->size;
     n = n < 0 ? 0 : (n > P.n_max ? P.n_max : n);
     const uint32_t nlive = live_blocks(n, W.parts, nblocks);
@@ -958,20 +994,57 @@ __global__ void __launch_bounds__(kBlock) fempic_walk_kernel(StepArgs P, WorkLis
     const uint32_t chunks = (mine + per - 1) / per;
     const int64_t S = P.stride;
     __shared__ DepositTable s_table;
-    __shared__ int s_off[kBlock], s_wave[kBlock / kWave];
+    __shared__ int s_off[BT], s_wave[BT / kWave];
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
 
     long long hsum = 0;
     int hmax = 0, nrem = 0, nfault = 0;
-    for (uint32_t c = blockIdx.x / kXcds; c < chunks; c += gridDim.x / kXcds) {
-        const uint32_t first = x + kXcds * c * (uint32_t)per;  // first-pass blocks first, first + 8, ...
-        BlockStat t{0ull, 0, 0, 0, 0};
-        if ((int)threadIdx.x < per && c * (uint32_t)per + threadIdx.x < mine) t = W.rec[first + kXcds * threadIdx.x];
+    bool used = false;  // s_dense holds something (uniform over the block)
+    auto take = [&](const BlockStat& t) {
         hsum += (long long)t.hops;
         hmax = hmax > t.max_hops ? hmax : t.max_hops;
         nrem += t.removed;
         nfault += t.faults;
+    };
+    if (DENSE && blockIdx.x < 2 * kXcds)  // its chunks are many and small: a few blocks add up all the records
+        for (uint32_t q = blockIdx.x * BT + threadIdx.x; q < nlive; q += 2 * kXcds * BT) take(W.rec[q]);
+    for (uint32_t c = blockIdx.x / kXcds; c < chunks; c += gridDim.x / kXcds) {
+        const uint32_t first = x + kXcds * c * (uint32_t)per;  // first-pass blocks first, first + 8, ...
+        BlockStat t{0ull, 0, 0, 0, 0};
+        if ((int)threadIdx.x < per && c * (uint32_t)per + threadIdx.x < mine) t = W.rec[first + kXcds * threadIdx.x];
+        if (!DENSE) take(t);
         if (!__syncthreads_or(t.pending)) continue;  // the usual case: nothing was handed over
+        if constexpr (DENSE) {
+            s_off[threadIdx.x] = t.pending;
+            if (__syncthreads_or(t.pending == kScattered)) {
+                if (!used) {
+                    for (int64_t q = threadIdx.x; q < P.n_nodes; q += BT) s_dense[q] = 0.0;
+                    used = true;
+                    __syncthreads();
+                }
+                for (int e = threadIdx.x; e < per * kBlock; e += BT) {
+                    const int k = e / kBlock;  // the chunk's k-th first-pass block
+                    if (s_off[k] != kScattered) continue;
+                    const int64_t i = (int64_t)xcd_block(first + kXcds * (uint32_t)k, nlive) * kBlock + e % kBlock;
+                    if (i >= n) continue;
+                    const int cell = ld_stream(P.p2c + i);
+                    const double l0 = ld_stream(P.lc + i), l1 = ld_stream(P.lc + S + i),
+                                 l2 = ld_stream(P.lc + 2 * S + i), l3 = ld_stream(P.lc + 3 * S + i);
+                    if (!((unsigned)cell < (unsigned)P.n_cells)) continue;  // removed
+                    const int4 m = *reinterpret_cast<const int4*>(P.c2n + 4 * (int64_t)cell);
+                    auto add = [&](int node, double v) {
+                        if ((uint64_t)node < (uint64_t)P.n_nodes) atomicAdd(&s_dense[node], v);
+                        else atomicAdd(P.charge + node, v);
+                    };
+                    add(m.x, l0);
+                    add(m.y, l1);
+                    add(m.z, l2);
+                    add(m.w, l3);
+                }
+            }
+            __syncthreads();
+            t.pending = t.pending == kScattered ? 0 : t.pending;
+        }
         int inc = t.pending;  // exclusive scan of the worklist lengths over the block
 #pragma unroll
         for (int d = 1; d < kWave; d <<= 1) {
@@ -981,14 +1054,14 @@ __global__ void __launch_bounds__(kBlock) fempic_walk_kernel(StepArgs P, WorkLis
         if (lane == kWave - 1) s_wave[wave] = inc;
         __syncthreads();
         int off = 0, total = 0;
-        for (int q = 0; q < kBlock / kWave; q++) {
+        for (int q = 0; q < BT / kWave; q++) {
             if (q < wave) off += s_wave[q];
             total += s_wave[q];
         }
         s_off[threadIdx.x] = off + inc - t.pending;
-        // block-uniform rounds of kBlock entries; with the deposit, the LDS table is flushed after every
+        // block-uniform rounds of BT entries; with the deposit, the LDS table is flushed after every
         // round so that it never fills (a full table sends every further add to a global atomic)
-        for (int base = 0; base < total; base += kBlock) {
+        for (int base = 0; base < total; base += BT) {
             if (DEPOSIT) table_clear(s_table);
             __syncthreads();  // table cleared, offsets written
             const int e = base + (int)threadIdx.x;
@@ -1041,6 +1114,14 @@ __global__ void __launch_bounds__(kBlock) fempic_walk_kernel(StepArgs P, WorkLis
                 table_flush(s_table, P.charge);
                 __syncthreads();
             }
+        }
+    }
+    if (DENSE && used) {
+        __syncthreads();
+        const int64_t from = P.n_nodes * blockIdx.x / gridDim.x;  // blocks start at different nodes
+        for (int64_t q = threadIdx.x; q < P.n_nodes; q += BT) {
+            const int64_t node = q + from < P.n_nodes ? q + from : q + from - P.n_nodes;
+            if (s_dense[node] != 0.0) atomicAdd(P.charge + node, s_dense[node]);
         }
     }
     block_stats(P, hsum, hmax, nrem, nfault);
@@ -1335,6 +1416,7 @@ int fill_args(StepArgs& P, const oppx_fempic_parts* parts, const oppx_tet_mesh* 
     OPPX_ARG_CHECK(parts->stride >= 0, "fempic: negative stride");
     P = StepArgs{};
     P.n_cells = mesh->n_cells;
+    P.n_nodes = mesh->n_nodes;
     P.det = mesh->det;
     P.aux = mesh->aux;
     P.c2n = mesh->c2n;
@@ -1380,6 +1462,8 @@ void launch_tile(const StepArgs& P, int64_t n_max, hipStream_t s) {
     kern<<<g, kBlock, 0, s>>>(P, nbt);
 }
 
+constexpr int kDenseNodes = 16384;  // nodes of the largest LDS charge copy (128 KB)
+
 // Work buffer of the move. Tile walk: statistics slots [kSlots]. Two-pass move: one record per block of the
 // first pass (64, 256 or 1024 particles), then the blocks' worklists.
 constexpr size_t kSlotBytes = kSlots * sizeof(StatSlot);
@@ -1412,6 +1496,11 @@ bool launch_two_pass(const StepArgs& P, int64_t n_max, void* work, size_t work_b
     if (!work || g_tuning.inline_hops < 1 || work_bytes < work_need(n_max)) return false;
     WorkList W{reinterpret_cast<BlockStat*>(work),
                reinterpret_cast<int2*>(reinterpret_cast<char*>(work) + record_bytes(n_max)), kBlock};
+    // Scattered blocks' deposits through LDS copies of the charge: 256 blocks sweep n_nodes adds each at 100 a
+    // nanosecond where the particles' adds would go at 20, so from some 14 particles a node on; 32, to be clear of
+    // the second read of lc and p2c. A copy fits a CU's LDS beside the rest up to 16,384 nodes.
+    const bool dense = DEPOSIT && g_tuning.lanes == 1 && g_tuning.first_block == kBlock && P.n_nodes > 0 &&
+                       P.n_nodes <= kDenseNodes && n_max >= 32 * P.n_nodes && n_max >= (1 << 18);
     unsigned g;
     if (g_tuning.lanes == 4) {
         W.parts = kQuadParts;
@@ -1420,21 +1509,36 @@ bool launch_two_pass(const StepArgs& P, int64_t n_max, void* work, size_t work_b
     } else if (g_tuning.first_block == kMaxBlock) {
         W.parts = kMaxBlock;
         g = grid_for(n_max, kMaxBlock);
-        fempic_first_kernel<kMaxBlock, PUSH, DH, DEPOSIT, BATCH, GATHER><<<g, kMaxBlock, 0, s>>>(P, g, g_tuning.inline_hops, W);
+        fempic_first_kernel<kMaxBlock, PUSH, DH, DEPOSIT, BATCH, GATHER, false>
+            <<<g, kMaxBlock, 0, s>>>(P, g, g_tuning.inline_hops, W);
     } else {
         g = grid_for(n_max, kBlock);
-        fempic_first_kernel<kBlock, PUSH, DH, DEPOSIT, BATCH, GATHER><<<g, kBlock, 0, s>>>(P, g, g_tuning.inline_hops, W);
+        auto first = fempic_first_kernel<kBlock, PUSH, DH, DEPOSIT, BATCH, GATHER, false>;
+        if constexpr (DEPOSIT) {
+            if (dense) first = fempic_first_kernel<kBlock, PUSH, DH, true, BATCH, GATHER, true>;
+        }
+        first<<<g, kBlock, 0, s>>>(P, g, g_tuning.inline_hops, W);
     }
     // A first pass that walks 16 evaluations itself hands over next to nothing: 256 records a walk block, at most
-    // 256 blocks (each adds to the one counters record). Below that the walk spreads over the resident grid.
+    // 256 blocks (each adds to the one counters record). Below that the walk spreads over the resident grid. With dense
+    // deposits 8 records, 2048 particles, a block, one block a CU.
     const bool rare = g_tuning.inline_hops >= 16;
-    const int per = rare ? kBlock : 8;
-    auto walk = fempic_walk_kernel<DEPOSIT>;
-    const unsigned cap = rare ? 256u : resident_blocks(reinterpret_cast<const void*>(walk), kBlock);
+    const int per = rare && !dense ? kBlock : 8;
+    const void* plain = reinterpret_cast<const void*>(fempic_walk_kernel<DEPOSIT, false>);
+    const unsigned cap = rare || dense ? 256u : resident_blocks(plain, kBlock);
     unsigned wg = ((g + kXcds - 1) / kXcds + per - 1) / per * kXcds;  // every chunk of every XCD
     if (wg > cap) wg = cap / kXcds * kXcds;
     if (wg < (unsigned)kXcds) wg = kXcds;
-    walk<<<wg, kBlock, 0, s>>>(P, W, g, per);
+    if constexpr (DEPOSIT) {
+        if (dense) {
+            const size_t bytes = (size_t)P.n_nodes * sizeof(double);
+            (void)hipFuncSetAttribute(reinterpret_cast<const void*>(fempic_walk_kernel<true, true>),
+                                      hipFuncAttributeMaxDynamicSharedMemorySize, kDenseNodes * (int)sizeof(double));
+            fempic_walk_kernel<true, true><<<wg, kMaxBlock, bytes, s>>>(P, W, g, per);
+            return true;
+        }
+    }
+    fempic_walk_kernel<DEPOSIT, false><<<wg, kBlock, 0, s>>>(P, W, g, per);
     return true;
 }
 
