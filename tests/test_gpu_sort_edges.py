@@ -21,6 +21,8 @@ def _restore_tuning():
 @pytest.mark.parametrize("live,bound,n_cells", [
     (0, 1, 5), (1, 1, 1), (1, 300_000, 300), (1023, 1024, 255), (1025, 4097, 256), (4096, 4096, 70_000),
     (32_769, 40_000, 65_535), (300_001, 2_000_000, 17_000_000), (5_000_000, 5_000_001, 1_000_003),
+    (300_001, 1 << 20, 17_000_000), (9_000, 12_000_001, 255), (40_000, 12_000_000, 70_000),
+    (1_300_000, 12_000_000, 1_000_003),  # the bounds from which a tile takes more keys per thread
 ])
 def test_gpu_sort_edges(items, live, bound, n_cells):
     oppx.set_tuning(**dict(DEFAULT, sort_items=items))
