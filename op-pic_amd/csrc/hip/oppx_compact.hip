@@ -27,7 +27,7 @@ constexpr int kB = 256;
 constexpr int kMaxDats = 16;
 constexpr int kMaxComps = 64;   // components one fill launch moves (more take further launches)
 constexpr int kMaxGroups = 4096;  // group prefixes a fill block holds in LDS
-constexpr int kCopyBatch = 8;   // components loaded before any of them is stored
+constexpr int kCopyBatch = 12;  // components loaded before any of them is stored (a FEM-PIC particle has 11)
 
 // The dats as single components: base address of each, and which of them have 8-byte elements.
 struct CompTable {

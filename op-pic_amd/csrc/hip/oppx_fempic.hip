@@ -1006,14 +1006,28 @@ __global__ void __launch_bounds__(DENSE ? kMaxBlock : kBlock) fempic_walk_kernel
         nrem += t.removed;
         nfault += t.faults;
     };
-    if (DENSE && blockIdx.x < 2 * kXcds)  // its chunks are many and small: a few blocks add up all the records
-        for (uint32_t q = blockIdx.x * BT + threadIdx.x; q < nlive; q += 2 * kXcds * BT) take(W.rec[q]);
+    if constexpr (DENSE) {
+        if (blockIdx.x < 2 * kXcds)  // its chunks are many and small: a few blocks add up all the records
+            for (uint32_t q = blockIdx.x * BT + threadIdx.x; q < nlive; q += 2 * kXcds * BT) take(W.rec[q]);
+    } else {  // the records of the block's chunks, without a barrier between them
+        int any = 0;
+#pragma unroll 4
+        for (uint32_t c = blockIdx.x / kXcds; c < chunks; c += gridDim.x / kXcds) {
+            if ((int)threadIdx.x >= per || c * (uint32_t)per + threadIdx.x >= mine) continue;
+            const BlockStat t = W.rec[x + kXcds * (c * (uint32_t)per + threadIdx.x)];
+            take(t);
+            any |= t.pending;
+        }
+        if (!__syncthreads_or(any)) {  // the usual case: nothing was handed over
+            block_stats(P, hsum, hmax, nrem, nfault);
+            return;
+        }
+    }
     for (uint32_t c = blockIdx.x / kXcds; c < chunks; c += gridDim.x / kXcds) {
         const uint32_t first = x + kXcds * c * (uint32_t)per;  // first-pass blocks first, first + 8, ...
         BlockStat t{0ull, 0, 0, 0, 0};
         if ((int)threadIdx.x < per && c * (uint32_t)per + threadIdx.x < mine) t = W.rec[first + kXcds * threadIdx.x];
-        if (!DENSE) take(t);
-        if (!__syncthreads_or(t.pending)) continue;  // the usual case: nothing was handed over
+        if (!__syncthreads_or(t.pending)) continue;
         if constexpr (DENSE) {
             s_off[threadIdx.x] = t.pending;
             if (__syncthreads_or(t.pending == kScattered)) {
@@ -1520,12 +1534,12 @@ bool launch_two_pass(const StepArgs& P, int64_t n_max, void* work, size_t work_b
         first<<<g, kBlock, 0, s>>>(P, g, g_tuning.inline_hops, W);
     }
     // A first pass that walks 16 evaluations itself hands over next to nothing: 256 records a walk block, at most
-    // 256 blocks (each adds to the one counters record). Below that the walk spreads over the resident grid. With dense
+    // 64 blocks (each adds to the one counters record; 94,000 records: 9.0 us, with 256 blocks 13.4). Below that the walk spreads over the resident grid. With dense
     // deposits 8 records, 2048 particles, a block, one block a CU.
     const bool rare = g_tuning.inline_hops >= 16;
     const int per = rare && !dense ? kBlock : 8;
     const void* plain = reinterpret_cast<const void*>(fempic_walk_kernel<DEPOSIT, false>);
-    const unsigned cap = rare || dense ? 256u : resident_blocks(plain, kBlock);
+    const unsigned cap = dense ? 256u : (rare ? 64u : resident_blocks(plain, kBlock));
     unsigned wg = ((g + kXcds - 1) / kXcds + per - 1) / per * kXcds;  // every chunk of every XCD
     if (wg > cap) wg = cap / kXcds * kXcds;
     if (wg < (unsigned)kXcds) wg = kXcds;
