@@ -7,8 +7,8 @@
 // One lane per particle on a resident grid; each block walks one contiguous run of 256-particle
 // tiles. Deposits go into a workgroup LDS table keyed by cell (ds_add_f64), flushed with one
 // device-scope atomic per (cell, entry) every few tiles: particles of one cell share a block, so this
-// removes most of the global atomics; a wave whose first evaluations all deposit into one cell sums
-// them with shuffles first. The arithmetic is the reference GCC build's, FMA for FMA (the file is built with
+// removes most of the global atomics; the first evaluations of a wave that deposit into one cell are
+// summed in registers first. The arithmetic is the reference GCC build's, FMA for FMA (the file is built with
 // -ffp-contract=off): the interpolated fields and the Boris cross products are FMA chains, the
 // half-advance products stay unfused (their second use lies past the errno branch GCC places around
 // sqrt), v5 = q*ux*uy*uz/3 is fused into all twelve accumulator terms and v1 = v4*d into both of
@@ -22,6 +22,8 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kCabTable = 64;  // cells per workgroup table (a 256-particle tile spans a few)
 constexpr int kCabProbe = 8;
+constexpr int kCabGroups = 2;   // cells of a wave whose deposits are summed in registers
+constexpr int kCabShare = 8;    // lanes from which on that is done
 constexpr int kCabFlushTiles = 4;  // tiles of one block between table flushes
 
 struct CabArgs {
@@ -78,6 +80,75 @@ __device__ __forceinline__ void cab_table_add(CabTable& T, double* __restrict__ 
     }
 #pragma unroll
     for (int j = 0; j < 12; j++) atomicAdd(acc + 12 * (int64_t)cell + j, v[j]);
+}
+
+// ---- sums over the lanes of a wave, in registers ----
+// Two 32-bit words of a and of b swapped between the wave's halves (or between the even and odd rows of 16 lanes): a
+// then holds [a.low, b.low] and b [a.high, b.high], so that a + b is a's sum in the low half and b's in the high one.
+template <bool ROWS>
+__device__ __forceinline__ double swap_add(double a, double b) {
+    const uint2 x = __builtin_bit_cast(uint2, a), y = __builtin_bit_cast(uint2, b);
+    unsigned p0, q0, p1, q1;
+    if constexpr (ROWS) {
+        const auto lo = __builtin_amdgcn_permlane16_swap(x.x, y.x, false, false);
+        const auto hi = __builtin_amdgcn_permlane16_swap(x.y, y.y, false, false);
+        p0 = lo[0]; q0 = lo[1]; p1 = hi[0]; q1 = hi[1];
+    } else {
+        const auto lo = __builtin_amdgcn_permlane32_swap(x.x, y.x, false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap(x.y, y.y, false, false);
+        p0 = lo[0]; q0 = lo[1]; p1 = hi[0]; q1 = hi[1];
+    }
+    return __builtin_bit_cast(double, make_uint2(p0, p1)) + __builtin_bit_cast(double, make_uint2(q0, q1));
+}
+
+// x plus the value N lanes on in the row of 16 (DPP row rotation).
+template <int N>
+__device__ __forceinline__ double row_add(double x) {
+    const int2 w = __builtin_bit_cast(int2, x);
+    const int lo = __builtin_amdgcn_update_dpp(0, w.x, 0x120 + N, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, w.y, 0x120 + N, 0xF, 0xF, false);
+    return x + __builtin_bit_cast(double, make_int2(lo, hi));
+}
+
+// Adds the twelve values of the lanes in `mask` (wave-uniform, not empty), whose particles all deposit into `cell`
+// (wave-uniform), to the cell's entry. Called by whole waves. Each exchange halves the values a lane carries: twelve to six across the wave's
+// halves, six to three across the rows of 16, then three sums inside the rows -- 63 vector instructions where summing
+// every value over the whole wave by shuffles took 144 LDS-crossbar moves. Row r then holds values 3 r .. 3 r + 2,
+// and twelve lanes add one each.
+__device__ __forceinline__ void cab_wave_add(CabTable& T, double* __restrict__ acc, int cell, unsigned long long mask, int lane,
+                                             const double* v) {
+    const bool in = (mask >> lane) & 1ull;
+    double w[6];
+#pragma unroll
+    for (int j = 0; j < 6; j++) w[j] = swap_add<false>(in ? v[j] : 0.0, in ? v[j + 6] : 0.0);
+    double x[3];
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        x[j] = swap_add<true>(w[j], w[j + 3]);
+        x[j] = row_add<8>(x[j]);
+        x[j] = row_add<4>(x[j]);
+        x[j] = row_add<2>(x[j]);
+        x[j] = row_add<1>(x[j]);
+    }
+    uint32_t h = ((uint32_t)cell * 2654435761u) >> 26;
+    int slot = -1;
+    for (int p = 0; p < kCabProbe && slot < 0; p++) {
+        int k = __builtin_amdgcn_readfirstlane(T.key[h]);
+        if (k == -1) {
+            int prev = 0;
+            if (lane == 0) prev = atomicCAS(&T.key[h], -1, cell);
+            prev = __builtin_amdgcn_readfirstlane(prev);
+            k = prev == -1 ? cell : prev;
+        }
+        if (k == cell) slot = (int)h;
+        h = (h + 1) & (kCabTable - 1);
+    }
+    const int q = lane & 15, j = 3 * (lane >> 4) + q;
+    if (q < 3) {
+        const double t = q == 0 ? x[0] : (q == 1 ? x[1] : x[2]);
+        if (slot >= 0) atomicAdd(&T.val[slot][j], t);
+        else atomicAdd(acc + 12 * (int64_t)cell + j, t);
+    }
 }
 
 // Flushes the used entries and leaves the table cleared for the next tile (the caller separates the
@@ -264,26 +335,22 @@ __global__ void __launch_bounds__(kBlock) cabana_move_deposit_kernel(CabArgs P) 
                 }
             }
         }
-        // First-evaluation deposits: in cell order nearly every wave's particles share one cell, and
-        // 64 lanes adding to the same 12 LDS words would serialise; such a wave sums its 12 values
-        // with a butterfly and one lane adds them. A wave spanning several cells adds lane by lane.
-        const unsigned long long has = __ballot(c1st >= 0);
-        if (has) {
-            const int lead = __shfl(c1st, __ffsll((long long)has) - 1);
-            if ((has & ~__ballot(c1st == lead)) == 0ull) {
-                double sum[12];
-#pragma unroll
-                for (int j = 0; j < 12; j++) {
-                    double x = c1st >= 0 ? v1st[j] : 0.0;
-#pragma unroll
-                    for (int o = 1; o < kWave; o <<= 1) x += __shfl_xor(x, o);
-                    sum[j] = x;
-                }
-                if (lane == 0) cab_table_add(T, P.acc, lead, sum);
-            } else if (c1st >= 0) {
-                cab_table_add(T, P.acc, c1st, v1st);
-            }
+        // First-evaluation deposits: in cell order a wave's particles share one cell, or a few (two streams that
+        // have moved apart), and 64 lanes adding to the same 12 LDS words would serialise: the lanes of up to
+        // kCabGroups cells are summed in registers, cell by cell, the rest add lane by lane. The step, us, with
+        // shuffles and waves of one cell only, and now: 9 M particles in 12,000 cells 363 -> 316 (without any
+        // first-evaluation deposit 314: what is left streams 160 bytes a particle), 750 k in 1,000 cells 55 -> 49,
+        // 164 k in 4,096 cells 34 -> 30, 28 k in 13,824 cells 22 -> 22. One cell instead of two: 34 at the third;
+        // four cells, or cells of 4 lanes: no faster.
+        unsigned long long left = __ballot(c1st >= 0);
+        for (int group = 0; group < kCabGroups && left; group++) {
+            const int lead = __builtin_amdgcn_readlane(c1st, __ffsll((long long)left) - 1);
+            const unsigned long long mask = __ballot(c1st == lead);  // lead >= 0: lanes without a deposit hold -1
+            if (__popcll(mask) < kCabShare) break;
+            cab_wave_add(T, P.acc, lead, mask, lane, v1st);
+            left &= ~mask;
         }
+        if ((left >> lane) & 1ull) cab_table_add(T, P.acc, c1st, v1st);
         // later streaks: each evaluation deposits one streak and hops across the face it ends on
         while (active) {
             h++;
