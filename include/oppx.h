@@ -168,6 +168,23 @@ int oppx_fill_pattern(void* dst, int64_t n, int dim, int elem_bytes, const void*
 int oppx_offset_indices(int32_t* base, int64_t n_records, int rec_ints, int first, int count, int32_t offset,
                         void* stream);
 
+/* One job of oppx_copy_batch: `rows` rows of `bytes` bytes each, dst_stride / src_stride bytes apart (not read when
+ * rows == 1), copied from src, or filled with the 8 bytes of `fill` over and over when src is NULL (each row starts
+ * at its first byte). With add != 0 the copied words are indices to rebase as oppx_offset_indices does: the words
+ * [first, first+count) of every record of rec_ints (a power of two up to 128), counted from the row's start. */
+typedef struct oppx_copy_job {
+    void* dst;
+    const void* src;
+    int64_t bytes, rows, dst_stride, src_stride;
+    uint64_t fill;
+    int32_t add, rec_ints, first, count;
+} oppx_copy_job;
+
+/* Runs n jobs in one launch for every 32 rows (a kernel, so it can be graph-captured). Pointers are device memory or
+ * pinned host memory, and with sizes and strides multiples of 4. Jobs may run in any order: none may write what
+ * another one touches; src == dst (rebasing in place) is allowed. No reference counterpart. */
+int oppx_copy_batch(int n, const oppx_copy_job* jobs, void* stream);
+
 /* AoS (host layout, doc/api.rst:115-118) <-> SoA (device layout) transposes on the device,
  * replacing the host transposes of opp_lib/src/hip/opp_hip_utils.cpp:35-153. */
 int oppx_aos_to_soa(const void* aos, void* soa, int64_t n, int dim, int64_t stride, int elem_bytes, void* stream);

@@ -3,6 +3,7 @@
 // conversions of opp_lib/src/hip/opp_hip_utils.cpp:35-153, which here run on the device.
 
 #include <cstring>
+#include <type_traits>
 
 #include "oppx_internal.h"
 
@@ -89,6 +90,93 @@ __global__ void offset_indices_kernel(int32_t* __restrict__ base, int64_t n, int
             const int32_t v = p[k];
             if (v >= 0 && v != kMaxCell) p[k] = v + offset;
         }
+    }
+}
+
+// ---- many copies and fills in one launch ----
+// Small copies are bound by their launches (2 us each on the device, 8 to 10 us apart from a Python caller), large ones
+// by HBM. Admitting a request took 21 copies, fills and rebasing passes, handing it back 11, a clone 9; each is one
+// launch now: five requests admitted 560 -> 200 us and handed back 900 -> 620 us (of which 20 MB over the host link at
+// 54 GB/s take 350), a clone of 3,000 particles 89 -> 39 us, one of 24 M 807 -> 746. 1.92 GB in 10 rows: 671 us with
+// 2 units in flight a thread, 697 with 4, 722 with 8 (the runtime's own copy 775).
+constexpr int kSegs = 32;      // row segments a launch takes (their table is a kernel argument)
+constexpr int kSegBlock = 256;
+constexpr int kSegUnits = 2;   // units a thread has in flight
+constexpr int64_t kMaxGrid = 1 << 30;
+
+// One contiguous piece of memory: `units` units of 1 << shift bytes and the words behind them.
+struct CopySeg {
+    unsigned char* dst;
+    const unsigned char* src;  // nullptr: the two words of `fill` over and over
+    int64_t units;
+    uint32_t fill[2];
+    uint32_t block0;           // its first block
+    int32_t add;
+    uint8_t shift, tail, mask, first, count;
+};
+
+struct CopyTable {
+    CopySeg s[kSegs];
+    int n;
+};
+
+template <int W>
+struct Words {
+    uint32_t w[W];
+};
+
+// The words of one unit that hold indices, moved by S.add; w0 is the unit's first word in the segment.
+template <int W>
+__device__ __forceinline__ void rebase(Words<W>& v, int64_t w0, const CopySeg& S) {
+#pragma unroll
+    for (int k = 0; k < W; k++) {
+        const unsigned m = (unsigned)(w0 + k) & S.mask;
+        const int x = (int)v.w[k];
+        if (m - S.first < S.count && x >= 0 && x != kMaxCell) v.w[k] = (uint32_t)(x + S.add);
+    }
+}
+
+template <int W>
+__device__ __forceinline__ void copy_units(const CopySeg& S, int64_t first_unit) {
+    using V = std::conditional_t<W == 4, uint4, std::conditional_t<W == 2, uint2, uint32_t>>;
+    int64_t u[kSegUnits];
+    Words<W> v[kSegUnits];
+#pragma unroll
+    for (int j = 0; j < kSegUnits; j++) {
+        u[j] = first_unit + j * kSegBlock + threadIdx.x;
+        if (u[j] < S.units && S.src) v[j] = __builtin_bit_cast(Words<W>, reinterpret_cast<const V*>(S.src)[u[j]]);
+    }
+#pragma unroll
+    for (int j = 0; j < kSegUnits; j++) {
+        if (u[j] >= S.units) continue;
+        if (!S.src) {
+#pragma unroll
+            for (int k = 0; k < W; k++) v[j].w[k] = S.fill[(W == 1 ? u[j] : k) & 1];
+        } else if (S.add) {
+            rebase<W>(v[j], u[j] * W, S);
+        }
+        reinterpret_cast<V*>(S.dst)[u[j]] = __builtin_bit_cast(V, v[j]);
+    }
+}
+
+// Each block takes kSegBlock * kSegUnits consecutive units of one segment.
+__global__ void __launch_bounds__(kSegBlock) copy_segs_kernel(CopyTable T) {
+    int at = 0;
+    for (int step = kSegs / 2; step; step >>= 1)
+        if (at + step < T.n && T.s[at + step].block0 <= blockIdx.x) at += step;
+    const CopySeg& S = T.s[at];
+    const int64_t first_unit = (int64_t)(blockIdx.x - S.block0) * (kSegBlock * kSegUnits);
+    if (S.shift == 4) copy_units<4>(S, first_unit);
+    else if (S.shift == 3) copy_units<2>(S, first_unit);
+    else copy_units<1>(S, first_unit);
+    if (first_unit == 0 && threadIdx.x < S.tail) {  // the words that fill no unit
+        const int64_t w = (S.units << (S.shift - 2)) + threadIdx.x;
+        Words<1> v{{S.fill[w & 1]}};
+        if (S.src) {
+            v.w[0] = reinterpret_cast<const uint32_t*>(S.src)[w];
+            if (S.add) rebase<1>(v, w, S);
+        }
+        reinterpret_cast<uint32_t*>(S.dst)[w] = v.w[0];
     }
 }
 
@@ -220,6 +308,64 @@ int oppx_offset_indices(int32_t* base, int64_t n_records, int rec_ints, int firs
     offset_indices_kernel<<<(unsigned)g, 256, 0, as_stream(stream)>>>(base, n_records, rec_ints, first, count, offset);
     OPPX_LAUNCH_CHECK("offset_indices");
     return OPPX_OK;
+}
+
+int oppx_copy_batch(int n, const oppx_copy_job* jobs, void* stream) {
+    OPPX_ARG_CHECK(n >= 0 && (n == 0 || jobs), "oppx_copy_batch: bad job list");
+    for (int j = 0; j < n; j++) {
+        const oppx_copy_job& J = jobs[j];
+        OPPX_ARG_CHECK(J.bytes >= 0 && J.rows >= 0, "oppx_copy_batch: negative size");
+        if (J.bytes == 0 || J.rows == 0) continue;
+        const uintptr_t all = (uintptr_t)J.dst | (uintptr_t)J.src | (uintptr_t)J.bytes |
+                              (J.rows > 1 ? (uintptr_t)J.dst_stride | (uintptr_t)J.src_stride : 0);
+        OPPX_ARG_CHECK(J.dst && all % 4 == 0, "oppx_copy_batch: null destination, or not whole 4-byte words");
+        OPPX_ARG_CHECK(J.rows == 1 || (J.dst_stride >= J.bytes && (!J.src || J.src_stride >= J.bytes)),
+                       "oppx_copy_batch: row stride below the row");
+        OPPX_ARG_CHECK(J.add == 0 || (J.rec_ints >= 1 && J.rec_ints <= 128 && (J.rec_ints & (J.rec_ints - 1)) == 0 &&
+                                      J.first >= 0 && J.count >= 1 && J.first + J.count <= J.rec_ints),
+                       "oppx_copy_batch: bad record layout");
+    }
+    CopyTable T;
+    T.n = 0;
+    int64_t blocks = 0;
+    const auto launch = [&]() -> int {
+        if (T.n == 0) return OPPX_OK;
+        copy_segs_kernel<<<(unsigned)blocks, kSegBlock, 0, as_stream(stream)>>>(T);
+        OPPX_LAUNCH_CHECK("copy_batch");
+        T.n = 0;
+        blocks = 0;
+        return OPPX_OK;
+    };
+    for (int j = 0; j < n; j++) {
+        const oppx_copy_job& J = jobs[j];
+        if (J.bytes == 0) continue;
+        for (int64_t r = 0; r < J.rows; r++) {
+            CopySeg S;
+            S.dst = (unsigned char*)J.dst + r * J.dst_stride;
+            S.src = J.src ? (const unsigned char*)J.src + r * J.src_stride : nullptr;
+            // the widest unit both ends are aligned to: a wave then moves 1 KiB per instruction, not 256 B
+            const uintptr_t a = (uintptr_t)S.dst | (uintptr_t)S.src;
+            S.shift = a % 16 == 0 ? 4 : (a % 8 == 0 ? 3 : 2);
+            S.units = J.bytes >> S.shift;
+            S.tail = (uint8_t)((J.bytes - (S.units << S.shift)) / 4);
+            memcpy(S.fill, &J.fill, 8);
+            S.add = J.add;
+            S.mask = (uint8_t)(J.add ? J.rec_ints - 1 : 0);
+            S.first = (uint8_t)J.first;
+            S.count = (uint8_t)J.count;
+            int64_t need = (S.units + kSegBlock * kSegUnits - 1) / (kSegBlock * kSegUnits);
+            if (need == 0) need = 1;
+            if (T.n == kSegs || blocks + need > kMaxGrid) {
+                const int rc = launch();
+                if (rc != OPPX_OK) return rc;
+            }
+            OPPX_ARG_CHECK(need <= kMaxGrid, "oppx_copy_batch: row too long");
+            S.block0 = (uint32_t)blocks;
+            T.s[T.n++] = S;
+            blocks += need;
+        }
+    }
+    return launch();
 }
 
 }  // extern "C"

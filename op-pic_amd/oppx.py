@@ -92,6 +92,11 @@ class DatDesc(Structure):
 
 
 assert ctypes.sizeof(TetAux) == 32 and ctypes.sizeof(MoveCounters) == 4 * COUNTER_WORDS
+# oppx_copy_job: one row-wise copy (src != 0) or fill of oppx_copy_batch
+COPY_JOB = np.dtype([("dst", "u8"), ("src", "u8"), ("bytes", "i8"), ("rows", "i8"), ("dst_stride", "i8"),
+                     ("src_stride", "i8"), ("fill", "u8"), ("add", "i4"), ("rec_ints", "i4"), ("first", "i4"),
+                     ("count", "i4")])
+assert COPY_JOB.itemsize == 72
 assert ctypes.sizeof(BatchInst) == 112 and ctypes.sizeof(Tuning) == 32
 
 # name -> (restype, argtypes): every symbol include/oppx.h declares
@@ -106,6 +111,7 @@ _SIGS = {
     "oppx_memset_zero": (c_int, [c_void_p, c_size_t, c_void_p]),
     "oppx_stream_sync": (c_int, [c_void_p]),
     "oppx_offset_indices": (c_int, [c_void_p, c_int64, c_int, c_int, c_int, c_int32, c_void_p]),
+    "oppx_copy_batch": (c_int, [c_int, c_void_p, c_void_p]),
     "oppx_fill_pattern": (c_int, [c_void_p, c_int64, c_int, c_int, c_void_p, c_int64, c_void_p]),
     "oppx_aos_to_soa": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_int64, c_int, c_void_p]),
     "oppx_soa_to_aos": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_int64, c_int, c_void_p]),
@@ -243,6 +249,17 @@ def check(rc: int, what: str = ""):
     if rc != OK:
         msg = lib().oppx_last_error().decode(errors="replace")
         raise OppxError(f"{what} failed (rc={rc}): {msg}")
+
+
+def copy_job(dst: int, src: int, nbytes: int, rows=1, dst_stride=0, src_stride=0, fill=0, add=0, rec=(1, 0, 1)):
+    """One COPY_JOB row: addresses and byte counts; `rec` is (rec_ints, first, count) of the words `add` rebases."""
+    return dst, src, nbytes, rows, dst_stride, src_stride, fill, add, *rec
+
+
+def copy_batch(jobs, stream):
+    """Runs copy_job rows on `stream` (one launch for every 32 rows of memory)."""
+    a = np.array(jobs, dtype=COPY_JOB)
+    check(lib().oppx_copy_batch(len(a), a.ctypes.data, stream), "copy_batch")
 
 
 def raw_stream(dev) -> int:
@@ -553,16 +570,21 @@ class FempicDevice:
         self.materialize()
         g = object.__new__(type(self))
         g.__dict__.update({k: v for k, v in self.__dict__.items() if k not in self._PER_INSTANCE})
-        g.pos, g.vel, g.lc, g.p2c = (t.clone() for t in (self.pos, self.vel, self.lc, self.p2c))
-        g.counters = self.counters.clone()
-        for name in ("hole_bits", "charge", "hops"):
-            setattr(g, name, torch.zeros_like(getattr(self, name)))
-        for name in ("work", "scratch"):  # workspaces: nothing in them has to be set
-            setattr(g, name, torch.empty_like(getattr(self, name)))
+        copied, cleared = ["pos", "vel", "lc", "p2c", "counters"], ["hole_bits", "charge", "hops"]
+        fresh = ["work", "scratch"]  # workspaces: nothing in them has to be set
         if hasattr(self, "charge_f32"):  # the FP32 deposit's node rows are shared, its outputs are not
-            g.charge_f32 = torch.zeros_like(self.charge_f32)
-            for name in ("cell_partials", "dep_scratch"):
-                setattr(g, name, torch.empty_like(getattr(self, name)))
+            cleared.append("charge_f32")
+            fresh += ["cell_partials", "dep_scratch"]
+        jobs = []
+        for name in copied + cleared + fresh:
+            src = getattr(self, name)
+            to = torch.empty_like(src, memory_format=torch.contiguous_format)
+            setattr(g, name, to)
+            if name not in fresh:
+                src = src.contiguous()
+                jobs.append(copy_job(to.data_ptr(), src.data_ptr() if name in copied else 0,
+                                     to.numel() * to.element_size()))
+        copy_batch(jobs, self.stream())
         g.pending = g.staged = False
         g._rebind()
         return g

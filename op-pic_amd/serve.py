@@ -26,7 +26,7 @@ from dataclasses import dataclass, field
 import numpy as np
 
 import oppx
-from oppx import MAX_CELL_INDEX, BatchInst, DatDesc, FempicParts, TetMesh, check, lib
+from oppx import (MAX_CELL_INDEX, BatchInst, DatDesc, FempicParts, TetMesh, check, copy_batch, copy_job, lib)
 
 
 class RangeAlloc:
@@ -209,27 +209,34 @@ class FempicArena:
         cb, nb = self.cells.alloc(nc), self.nodes.alloc(nn)
         ob = self.ovl.alloc(tpl.overlay_words) if tpl.overlay_words else -1
         slot = self.slots_free.pop()
-        cp = lambda dst, src: dst.copy_(src, non_blocking=True)
-        cp(self.det[16 * cb:16 * (cb + nc)], h["det"])
-        cp(self.aux[4 * cb:4 * (cb + nc)], h["aux"])
-        cp(self.c2n[4 * cb:4 * (cb + nc)], h["c2n"])
-        cp(self.ef[3 * cb:3 * (cb + nc)], h["ef"])
-        cp(self.node_start[nb:nb + nn], h["nstart"])
-        cp(self.node_end[nb:nb + nn], h["nend"])
-        cp(self.node_ref[4 * cb:4 * (cb + nc)], h["nref"])
-        i4 = lambda t, off: t.data_ptr() + 4 * off
-        check(L.oppx_offset_indices(i4(self.aux, 8 * cb), nc, 8, 2, 4, cb, s), "rebase c2c")  # aux: c2c at ints 2..5
-        check(L.oppx_offset_indices(i4(self.c2n, 4 * cb), 4 * nc, 1, 0, 1, nb, s), "rebase c2n")
-        check(L.oppx_offset_indices(i4(self.node_start, nb), nn, 1, 0, 1, 4 * cb, s), "rebase rows")
-        check(L.oppx_offset_indices(i4(self.node_end, nb), nn, 1, 0, 1, 4 * cb, s), "rebase rows")
-        check(L.oppx_offset_indices(i4(self.node_ref, 4 * cb), 4 * nc, 1, 0, 1, 4 * cb, s), "rebase refs")
-        pat = np.array([slot], np.int32)
-        check(L.oppx_fill_pattern(i4(self.cell_inst, cb), nc, 1, 4, pat.ctypes.data, 0, s), "cell_inst")
+        n0, jobs = self.size, []
+
+        def put(dst, at, count, src, add=0, rec=(1, 0, 1)):
+            """Job: the staged array `src` to the `count` elements from `at` on (of every row) of `dst`, its indices
+            moved by `add`. What is not resident (or has to be converted) goes through copy_ and is rebased in place."""
+            el, rows, ptr = dst.element_size(), (dst.shape[0] if dst.dim() == 2 else 1), src.data_ptr()
+            stride, row = dst.shape[-1] * el, count * el
+            src_stride, to = row, dst.data_ptr() + at * el
+            if (src.numel() != rows * count or src.dim() != dst.dim() or src.dtype != dst.dtype or
+                    src.device != dst.device or not src.is_contiguous()):
+                dst[..., at:at + count].copy_(src, non_blocking=True)
+                if not add:
+                    return
+                src_stride, ptr = stride, to
+            jobs.append(copy_job(to, ptr, row, rows, stride, src_stride, 0, add, rec))
+
+        put(self.det, 16 * cb, 16 * nc, h["det"])
+        put(self.aux, 4 * cb, 4 * nc, h["aux"], cb, (8, 2, 4))  # 32-byte records, c2c at ints 2..5
+        put(self.c2n, 4 * cb, 4 * nc, h["c2n"], nb)
+        put(self.ef, 3 * cb, 3 * nc, h["ef"])
+        put(self.node_start, nb, nn, h["nstart"], 4 * cb)
+        put(self.node_end, nb, nn, h["nend"], 4 * cb)
+        put(self.node_ref, 4 * cb, 4 * nc, h["nref"], 4 * cb)
+        jobs.append(copy_job(self.cell_inst.data_ptr() + 4 * cb, 0, 4 * nc, fill=slot * 0x100000001))
         rec = BatchInst()
         rec.cell_base, rec.n_cells, rec.node_base, rec.n_nodes = cb, nc, nb, nn
         if ob >= 0:
-            cp(self.overlay[ob:ob + tpl.overlay_words], h["overlay"])
-            check(L.oppx_offset_indices(i4(self.overlay, ob), tpl.overlay_words, 1, 0, 1, cb, s), "rebase overlay")
+            put(self.overlay, ob, tpl.overlay_words, h["overlay"], cb)
             dims = oppx.dh_dims(d["bmin"], d["bmax"], d["gs"])
             rec.dh_cell = self.overlay.data_ptr() + 4 * ob
             for a in range(3):
@@ -238,16 +245,14 @@ class FempicArena:
         rec.dt = float(d["dt"])
         rec.k = float(d["charge"]) / float(d["mass"]) * float(d["dt"])
         sz = ctypes.sizeof(BatchInst)
-        self.h_table[slot * sz:(slot + 1) * sz] = torch.frombuffer(bytearray(bytes(rec)), dtype=torch.uint8)
-        self.inst_table[slot * sz:(slot + 1) * sz].copy_(self.h_table[slot * sz:(slot + 1) * sz], non_blocking=True)
-        n0 = self.size
+        ctypes.memmove(self.h_table.data_ptr() + slot * sz, ctypes.byref(rec), sz)
+        jobs.append(copy_job(self.inst_table.data_ptr() + slot * sz, self.h_table.data_ptr() + slot * sz, sz))
         if n:
-            cp(self.pos[:, n0:n0 + n], h["pos"])
-            cp(self.vel[:, n0:n0 + n], h["vel"])
-            cp(self.p2c[n0:n0 + n], h["p2c"])
-            check(L.oppx_offset_indices(i4(self.p2c, n0), n, 1, 0, 1, cb, s), "rebase p2c")
-            zero = np.zeros(1, np.float64)
-            check(L.oppx_fill_pattern(self.lc.data_ptr() + 8 * n0, n, 4, 8, zero.ctypes.data, self.cap, s), "lc")
+            put(self.pos, n0, n, h["pos"])
+            put(self.vel, n0, n, h["vel"])
+            put(self.p2c, n0, n, h["p2c"], cb)
+            jobs.append(copy_job(self.lc.data_ptr() + 8 * n0, 0, 8 * n, 4, 8 * self.cap))
+        copy_batch(jobs, s)
         self.size = n0 + n
         self.res[slot] = (tpl, cb, nb, ob)
         return slot
@@ -318,36 +323,36 @@ class FempicArena:
         b = bounds.cpu().numpy()  # the step is complete from here on
         main = torch.cuda.current_stream(self.dev)
         self.copy_stream.wait_stream(main)
-        staged = []
-        pat = np.array([MAX_CELL_INDEX], np.int32)
+        staged, now, beside, after = [], [], [], []
         for j, slot in enumerate(slots):
             tpl, cb, nb, ob = self.res.pop(slot)
             lo, hi = int(b[2 * j]), int(b[2 * j + 1])
-            k = hi - lo
+            k, nn = hi - lo, tpl.n_nodes
             pin = lambda shape, dt: torch.empty(shape, dtype=dt, pin_memory=True)
             out = dict(pos=pin((3, k), torch.float64), vel=pin((3, k), torch.float64), lc=pin((4, k), torch.float64),
-                       p2c=pin((k,), torch.int32), charge_f32=pin((tpl.n_nodes,), torch.float32))
-            out["p2c"].copy_(self.p2c[lo:hi], non_blocking=True)
-            out["charge_f32"].copy_(self.charge_f32[nb:nb + tpl.n_nodes], non_blocking=True)
-            with torch.cuda.stream(self.copy_stream):
-                out["pos"].copy_(self.pos[:, lo:hi], non_blocking=True)
-                out["vel"].copy_(self.vel[:, lo:hi], non_blocking=True)
-                out["lc"].copy_(self.lc[:, lo:hi], non_blocking=True)
+                       p2c=pin((k,), torch.int32), charge_f32=pin((nn,), torch.float32))
+            now += [copy_job(out["p2c"].data_ptr(), self.p2c.data_ptr() + 4 * lo, 4 * k),
+                    copy_job(out["charge_f32"].data_ptr(), self.charge_f32.data_ptr() + 4 * nb, 4 * nn)]
+            beside += [copy_job(out[name].data_ptr(), t.data_ptr() + 8 * lo, 8 * k, t.shape[0], 8 * k, 8 * self.cap)
+                       for name, t in (("pos", self.pos), ("vel", self.vel), ("lc", self.lc))]
             staged.append((out, k, cb))
             self.dropping += k
-            if k:  # leaves the particle set at the next sort
-                check(L.oppx_fill_pattern(self.p2c.data_ptr() + 4 * lo, k, 1, 4, pat.ctypes.data, 0, s),
-                      "fill_pattern")
-            zero = np.zeros(1, np.int32)
-            check(L.oppx_fill_pattern(self.node_start.data_ptr() + 4 * nb, tpl.n_nodes, 1, 4, zero.ctypes.data, 0, s),
-                  "rows")  # empty node rows
-            check(L.oppx_fill_pattern(self.node_end.data_ptr() + 4 * nb, tpl.n_nodes, 1, 4, zero.ctypes.data, 0, s),
-                  "rows")
+            after += [copy_job(self.p2c.data_ptr() + 4 * lo, 0, 4 * k, fill=MAX_CELL_INDEX * 0x100000001),
+                      # leaves the particle set at the next sort; its node rows are empty
+                      copy_job(self.node_start.data_ptr() + 4 * nb, 0, 4 * nn),
+                      copy_job(self.node_end.data_ptr() + 4 * nb, 0, 4 * nn)]
             self.cells.release(cb)
             self.nodes.release(nb)
             if ob >= 0:
                 self.ovl.release(ob)
             self.slots_free.append(slot)
+        try:
+            copy_batch(now, s)
+            copy_batch(beside, self.copy_stream.cuda_stream)
+            copy_batch(after, s)
+        except BaseException:  # nothing may still write the pinned arrays once they go back to the allocator
+            torch.cuda.synchronize(self.dev)
+            raise
         done = (torch.cuda.Event(), torch.cuda.Event())
         done[0].record(main)
         done[1].record(self.copy_stream)
@@ -364,17 +369,24 @@ class FempicArena:
 
 
 class PendingResults:
-    """Results of retire_async(): counts at once, the arrays after wait()."""
+    """Results of retire_async(): counts at once, the arrays after wait(). Kernels write the pinned arrays, which the
+    host allocator cannot see: dropped without a wait(), they go back to it only once the copies have ended."""
 
     def __init__(self, staged, events):
         self.staged, self.events = staged, events
         self.counts = [k for _, k, _ in staged]
 
-    def wait(self) -> list:
+    def _finish(self):
         if self.events is not None:
             for e in self.events:
                 e.synchronize()
             self.events = None
+
+    def __del__(self):
+        self._finish()
+
+    def wait(self) -> list:
+        self._finish()
         return [dict(n=k, pos=o["pos"].numpy().T, vel=o["vel"].numpy().T, lc=o["lc"].numpy().T,
                      p2c=o["p2c"].numpy() - cb, charge_f32=o["charge_f32"].numpy()) for o, k, cb in self.staged]
 
