@@ -8,7 +8,7 @@
 //   #holes below index v        = wp[v/64] + popcount(word & low bits)      (wp = word prefix)
 //   rank of live v >= S from top = (N-1-v) - (R - #holes below v)
 // so every live tail record finds its destination hole by a binary search over wp and a
-// select inside one word. Two launches: the word prefixes inside each block of words and the block counts;
+// select inside one word. Two launches (one for a small set): the word prefixes inside each block of words and the block counts;
 // then the tail copy, whose blocks scan the block counts themselves and one of which writes the counters.
 
 #include <mutex>
@@ -27,6 +27,8 @@ constexpr int kB = 256;
 constexpr int kMaxDats = 16;
 constexpr int kMaxComps = 64;   // components one fill launch moves (more take further launches)
 constexpr int kMaxGroups = 4096;  // group prefixes a fill block holds in LDS
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallWords = 128;  // bitmap words of a set one block fills alone
 constexpr int kCopyBatch = 12;  // components loaded before any of them is stored (a FEM-PIC particle has 11)
 
 // The dats as single components: base address of each, and which of them have 8-byte elements.
@@ -80,6 +82,25 @@ __global__ void __launch_bounds__(kB) hf_count(const uint64_t* __restrict__ bits
     if (w < W) wp[w] = ex;
     if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
     if (blockIdx.x == 0 && threadIdx.x == 0) head[0] = (uint32_t)N;
+}
+
+// Record v to hole h.
+__device__ __forceinline__ void move_record(const CompTable& T, int64_t v, int64_t h) {
+            for (int c0 = 0; c0 < T.n; c0 += kCopyBatch) {
+                uint64_t x[kCopyBatch];
+    #pragma unroll
+                for (int u = 0; u < kCopyBatch; u++) {
+                    if (c0 + u >= T.n) continue;
+                    if ((T.wide >> (c0 + u)) & 1ull) x[u] = reinterpret_cast<const uint64_t*>(T.base[c0 + u])[v];
+                    else x[u] = reinterpret_cast<const uint32_t*>(T.base[c0 + u])[v];
+                }
+    #pragma unroll
+                for (int u = 0; u < kCopyBatch; u++) {
+                    if (c0 + u >= T.n) continue;
+                    if ((T.wide >> (c0 + u)) & 1ull) reinterpret_cast<uint64_t*>(T.base[c0 + u])[h] = x[u];
+                    else reinterpret_cast<uint32_t*>(T.base[c0 + u])[h] = (uint32_t)x[u];
+                }
+            }
 }
 
 // Every block scans the block counts into LDS itself (group e: blocks [e * per, (e + 1) * per)), then its
@@ -159,21 +180,65 @@ __global__ void __launch_bounds__(kB) hf_fill(const uint64_t* __restrict__ bits,
         if (hw == 0ull) continue;  // inconsistent bitmap: never write outside [0, S)
         const int64_t h = lo * 64 + (__ffsll((long long)hw) - 1);
         if (h < 0 || h >= S) continue;
-        for (int c0 = 0; c0 < T.n; c0 += kCopyBatch) {
-            uint64_t x[kCopyBatch];
+        move_record(T, v, h);
+    }
+}
+
+// The whole fill of a small set by one block: words, prefixes and searches in LDS, one launch instead of two. A set of up
+// to 8,192 particles is filled so, whatever share of it was removed: us in a graph, two launches and one, with 3, 10, 30
+// and 60% removed: 4,000 particles 7.1 / 8.1 / 16.5 / 26.7 and 5.2 / 5.6 / 10.1 / 15.7, 8,192 7.8 / 8.6 / 17.4 / 28.5
+// and 5.6 / 6.9 / 15.9 / 27.9. Beyond, one block is too few where many records move: 16,384 with 10% 9.2 and 12.6.
+__global__ void __launch_bounds__(kSmallThreads) hf_small(const uint64_t* __restrict__ bits,
+                                                          oppx_move_counters* __restrict__ ctr, CompTable T, int64_t n_max) {
+    __shared__ uint64_t s_bits[kSmallWords];
+    __shared__ uint32_t s_pre[kSmallWords], s_wave[kSmallThreads / kWave];
+    const int N = (int)live_count(ctr, n_max), W = (int)words_of(N);
+    const int w = threadIdx.x, lane = w & (kWave - 1);
+    const uint64_t mine = w < W ? bits[w] : 0ull;
+    const uint32_t c = (uint32_t)__popcll(mine);
+    uint32_t inc = c;
 #pragma unroll
-            for (int u = 0; u < kCopyBatch; u++) {
-                if (c0 + u >= T.n) continue;
-                if ((T.wide >> (c0 + u)) & 1ull) x[u] = reinterpret_cast<const uint64_t*>(T.base[c0 + u])[v];
-                else x[u] = reinterpret_cast<const uint32_t*>(T.base[c0 + u])[v];
-            }
+    for (int d = 1; d < kWave; d <<= 1) {
+        const uint32_t t = __shfl_up(inc, d);
+        if (lane >= d) inc += t;
+    }
+    if (lane == kWave - 1) s_wave[w / kWave] = inc;
+    if (w < kSmallWords) s_bits[w] = mine;
+    __syncthreads();  // also: every thread has read the live count
+    uint32_t off = 0, total = 0;
 #pragma unroll
-            for (int u = 0; u < kCopyBatch; u++) {
-                if (c0 + u >= T.n) continue;
-                if ((T.wide >> (c0 + u)) & 1ull) reinterpret_cast<uint64_t*>(T.base[c0 + u])[h] = x[u];
-                else reinterpret_cast<uint32_t*>(T.base[c0 + u])[h] = (uint32_t)x[u];
-            }
+    for (int q = 0; q < kSmallThreads / kWave; q++) {
+        off += q < w / kWave ? s_wave[q] : 0u;
+        total += s_wave[q];
+    }
+    if (w < kSmallWords) s_pre[w] = off + inc - c;
+    __syncthreads();
+    const int R = (int)total, S = N - R;
+    const bool some = R > 0 && R <= N;
+    if (threadIdx.x == 0) {
+        ctr->removed = R;
+        const uint64_t lowmask = (1ull << (S & 63)) - 1ull;
+        ctr->holes_low = some && S < N ? (int)s_pre[S >> 6] + __popcll(s_bits[S >> 6] & lowmask) : 0;
+        if (some) ctr->size = S;
+    }
+    if (!some) return;
+    for (int v = S + (int)threadIdx.x; v < N; v += kSmallThreads) {
+        const uint64_t word = s_bits[v >> 6];
+        const int j = v & 63;
+        if ((word >> j) & 1ull) continue;  // a hole itself
+        const int k = (N - 1 - v) - (R - ((int)s_pre[v >> 6] + __popcll(word & ((1ull << j) - 1ull))));
+        int lo = 0, hi = W - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if ((int)s_pre[mid] <= k) lo = mid;
+            else hi = mid - 1;
         }
+        uint64_t hw = s_bits[lo];
+        for (int r = k - (int)s_pre[lo]; r > 0 && hw; r--) hw &= hw - 1ull;
+        if (hw == 0ull) continue;  // inconsistent bitmap: never write outside [0, S)
+        const int h = lo * 64 + (__ffsll((long long)hw) - 1);
+        if (h >= S) continue;
+        move_record(T, v, h);
     }
 }
 
@@ -210,10 +275,15 @@ int holefill_impl(int64_t n_max, int64_t stride, oppx_move_counters* counters, c
         OPPX_ARG_CHECK(dats[q].base && dats[q].dim > 0, "oppx_holefill: bad dat descriptor");
         OPPX_ARG_CHECK(dats[q].elem_bytes == 4 || dats[q].elem_bytes == 8, "oppx_holefill: elem_bytes 4 or 8");
     }
+    int comps = 0;
+    for (int q = 0; q < n_dats && comps <= kMaxComps; q++) comps += dats[q].dim;
+    const bool small = n_max <= 64 * kSmallWords && comps <= kMaxComps;
     // every scratch word a pass reads was written by an earlier pass of the same call: nothing to clear
     Scratch sc = carve(work, n_max);
-    hf_count<<<(unsigned)sc.nb, kB, 0, s>>>(hole_bits, counters, sc.bsum, sc.wp, sc.head, n_max);
-    OPPX_LAUNCH_CHECK("hf_count");
+    if (!small) {
+        hf_count<<<(unsigned)sc.nb, kB, 0, s>>>(hole_bits, counters, sc.bsum, sc.wp, sc.head, n_max);
+        OPPX_LAUNCH_CHECK("hf_count");
+    }
     const int per = (int)((sc.nb + kMaxGroups - 1) / kMaxGroups);
     // one block for 8 * kB particles: with a few percent removed, a thread has at most one record to move
     int64_t g = (n_max + 8 * kB - 1) / (8 * kB);
@@ -224,7 +294,8 @@ int holefill_impl(int64_t n_max, int64_t stride, oppx_move_counters* counters, c
         T.base[T.n++] = reinterpret_cast<char*>(dats[q].base) + (size_t)d * (size_t)stride * (size_t)dats[q].elem_bytes;
         if (++d == dats[q].dim) { d = 0; q++; }
         if (T.n == kMaxComps || q == n_dats) {
-            hf_fill<<<(unsigned)g, kB, 0, s>>>(hole_bits, counters, sc.bsum, sc.wp, sc.head, T, sc.nb, per, q == n_dats);
+            if (small) hf_small<<<1, kSmallThreads, 0, s>>>(hole_bits, counters, T, n_max);
+            else hf_fill<<<(unsigned)g, kB, 0, s>>>(hole_bits, counters, sc.bsum, sc.wp, sc.head, T, sc.nb, per, q == n_dats);
             OPPX_LAUNCH_CHECK("hf_fill");
             T = CompTable{};
         }
