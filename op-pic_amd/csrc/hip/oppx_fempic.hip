@@ -128,6 +128,14 @@ __device__ __forceinline__ BlockStat block_totals(long long hsum, int hmax, int 
     return t;
 }
 
+// One thread adds a block's totals to the counters.
+__device__ __forceinline__ void add_stats(const StepArgs& P, const BlockStat& t) {
+    if (t.hops) atomicAdd((unsigned long long*)&P.ctr->total_hops, t.hops);
+    if (t.max_hops) atomicMax(&P.ctr->max_hops, t.max_hops);
+    if (t.removed) atomicAdd(&P.ctr->removed, t.removed);
+    if (t.faults) atomicAdd(&P.ctr->faults, t.faults);
+}
+
 __device__ __forceinline__ void block_stats(const StepArgs& P, long long hsum, int hmax, int nrem, int nfault) {
     const BlockStat t = block_totals(hsum, hmax, nrem, nfault);
     if (threadIdx.x == 0) {
@@ -138,10 +146,7 @@ __device__ __forceinline__ void block_stats(const StepArgs& P, long long hsum, i
             if (t.removed) atomicAdd(&sl->removed, t.removed);
             if (t.faults) atomicAdd(&sl->faults, t.faults);
         } else {
-            if (t.hops) atomicAdd((unsigned long long*)&P.ctr->total_hops, t.hops);
-            if (t.max_hops) atomicMax(&P.ctr->max_hops, t.max_hops);
-            if (t.removed) atomicAdd(&P.ctr->removed, t.removed);
-            if (t.faults) atomicAdd(&P.ctr->faults, t.faults);
+            add_stats(P, t);
         }
     }
 }
@@ -749,7 +754,8 @@ __global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(7))) fe
     BlockStat t = block_totals(done ? h : 0, done ? h : 0, (live && removed) ? 1 : 0, fault ? 1 : 0);
     if (threadIdx.x == 0) {
         t.pending = scattered ? kScattered : s_pending;
-        W.rec[blockIdx.x] = t;
+        if (W.rec) W.rec[blockIdx.x] = t;
+        else add_stats(P, t);
     }
 }
 
@@ -969,7 +975,8 @@ __global__ void __launch_bounds__(kQuadBlock) fempic_quad_kernel(StepArgs P, uin
     BlockStat t = block_totals(done ? h : 0, done ? h : 0, (live && removed && lead) ? 1 : 0, (fault && lead) ? 1 : 0);
     if (threadIdx.x == 0) {
         t.pending = s_pending;
-        W.rec[blockIdx.x] = t;
+        if (W.rec) W.rec[blockIdx.x] = t;
+        else add_stats(P, t);
     }
 }
 
@@ -1503,6 +1510,8 @@ void fold_slots(const StepArgs& P, hipStream_t s) {
     if (P.slots) slots_reduce_kernel<<<1, kSlots, 0, s>>>(P.slots, P.ctr);
 }
 
+constexpr int kFewBlocks = 256;  // first-pass blocks up to which there is no walk pass
+
 // Two-pass move (first-hop pass + worklist walk) when the work buffer is large enough and the
 // tuning asks for it; returns false when the caller should use the cooperative tile walk instead.
 template <bool PUSH, bool DH, bool DEPOSIT, bool BATCH, bool GATHER = false>
@@ -1515,24 +1524,33 @@ bool launch_two_pass(const StepArgs& P, int64_t n_max, void* work, size_t work_b
     // the second read of lc and p2c. A copy fits a CU's LDS beside the rest up to 16,384 nodes.
     const bool dense = DEPOSIT && g_tuning.lanes == 1 && g_tuning.first_block == kBlock && P.n_nodes > 0 &&
                        P.n_nodes <= kDenseNodes && n_max >= 32 * P.n_nodes && n_max >= (1 << 18);
+    // A few blocks walk everything themselves and add their totals to the counters, one after the other in some 10 ns
+    // each: no walk pass, whose launch the smallest sets wait for. A fused step, us, with it and without: 1,000 particles
+    // 21.4 and 18.4, 4,000 22.8 and 19.3, 16,000 28.9 and 25.6, 32,000 35.3 and 31.8, 65,000 36.4 and 34.4, 130,000 (508
+    // blocks) 41 and 41. Not where the pass also clears the counters: its blocks' adds would race that.
+    const int per_block = g_tuning.lanes == 4 ? kQuadParts : (g_tuning.first_block == kMaxBlock ? kMaxBlock : kBlock);
+    const bool alone = !P.reset && !dense && g_tuning.inline_hops >= 16 && n_max <= (int64_t)kFewBlocks * per_block;
+    const int inline_hops = alone ? OPPX_MAX_HOPS : g_tuning.inline_hops;
+    if (alone) W.rec = nullptr;
     unsigned g;
     if (g_tuning.lanes == 4) {
         W.parts = kQuadParts;
         g = grid_for(n_max, kQuadParts);
-        fempic_quad_kernel<PUSH, DH, DEPOSIT, BATCH, GATHER><<<g, kQuadBlock, 0, s>>>(P, g, g_tuning.inline_hops, W);
+        fempic_quad_kernel<PUSH, DH, DEPOSIT, BATCH, GATHER><<<g, kQuadBlock, 0, s>>>(P, g, inline_hops, W);
     } else if (g_tuning.first_block == kMaxBlock) {
         W.parts = kMaxBlock;
         g = grid_for(n_max, kMaxBlock);
         fempic_first_kernel<kMaxBlock, PUSH, DH, DEPOSIT, BATCH, GATHER, false>
-            <<<g, kMaxBlock, 0, s>>>(P, g, g_tuning.inline_hops, W);
+            <<<g, kMaxBlock, 0, s>>>(P, g, inline_hops, W);
     } else {
         g = grid_for(n_max, kBlock);
         auto first = fempic_first_kernel<kBlock, PUSH, DH, DEPOSIT, BATCH, GATHER, false>;
         if constexpr (DEPOSIT) {
             if (dense) first = fempic_first_kernel<kBlock, PUSH, DH, true, BATCH, GATHER, true>;
         }
-        first<<<g, kBlock, 0, s>>>(P, g, g_tuning.inline_hops, W);
+        first<<<g, kBlock, 0, s>>>(P, g, inline_hops, W);
     }
+    if (alone) return true;
     // A first pass that walks 16 evaluations itself hands over next to nothing: 256 records a walk block, at most
     // 64 blocks (each adds to the one counters record; 94,000 records: 9.0 us, with 256 blocks 13.4). Below that the walk spreads over the resident grid. With dense
     // deposits 8 records, 2048 particles, a block, one block a CU.
