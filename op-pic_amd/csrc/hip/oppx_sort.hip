@@ -65,6 +65,16 @@ __device__ __forceinline__ void finish_sort(const Finish& F) {
     if (F.drop) F.ctr->size = F.state[0] - F.state[1];
 }
 
+constexpr uint32_t kFewBatch = 32;  // tile counts of a digit in flight
+
+// A sort of few tiles: its scatters sum the tiles' counts themselves (hist is tile-major, no row scan runs), and the
+// first one also leaves the live and removed counts in `state`.
+struct Few {
+    const uint32_t* rem_block;
+    unsigned rem_blocks;
+    int32_t* state;
+};
+
 // lanes of the wave (among `active`) holding the same 8-bit digit as this lane
 __device__ __forceinline__ unsigned long long digit_peers(uint32_t d, unsigned long long active) {
     unsigned long long peers = active;
@@ -86,7 +96,7 @@ __device__ __forceinline__ uint32_t cell_key(int32_t c, uint32_t n_cells) {
 // Per-block digit counts of one pass. All of a thread's keys are loaded before any is counted
 // (independent loads in flight). Counting needs no ranks: a wave whose live lanes share one digit adds
 // once (nearly sorted keys), any other wave adds per lane.
-template <int ITEMS, bool FIRST>
+template <int ITEMS, bool FIRST, bool FEW>
 __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(8))) sort_hist(const uint32_t* __restrict__ keys, const int32_t* __restrict__ p2c,
                                                 uint32_t n_cells, const int32_t* __restrict__ live, int64_t n_max,
                                                 int shift, uint32_t* __restrict__ hist,
@@ -126,7 +136,8 @@ __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(8))) so
             }
         }
         __syncthreads();
-        hist[(int64_t)threadIdx.x * tiles + t] = s_h[threadIdx.x];  // digit-major rows of the live tiles
+        // digit-major rows of the live tiles; tile-major where the scatter sums the tiles itself
+        hist[FEW ? t * kBins + threadIdx.x : (int64_t)threadIdx.x * tiles + t] = s_h[threadIdx.x];
     }
     // the block's removed particles: a word of its own, which nothing has to clear beforehand
     if (FIRST) {
@@ -274,18 +285,26 @@ __device__ __forceinline__ uint32_t block_scan_excl(uint32_t v, uint32_t* total)
 // costs it one read of 1 KB; before, scanning digits and tiles as one array took three launches a pass.
 // Four waves per SIMD: the occupancy the 16-key tile's LDS allows (four 39 KB blocks per CU), reached
 // without spilling.
-template <int ITEMS, bool LAST, bool FIRST>
+template <int ITEMS, bool LAST, bool FIRST, bool FEW>
 __global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(4)))
 sort_scatter(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin, const int32_t* __restrict__ p2c,
              uint32_t n_cells, const int32_t* __restrict__ live, int64_t n_max, int shift,
              const uint32_t* __restrict__ offs, const uint32_t* __restrict__ row_total, uint32_t* __restrict__ kout,
-             uint32_t* __restrict__ vout, int32_t* __restrict__ p2c_out, Finish F) {
+             uint32_t* __restrict__ vout, int32_t* __restrict__ p2c_out, Finish F, Few W) {
     __shared__ TileLds<ITEMS> L;
     const int64_t n = live_n(live, n_max);
-    {
+    if constexpr (!FEW) {
         uint32_t all;
         const uint32_t b = block_scan_excl(row_total[threadIdx.x], &all);
         L.base[threadIdx.x] = b;
+    } else if (FIRST && blockIdx.x == 0 && threadIdx.x < kWave) {  // what the row scan's last block does otherwise
+        uint32_t r = 0;
+        for (unsigned q = threadIdx.x; q < W.rem_blocks; q += kWave) r += W.rem_block[q];
+        r = (uint32_t)wave_sum_i32((int)r);
+        if (threadIdx.x == 0) {
+            W.state[0] = (int32_t)n;
+            W.state[1] = (int32_t)r;
+        }
     }
     finish_sort(F);
     // the grid (at most the blocks that fit the chip at once) strides over the tiles that hold live
@@ -301,7 +320,25 @@ sort_scatter(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
         int tid = (int)threadIdx.x;
         asm volatile("" : "+v"(tid));
         for (int q = 0; q < kB / kWave; q++) L.wave[q][tid] = 0;
-        L.dst[tid] = L.base[tid] + offs[(uint32_t)tid * (uint32_t)tiles + (uint32_t)t];  // < 2^31 counts (n below 2^32)
+        if constexpr (FEW) {
+            uint32_t before = 0, all = 0, total;  // of digit tid, in the tiles before and in all
+            for (uint32_t q0 = 0; q0 < (uint32_t)tiles; q0 += kFewBatch) {
+                uint32_t c[kFewBatch];  // loaded together: the reads' latency is what this costs
+#pragma unroll
+                for (uint32_t k = 0; k < kFewBatch; k++) {
+                    const uint32_t q = q0 + k;
+                    c[k] = q < (uint32_t)tiles ? offs[q * kBins + (uint32_t)tid] : 0u;
+                }
+#pragma unroll
+                for (uint32_t k = 0; k < kFewBatch; k++) {
+                    before += q0 + k < (uint32_t)t ? c[k] : 0u;
+                    all += c[k];
+                }
+            }
+            L.dst[tid] = block_scan_excl(all, &total) + before;
+        } else {
+            L.dst[tid] = L.base[tid] + offs[(uint32_t)tid * (uint32_t)tiles + (uint32_t)t];  // < 2^31 counts (n below 2^32)
+        }
         uint32_t key[ITEMS], val[ITEMS], rank[ITEMS];
         tile_load<ITEMS, FIRST>(kin, vin, p2c, n_cells, base, m, tid, key, val);
         __syncthreads();
@@ -473,6 +510,11 @@ __global__ void sort_empty(oppx_move_counters* ctr, int drop) {
     if (drop) ctr->size = 0;
 }
 
+// Tiles up to which a sort runs without its row scans, one launch less a pass: every scatter block then reads all the
+// tiles' counts, 1 KB each. us, two digit passes of a lazy sort in a graph, with the scans and without: 1,000 particles
+// 21.7 and 16.4, 10,000 23.5 and 18.6, 30,000 24.3 and 19.3, 60,000 (59 tiles) 25.3 and 22.8, 120,000 25.0 and 28.5 (with 16
+// counts in flight 15.5 / 17.8 / 20.3 / 24.9, with 64 18.0 / 20.1 / 20.6 / 21.8 at the first four). Not where one launch does it all: it would set the live count while its other blocks read it.
+constexpr int64_t kFewTiles = 64;
 struct SortScratch {
     uint32_t *ka, *va, *kb, *vb, *hist, *row_total, *rem_block;
     int32_t* state;
@@ -574,6 +616,7 @@ int oppx_sort_by_cell(int64_t n_max, int64_t stride, oppx_move_counters* counter
         // no dat left to gather: the last digit pass writes the permutation straight into perm_out
         const bool direct = T.n == 0 && perm_out != nullptr;
         const bool gather = !direct && (T.n > 0 || perm_out);
+        const bool few = items == 4 && sc.nblocks <= kFewTiles && (passes > 1 || gather);
         const Finish no_finish{nullptr, nullptr, 0}, finish{counters, sc.state, drop_removed};
         for (int pass = 0; pass < passes; pass++) {
             const int shift = 8 * pass;
@@ -584,38 +627,43 @@ int oppx_sort_by_cell(int64_t n_max, int64_t stride, oppx_move_counters* counter
                 // the first pass's histogram and row scan read the counters, the later launches the scratch copy
                 const int32_t* live = first ? &counters->size : sc.state;
                 unsigned hist_grid = 1;
-#define OPPX_HIST(I, F)                                                                                              \
+#define OPPX_HIST_W(I, F, W)                                                                                         \
     do {                                                                                                             \
-        hist_grid = stride_grid(reinterpret_cast<const void*>(sort_hist<I, F>), kB, sc.nblocks, kGridMult);          \
+        auto kern = sort_hist<I, F, W>;                                                                              \
+        hist_grid = stride_grid(reinterpret_cast<const void*>(kern), kB, sc.nblocks, kGridMult);                     \
         hist_grid = xcd_grid(hist_grid < kMaxHistGrid ? hist_grid : kMaxHistGrid);                                   \
-        sort_hist<I, F><<<hist_grid, kB, 0, s>>>(kin, p2c, kc, live, n_max, shift, sc.hist, sc.rem_block);           \
+        kern<<<hist_grid, kB, 0, s>>>(kin, p2c, kc, live, n_max, shift, sc.hist, sc.rem_block);                      \
     } while (0)
-                if (items == 4) { if (first) OPPX_HIST(4, true); else OPPX_HIST(4, false); }
+#define OPPX_HIST(I, F) OPPX_HIST_W(I, F, false)
+                if (few) { if (first) OPPX_HIST_W(4, true, true); else OPPX_HIST_W(4, false, true); }
+                else if (items == 4) { if (first) OPPX_HIST(4, true); else OPPX_HIST(4, false); }
                 else if (items == 8) { if (first) OPPX_HIST(8, true); else OPPX_HIST(8, false); }
                 else if (items == 16) { if (first) OPPX_HIST(16, true); else OPPX_HIST(16, false); }
                 else { if (first) OPPX_HIST(32, true); else OPPX_HIST(32, false); }
 #undef OPPX_HIST
+#undef OPPX_HIST_W
                 OPPX_LAUNCH_CHECK("sort_hist");
-                sort_rows<<<kBins + (first ? 1 : 0), kB, 0, s>>>(sc.hist, live, n_max, (int64_t)kB * items, sc.row_total,
+                if (!few) sort_rows<<<kBins + (first ? 1 : 0), kB, 0, s>>>(sc.hist, live, n_max, (int64_t)kB * items, sc.row_total,
                                                                  sc.rem_block, hist_grid, sc.state);
                 OPPX_LAUNCH_CHECK("sort_rows");
-#define OPPX_SCATTER(I, LST, F)                                                                      \
+#define OPPX_SCATTER(I, LST, F, FW)                                                                 \
     do {                                                                                              \
-        auto kern = sort_scatter<I, LST, F>;                                                          \
+        auto kern = sort_scatter<I, LST, F, FW>;                                                     \
         const unsigned res = resident_blocks(reinterpret_cast<const void*>(kern), kB);               \
         const unsigned g = xcd_grid((int64_t)res < sc.nblocks ? res : (unsigned)sc.nblocks);           \
-        kern<<<g, kB, 0, s>>>(kin, vin, p2c, kc, sc.state, n_max, shift, sc.hist, sc.row_total, kout, vdst, \
-                              p2c_out, last && !gather ? finish : no_finish);                        \
+        kern<<<g, kB, 0, s>>>(kin, vin, p2c, kc, FW ? live : sc.state, n_max, shift, sc.hist, sc.row_total, kout, vdst, \
+                              p2c_out, last && !gather ? finish : no_finish, Few{sc.rem_block, hist_grid, sc.state}); \
     } while (0)
-#define OPPX_SCATTER_LF(I)                                                     \
+#define OPPX_SCATTER_LF(I, FW)                                                 \
     do {                                                                       \
-        if (last) { if (first) OPPX_SCATTER(I, true, true); else OPPX_SCATTER(I, true, false); } \
-        else { if (first) OPPX_SCATTER(I, false, true); else OPPX_SCATTER(I, false, false); }   \
+        if (last) { if (first) OPPX_SCATTER(I, true, true, FW); else OPPX_SCATTER(I, true, false, FW); } \
+        else { if (first) OPPX_SCATTER(I, false, true, FW); else OPPX_SCATTER(I, false, false, FW); }   \
     } while (0)
-                if (items == 4) OPPX_SCATTER_LF(4);
-                else if (items == 8) OPPX_SCATTER_LF(8);
-                else if (items == 16) OPPX_SCATTER_LF(16);
-                else OPPX_SCATTER_LF(32);
+                if (few) OPPX_SCATTER_LF(4, true);
+                else if (items == 4) OPPX_SCATTER_LF(4, false);
+                else if (items == 8) OPPX_SCATTER_LF(8, false);
+                else if (items == 16) OPPX_SCATTER_LF(16, false);
+                else OPPX_SCATTER_LF(32, false);
 #undef OPPX_SCATTER_LF
 #undef OPPX_SCATTER
                 OPPX_LAUNCH_CHECK("sort_scatter");
