@@ -180,42 +180,6 @@ __global__ void slots_reduce_kernel(const StatSlot* slots, oppx_move_counters* c
     }
 }
 
-enum WalkEnd { kWalkDone = 0, kWalkRemoved = 1, kWalkFault = 2 };
-
-// Multi-hop walk from `cell` (apps/app_fempic/kernels.h:106-161 per hop, do/while of
-// apps_codegen/app_fempic_cg/hip/move_kernel_loop.hpp:162-183). lc = c2*fnma(d3,z,fma(d2,y,fnma(d1,x,d0))).
-__device__ __forceinline__ int walk(const StepArgs& P, double x, double y, double z, int& cell, double& l0,
-                                    double& l1, double& l2, double& l3, int& h) {
-    for (;;) {
-        const double2* __restrict__ d = reinterpret_cast<const double2*>(P.det + 16 * (int64_t)cell);
-        const double2 a0 = d[0], a1 = d[1], a2 = d[2], a3 = d[3], a4 = d[4], a5 = d[5], a6 = d[6], a7 = d[7];
-        const double4 au = *reinterpret_cast<const double4*>(P.aux + cell);  // {c2, c2c[0..1], c2c[2..3], pad}
-        const double c2 = au.x;
-        l0 = c2 * fma(-a1.y, z, fma(a1.x, y, fma(-a0.y, x, a0.x)));
-        l1 = c2 * fma(-a3.y, z, fma(a3.x, y, fma(-a2.y, x, a2.x)));
-        l2 = c2 * fma(-a5.y, z, fma(a5.x, y, fma(-a4.y, x, a4.x)));
-        l3 = c2 * fma(-a7.y, z, fma(a7.x, y, fma(-a6.y, x, a6.x)));
-        h++;
-        if ((l0 > -1e-10) && ((l0 - 1.0) < 1e-10) && (l1 > -1e-10) && ((l1 - 1.0) < 1e-10) && (l2 > -1e-10) &&
-            ((l2 - 1.0) < 1e-10) && (l3 > -1e-10) && ((l3 - 1.0) < 1e-10))
-            return kWalkDone;
-        // most negative weight, first index wins ties (strict <); neighbour picked without
-        // a dynamically indexed array so nothing spills to scratch or LDS
-        const int2 n01 = __builtin_bit_cast(int2, au.y), n23 = __builtin_bit_cast(int2, au.z);
-        int nb = n01.x;
-        double ml = l0;
-        if (l1 < ml) { ml = l1; nb = n01.y; }
-        if (l2 < ml) { ml = l2; nb = n23.x; }
-        if (l3 < ml) { ml = l3; nb = n23.y; }
-        if (nb < 0) {
-            cell = kMaxCell;
-            return kWalkRemoved;
-        }
-        if (nb >= P.n_cells || h >= OPPX_MAX_HOPS) return kWalkFault;
-        cell = nb;
-    }
-}
-
 // Workgroup-level deposit aggregation: (node, value) pairs go into an LDS open-addressing table
 // (ds_add_f64), then one device-scope atomic per distinct node leaves the workgroup. Cell-ordered
 // particles share most of their nodes, so this removes most of the global atomics. A pair that
@@ -229,32 +193,32 @@ __device__ __forceinline__ int walk(const StepArgs& P, double x, double y, doubl
 // unsorted steps) 612 / 887 / 1,298 -> 322 / 291 / 390 us; 1.5 M in x-fastest order 40 / 55 / 72 -> 26 / 26 / 32 us;
 // 1 M in no order 229 -> 195 us. Groups of 8 and 4 slots, one group of 1024 (low bits only), and probes to the next
 // slot measured between the two.
-constexpr int kTable = 1024;
 constexpr int kLine = 16;  // nodes of a 128-byte line
 constexpr int kProbe = 16;
 constexpr int kProbeStep = 11 * kLine;
-static_assert(kTable == 64 * kLine, "6 bits of hash choose the group");
 
-struct DepositTable {
-    int key[kTable];
-    double val[kTable];
+template <int GROUP_BITS>
+struct DepositTableOf {
+    static constexpr int kSlots = (1 << GROUP_BITS) * kLine;
+    static constexpr int kGroupBits = GROUP_BITS;
+    int key[kSlots];
+    double val[kSlots];
 };
+using DepositTable = DepositTableOf<6>;
 
-__device__ __forceinline__ void table_clear(DepositTable& T) {
-    for (int q = threadIdx.x; q < kTable; q += blockDim.x) {
+template <typename Table>
+__device__ __forceinline__ void table_clear(Table& T) {
+    for (int q = threadIdx.x; q < Table::kSlots; q += blockDim.x) {
         T.key[q] = -1;
         T.val[q] = 0.0;
     }
 }
 
-__device__ __forceinline__ uint32_t table_slot(int node) {
-    return ((((uint32_t)node / kLine) * 2654435761u) >> 26) * kLine + (uint32_t)node % kLine;
-}
-
 enum TableAdd { kOldEntry = 0, kNewEntry = 1, kNoEntry = 2 };  // kNoEntry: the value went to global memory
 
-__device__ __forceinline__ int table_add(DepositTable& T, double* __restrict__ charge, int node, double v) {
-    uint32_t h = table_slot(node);
+template <typename Table>
+__device__ __forceinline__ int table_add(Table& T, double* __restrict__ charge, int node, double v) {
+    uint32_t h = ((((uint32_t)node / kLine) * 2654435761u) >> (32 - Table::kGroupBits)) * kLine + (uint32_t)node % kLine;
     for (int p = 0; p < kProbe; p++) {
         const int k = T.key[h];
         if (k == node) {
@@ -268,102 +232,105 @@ __device__ __forceinline__ int table_add(DepositTable& T, double* __restrict__ c
                 return prev == -1 ? kNewEntry : kOldEntry;
             }
         }
-        h = (h + kProbeStep) & (kTable - 1);
+        h = (h + kProbeStep) & (Table::kSlots - 1);
     }
     atomicAdd(charge + node, v);
     return kNoEntry;
 }
 
-__device__ __forceinline__ void table_flush(DepositTable& T, double* __restrict__ charge) {
-    for (int q = threadIdx.x; q < kTable; q += blockDim.x) {
+template <typename Table>
+__device__ __forceinline__ void table_flush(Table& T, double* __restrict__ charge) {
+    for (int q = threadIdx.x; q < Table::kSlots; q += blockDim.x) {
         const int k = T.key[q];
         if (k >= 0) atomicAdd(charge + k, T.val[q]);
     }
 }
 
-template <bool PUSH, bool MOVE, bool DH, bool DEPOSIT, bool STATS>
-__global__ void __launch_bounds__(kBlock) fempic_pass_kernel(StepArgs P, uint32_t nblocks) {
+// The deposit by itself: PARTS particles a lane, their cells, weights and nodes loaded before the first add. It is bound
+// by the table's flush, one global add per distinct node of a block, and 512 particles have far fewer than twice the
+// nodes of 256 where a cell holds a few; their table has 2048 slots. A deposit after 1, 2, 3 unsorted steps, us, one
+// particle a lane and 1024 slots against two and 2048: 24 M particles in 3 M cells 324 / 293 / 382 and 255 / 215 / 237,
+// 1.5 M in 197,000 27 / 26 / 32 and 26 / 23 / 28, 1 M in no order in 48,000 190 and 171; but 200,000 in 663,000 10 and
+// 13: the clear and the sweep of the larger table.
+template <int PARTS, int GROUP_BITS>
+__global__ void __launch_bounds__(kBlock) fempic_deposit_kernel(StepArgs P, uint32_t nblocks) {
+    int64_t n = P.ctr->size;
+    n = n < 0 ? 0 : (n > P.n_max ? P.n_max : n);
+    const uint32_t nlive = live_blocks(n, kBlock * PARTS, nblocks);
+    if (blockIdx.x >= nlive) return;
+    const uint32_t b = xcd_block(blockIdx.x, nlive);
+    const int64_t S = P.stride, i0 = (int64_t)b * kBlock * PARTS + threadIdx.x;
+    __shared__ DepositTableOf<GROUP_BITS> T;
+    int cell[PARTS];
+    double l[PARTS][4];
+#pragma unroll
+    for (int u = 0; u < PARTS; u++) {
+        const int64_t i = i0 + u * kBlock;
+        cell[u] = i < n ? ld_stream(P.p2c + i) : kMaxCell;
+#pragma unroll
+        for (int d = 0; d < 4; d++) l[u][d] = i < n ? ld_stream(P.lc + d * S + i) : 0.0;
+    }
+    table_clear(T);
+    int4 m[PARTS];
+    int nfault = 0;
+#pragma unroll
+    for (int u = 0; u < PARTS; u++) {  // particles already removed hold MAX_CELL_INDEX and are skipped
+        const bool ok = (unsigned)cell[u] < (unsigned)P.n_cells;
+        if (!ok && cell[u] != kMaxCell) nfault++;
+        if (!ok) cell[u] = kMaxCell;
+        else m[u] = *reinterpret_cast<const int4*>(P.c2n + 4 * (int64_t)cell[u]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < PARTS; u++) {
+        if (cell[u] == kMaxCell) continue;
+        table_add(T, P.charge, m[u].x, l[u][0]);
+        table_add(T, P.charge, m[u].y, l[u][1]);
+        table_add(T, P.charge, m[u].z, l[u][2]);
+        table_add(T, P.charge, m[u].w, l[u][3]);
+    }
+    __syncthreads();
+    table_flush(T, P.charge);
+    nfault = wave_sum_i32(nfault);
+    if ((threadIdx.x & (kWave - 1)) == 0 && nfault) atomicAdd(&P.ctr->faults, nfault);
+}
+
+// The push, and with DH the relocation through the overlay (the walk runs in a second pass).
+template <bool DH>
+__global__ void __launch_bounds__(kBlock) fempic_push_kernel(StepArgs P, uint32_t nblocks) {
     int64_t n = P.ctr->size;
     n = n < 0 ? 0 : (n > P.n_max ? P.n_max : n);  // never beyond the host's bound
     const uint32_t nlive = live_blocks(n, kBlock, nblocks);
     if (blockIdx.x >= nlive) return;  // no block of live particles left for this workgroup
     const uint32_t b = xcd_block(blockIdx.x, nlive);
     const int64_t i = (int64_t)b * kBlock + threadIdx.x;
-    const bool live = i < n;
     const int64_t S = P.stride;
 
-    int cell = live ? P.p2c[i] : kMaxCell;
+    const int cell = i < n ? P.p2c[i] : kMaxCell;
     // a particle already holding MAX_CELL_INDEX is skipped, as the reference loops do
     // (apps_codegen/app_fempic_cg/seq/move_kernel_loop.hpp:92-94)
-    const bool skip = live && cell == kMaxCell;
-    bool fault = live && !skip && !((unsigned)cell < (unsigned)P.n_cells);
-    bool removed = false;
-    int h = 0;
-    double l0 = 0.0, l1 = 0.0, l2 = 0.0, l3 = 0.0;
-    __shared__ DepositTable s_table;
-    if (DEPOSIT) table_clear(s_table);
-
-    if (live && !skip && !fault && (PUSH || MOVE)) {
+    bool fault = cell != kMaxCell && !((unsigned)cell < (unsigned)P.n_cells);
+    if (cell != kMaxCell && !fault) {
+        // calculate_new_pos_vel_kernel: v = fma(k, E, v); x = fma(v, dt, x)
         double x = P.pos[i], y = P.pos[S + i], z = P.pos[2 * S + i];
-        if (PUSH) {
-            // calculate_new_pos_vel_kernel: v = fma(k, E, v); x = fma(v, dt, x)
-            const double* e = P.ef + 3 * (int64_t)cell;
-            const double ex = e[0], ey = e[1], ez = e[2];
-            double vx = P.vel[i], vy = P.vel[S + i], vz = P.vel[2 * S + i];
-            vx = fma(P.k, ex, vx);
-            x = fma(vx, P.dt, x);
-            vy = fma(P.k, ey, vy);
-            y = fma(vy, P.dt, y);
-            vz = fma(P.k, ez, vz);
-            z = fma(vz, P.dt, z);
-            P.vel[i] = vx; P.vel[S + i] = vy; P.vel[2 * S + i] = vz;
-            P.pos[i] = x; P.pos[S + i] = y; P.pos[2 * S + i] = z;
-        }
-        if (!MOVE && DH) {  // relocation only: the walk runs in a second pass
+        const double* e = P.ef + 3 * (int64_t)cell;
+        const double ex = e[0], ey = e[1], ez = e[2];
+        double vx = P.vel[i], vy = P.vel[S + i], vz = P.vel[2 * S + i];
+        vx = fma(P.k, ex, vx);
+        x = fma(vx, P.dt, x);
+        vy = fma(P.k, ey, vy);
+        y = fma(vy, P.dt, y);
+        vz = fma(P.k, ez, vz);
+        z = fma(vz, P.dt, z);
+        P.vel[i] = vx; P.vel[S + i] = vy; P.vel[2 * S + i] = vz;
+        P.pos[i] = x; P.pos[S + i] = y; P.pos[2 * S + i] = z;
+        if (DH) {
             const int c = dh_lookup(P.dh, x, y, z);
             P.p2c[i] = c;
-            removed = (c == kMaxCell);
-            if (!removed && !((unsigned)c < (unsigned)P.n_cells)) fault = true;
-        }
-        if (MOVE) {
-            if (DH) {
-                cell = dh_lookup(P.dh, x, y, z);
-                if (cell == kMaxCell) removed = true;
-                else if (!((unsigned)cell < (unsigned)P.n_cells)) fault = true;
-            }
-            if (!removed && !fault) {
-                const int r = walk(P, x, y, z, cell, l0, l1, l2, l3, h);
-                removed = (r == kWalkRemoved);
-                fault = (r == kWalkFault);
-                P.lc[i] = l0; P.lc[S + i] = l1; P.lc[2 * S + i] = l2; P.lc[3 * S + i] = l3;
-            }
-            if (!fault) P.p2c[i] = removed ? kMaxCell : cell;
-            if (P.hops) P.hops[i] = h;
+            if (c != kMaxCell && !((unsigned)c < (unsigned)P.n_cells)) fault = true;
         }
     }
-    if (DEPOSIT) {
-        __syncthreads();  // table cleared
-        if (live && !skip && !removed && !fault) {
-            if (!MOVE) {
-                l0 = P.lc[i]; l1 = P.lc[S + i]; l2 = P.lc[2 * S + i]; l3 = P.lc[3 * S + i];
-            }
-            const int4 m = *reinterpret_cast<const int4*>(P.c2n + 4 * (int64_t)cell);
-            table_add(s_table, P.charge, m.x, l0);
-            table_add(s_table, P.charge, m.y, l1);
-            table_add(s_table, P.charge, m.z, l2);
-            table_add(s_table, P.charge, m.w, l3);
-        }
-        __syncthreads();
-        table_flush(s_table, P.charge);
-    }
-
-    const int lane = threadIdx.x & (kWave - 1);
-    if (MOVE) {
-        // removal bitmap: one 64-bit word per wave, written for every word of [0, n_max)
-        const unsigned long long rmask = __ballot(live && removed);
-        if (lane == 0) P.hole_bits[i >> 6] = rmask;
-    }
-    block_stats(P, STATS ? h : 0, STATS ? h : 0, (MOVE && live && removed) ? 1 : 0, fault ? 1 : 0);
+    block_stats(P, 0, 0, 0, fault ? 1 : 0);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1164,7 +1131,7 @@ constexpr int kMaxTile = 512;
 constexpr int kMaxTileWords = kMaxTile / kWave;
 constexpr int kWavesPerBlock = kBlock / kWave;
 
-template <bool PUSH, bool DH, bool DEPOSIT, bool STATS, bool PRE, bool BATCH>
+template <bool PUSH, bool DH, bool DEPOSIT, bool PRE, bool BATCH>
 __global__ void __launch_bounds__(kBlock) fempic_tile_kernel(StepArgs P, uint32_t nblocks) {
     const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
     int64_t n = P.ctr->size;
@@ -1338,10 +1305,8 @@ __global__ void __launch_bounds__(kBlock) fempic_tile_kernel(StepArgs P, uint32_
                     nfault++;
                 }
                 if (P.hops) P.hops[p] = h;
-                if (STATS) {
-                    hsum += h;
-                    hmax = hmax > h ? hmax : h;
-                }
+                hsum += h;
+                hmax = hmax > h ? hmax : h;
                 have = false;
             }
             const unsigned long long free_mask = __ballot(!have);
@@ -1473,11 +1438,11 @@ unsigned tile_grid(const void* kernel, unsigned block_tiles, bool persistent) {
     return g < (unsigned)kXcds ? (unsigned)kXcds : g;
 }
 
-template <bool PUSH, bool DH, bool DEPOSIT, bool STATS, bool PRE, bool BATCH>
+template <bool PUSH, bool DH, bool DEPOSIT, bool PRE, bool BATCH>
 void launch_tile(const StepArgs& P, int64_t n_max, hipStream_t s) {
     const int64_t per_block = (int64_t)P.tile * kWavesPerBlock;
     const unsigned nbt = (unsigned)((n_max + per_block - 1) / per_block);
-    auto kern = fempic_tile_kernel<PUSH, DH, DEPOSIT, STATS, PRE, BATCH>;
+    auto kern = fempic_tile_kernel<PUSH, DH, DEPOSIT, PRE, BATCH>;
     const unsigned g = tile_grid(reinterpret_cast<const void*>(kern), nbt, P.persistent != 0);
     if (P.persistent) reset_queue_kernel<<<1, kWave, 0, s>>>(P.ctr);
     kern<<<g, kBlock, 0, s>>>(P, nbt);
@@ -1574,26 +1539,11 @@ bool launch_two_pass(const StepArgs& P, int64_t n_max, void* work, size_t work_b
     return true;
 }
 
-template <bool PUSH, bool MOVE, bool DEPOSIT>
-void launch_pass(const StepArgs& P, bool dh, bool stats, int64_t n_max, hipStream_t s) {
-    if constexpr (MOVE) {
-        if (dh) {
-            if (stats) launch_tile<PUSH, true, DEPOSIT, true, false, false>(P, n_max, s);
-            else launch_tile<PUSH, true, DEPOSIT, false, false, false>(P, n_max, s);
-        } else {
-            if (stats) launch_tile<PUSH, false, DEPOSIT, true, false, false>(P, n_max, s);
-            else launch_tile<PUSH, false, DEPOSIT, false, false, false>(P, n_max, s);
-        }
-    } else {
-        const unsigned g = grid_for(n_max, kBlock);
-#define OPPX_PASS(DHV, STV) fempic_pass_kernel<PUSH, MOVE, DHV, DEPOSIT, STV><<<g, kBlock, 0, s>>>(P, g)
-        if (dh) {
-            if (stats) OPPX_PASS(true, true); else OPPX_PASS(true, false);
-        } else {
-            if (stats) OPPX_PASS(false, true); else OPPX_PASS(false, false);
-        }
-#undef OPPX_PASS
-    }
+// The cooperative tile walk, with or without the overlay lookup.
+template <bool PUSH, bool DEPOSIT>
+void launch_walk(const StepArgs& P, bool dh, int64_t n_max, hipStream_t s) {
+    if (dh) launch_tile<PUSH, true, DEPOSIT, false, false>(P, n_max, s);
+    else launch_tile<PUSH, false, DEPOSIT, false, false>(P, n_max, s);
 }
 
 template <bool DH, bool BATCH, bool GATHER>
@@ -1672,7 +1622,8 @@ int oppx_fempic_push(int64_t n_max, const oppx_fempic_parts* parts, const oppx_t
     P.n_max = n_max;
     P.k = k;
     P.dt = dt;
-    launch_pass<true, false, false>(P, false, false, n_max, as_stream(stream));
+    const unsigned g = grid_for(n_max, kBlock);
+    fempic_push_kernel<false><<<g, kBlock, 0, as_stream(stream)>>>(P, g);
     OPPX_LAUNCH_CHECK("fempic_push");
     return OPPX_OK;
 }
@@ -1701,7 +1652,7 @@ int oppx_fempic_move(int64_t n_max, const oppx_fempic_parts* parts, const oppx_t
         reset_counters_kernel<<<1, 1, 0, s>>>(counters);
         OPPX_LAUNCH_CHECK("reset_counters");
         attach_slots(P, work, work_bytes, s);
-        launch_pass<false, true, false>(P, dh != nullptr, true, n_max, s);
+        launch_walk<false, false>(P, dh != nullptr, n_max, s);
         fold_slots(P, s);
     }
     OPPX_LAUNCH_CHECK("fempic_move");
@@ -1718,7 +1669,15 @@ int oppx_fempic_deposit_atomic(int64_t n_max, const oppx_fempic_parts* parts, co
     if (n_max == 0) return OPPX_OK;
     P.n_max = n_max;
     P.charge = node_charge;
-    launch_pass<false, false, true>(P, false, false, n_max, as_stream(stream));
+    hipStream_t s = as_stream(stream);
+    // two particles a lane where their block's nodes are mostly shared, and where half the blocks still fill the chip
+    if (n_max >= 2 * P.n_cells && n_max >= (1 << 18)) {
+        const unsigned g = grid_for(n_max, 2 * kBlock);
+        fempic_deposit_kernel<2, 7><<<g, kBlock, 0, s>>>(P, g);
+    } else {
+        const unsigned g = grid_for(n_max, kBlock);
+        fempic_deposit_kernel<1, 6><<<g, kBlock, 0, s>>>(P, g);
+    }
     OPPX_LAUNCH_CHECK("fempic_deposit");
     return OPPX_OK;
 }
@@ -1749,15 +1708,15 @@ int oppx_fempic_step_fused(int64_t n_max, const oppx_fempic_parts* parts, const 
     if (two) {
     } else if (g_tuning.split == 1 && dh != nullptr) {
         // two passes: coalesced push + overlay relocation, then the cooperative walk (+ deposit)
-        fempic_pass_kernel<true, false, true, false, false><<<grid_for(n_max, kBlock), kBlock, 0, s>>>(
+        fempic_push_kernel<true><<<grid_for(n_max, kBlock), kBlock, 0, s>>>(
             P, grid_for(n_max, kBlock));
         OPPX_LAUNCH_CHECK("fempic_push_relocate");
-        if (node_charge) launch_tile<false, false, true, true, true, false>(P, n_max, s);
-        else launch_tile<false, false, false, true, true, false>(P, n_max, s);
+        if (node_charge) launch_tile<false, false, true, true, false>(P, n_max, s);
+        else launch_tile<false, false, false, true, false>(P, n_max, s);
     } else if (node_charge) {
-        launch_pass<true, true, true>(P, dh != nullptr, true, n_max, s);
+        launch_walk<true, true>(P, dh != nullptr, n_max, s);
     } else {
-        launch_pass<true, true, false>(P, dh != nullptr, true, n_max, s);
+        launch_walk<true, false>(P, dh != nullptr, n_max, s);
     }
     fold_slots(P, s);
     OPPX_LAUNCH_CHECK("fempic_step_fused");
@@ -1870,8 +1829,8 @@ int oppx_fempic_batch_step_fused(int64_t n_max, const oppx_fempic_parts* parts, 
                                  : launch_two_pass<true, true, false, true>(P, n_max, work, work_bytes, s);
     if (!two) {
         attach_slots(P, work, work_bytes, s);
-        if (node_charge) launch_tile<true, true, true, true, false, true>(P, n_max, s);
-        else launch_tile<true, true, false, true, false, true>(P, n_max, s);
+        if (node_charge) launch_tile<true, true, true, false, true>(P, n_max, s);
+        else launch_tile<true, true, false, false, true>(P, n_max, s);
         fold_slots(P, s);
     }
     OPPX_LAUNCH_CHECK("fempic_batch_step_fused");
