@@ -184,6 +184,7 @@ class FempicArena:
         # results of retired requests go to the host on their own stream, beside the next step
         self.copy_stream = torch.cuda.Stream(device=self.dev)
         self.cap, self.size = P, 0
+        self.published = 0  # the live count in the device counters
 
     def stream(self):
         return oppx.raw_stream(self.dev)
@@ -262,6 +263,7 @@ class FempicArena:
         the pinned value is rewritten only after the step's closing synchronisation)."""
         self.h_size[0] = self.size
         self.counters[0:1].copy_(self.h_size, non_blocking=True)
+        self.published = self.size
 
     def step(self):
         """One batched step of every resident request: push/move, Sort_All finalize, FP32 deposit."""
@@ -272,7 +274,8 @@ class FempicArena:
         parts = FempicParts(self.cap, self.pos.data_ptr(), self.vel.data_ptr(), self.lc.data_ptr(),
                             self.p2c.data_ptr())
         n_insts = max(self.res) + 1 if self.res else 1
-        self.publish_size()
+        if self.size != self.published:  # admissions since the last step, which left its live count there itself
+            self.publish_size()
         check(L.oppx_fempic_step_begin(self.counters.data_ptr(), None, 0, s), "step_begin")
         if self.size:
             check(L.oppx_fempic_batch_step_fused(self.size, ctypes.byref(parts), ctypes.byref(mesh),
@@ -294,7 +297,7 @@ class FempicArena:
                                                self.cell_partials.data_ptr(), None, self.charge_f32.data_ptr(),
                                                self.dep_scratch.data_ptr(), self.dep_bytes, s),
               "deposit_f32")
-        self.size = int(self.counters[0].item())  # the live count after the finalize (host sync)
+        self.size = self.published = int(self.counters[0].item())  # the live count after the finalize (host sync)
         self.dropping = 0  # the finalize dropped the retired particles
 
     def retire(self, slots) -> list:
