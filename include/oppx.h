@@ -181,9 +181,11 @@ typedef struct oppx_copy_job {
 } oppx_copy_job;
 
 /* Runs n jobs in one launch for every 32 rows (a kernel, so it can be graph-captured). Pointers are device memory or
- * pinned host memory, and with sizes and strides multiples of 4. Jobs may run in any order: none may write what
+ * pinned host memory, and with sizes and strides multiples of 4. At most max_blocks workgroups of 256 run (0: as many
+ * as there is work): copies to host memory beside other kernels need few, and more would only wait for the link in
+ * the others' place. Jobs may run in any order: none may write what
  * another one touches; src == dst (rebasing in place) is allowed. No reference counterpart. */
-int oppx_copy_batch(int n, const oppx_copy_job* jobs, void* stream);
+int oppx_copy_batch(int n, const oppx_copy_job* jobs, int max_blocks, void* stream);
 
 /* AoS (host layout, doc/api.rst:115-118) <-> SoA (device layout) transposes on the device,
  * replacing the host transposes of opp_lib/src/hip/opp_hip_utils.cpp:35-153. */

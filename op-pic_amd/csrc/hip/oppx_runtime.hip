@@ -96,7 +96,7 @@ __global__ void offset_indices_kernel(int32_t* __restrict__ base, int64_t n, int
 // ---- many copies and fills in one launch ----
 // Small copies are bound by their launches (2 us each on the device, 8 to 10 us apart from a Python caller), large ones
 // by HBM. Admitting a request took 21 copies, fills and rebasing passes, handing it back 11, a clone 9; each is one
-// launch now: five requests admitted 560 -> 200 us and handed back 900 -> 620 us (of which 20 MB over the host link at
+// launch now: five requests admitted 560 -> 200 us and handed back 900 -> 660 us (of which 20 MB over the host link at
 // 54 GB/s take 350), a clone of 3,000 particles 89 -> 39 us, one of 24 M 807 -> 746. 1.92 GB in 10 rows: 671 us with
 // 2 units in flight a thread, 697 with 4, 722 with 8 (the runtime's own copy 775).
 constexpr int kSegs = 32;      // row segments a launch takes (their table is a kernel argument)
@@ -110,7 +110,7 @@ struct CopySeg {
     const unsigned char* src;  // nullptr: the two words of `fill` over and over
     int64_t units;
     uint32_t fill[2];
-    uint32_t block0;           // its first block
+    uint32_t chunk0;           // its first chunk
     int32_t add;
     uint8_t shift, tail, mask, first, count;
 };
@@ -159,24 +159,26 @@ __device__ __forceinline__ void copy_units(const CopySeg& S, int64_t first_unit)
     }
 }
 
-// Each block takes kSegBlock * kSegUnits consecutive units of one segment.
-__global__ void __launch_bounds__(kSegBlock) copy_segs_kernel(CopyTable T) {
-    int at = 0;
-    for (int step = kSegs / 2; step; step >>= 1)
-        if (at + step < T.n && T.s[at + step].block0 <= blockIdx.x) at += step;
-    const CopySeg& S = T.s[at];
-    const int64_t first_unit = (int64_t)(blockIdx.x - S.block0) * (kSegBlock * kSegUnits);
-    if (S.shift == 4) copy_units<4>(S, first_unit);
-    else if (S.shift == 3) copy_units<2>(S, first_unit);
-    else copy_units<1>(S, first_unit);
-    if (first_unit == 0 && threadIdx.x < S.tail) {  // the words that fill no unit
-        const int64_t w = (S.units << (S.shift - 2)) + threadIdx.x;
-        Words<1> v{{S.fill[w & 1]}};
-        if (S.src) {
-            v.w[0] = reinterpret_cast<const uint32_t*>(S.src)[w];
-            if (S.add) rebase<1>(v, w, S);
+// Each block takes kSegBlock * kSegUnits consecutive units of one segment at a time.
+__global__ void __launch_bounds__(kSegBlock) copy_segs_kernel(CopyTable T, uint32_t chunks) {
+    for (uint32_t b = blockIdx.x; b < chunks; b += gridDim.x) {
+        int at = 0;
+        for (int step = kSegs / 2; step; step >>= 1)
+            if (at + step < T.n && T.s[at + step].chunk0 <= b) at += step;
+        const CopySeg& S = T.s[at];
+        const int64_t first_unit = (int64_t)(b - S.chunk0) * (kSegBlock * kSegUnits);
+        if (S.shift == 4) copy_units<4>(S, first_unit);
+        else if (S.shift == 3) copy_units<2>(S, first_unit);
+        else copy_units<1>(S, first_unit);
+        if (first_unit == 0 && threadIdx.x < S.tail) {  // the words that fill no unit
+            const int64_t w = (S.units << (S.shift - 2)) + threadIdx.x;
+            Words<1> v{{S.fill[w & 1]}};
+            if (S.src) {
+                v.w[0] = reinterpret_cast<const uint32_t*>(S.src)[w];
+                if (S.add) rebase<1>(v, w, S);
+            }
+            reinterpret_cast<uint32_t*>(S.dst)[w] = v.w[0];
         }
-        reinterpret_cast<uint32_t*>(S.dst)[w] = v.w[0];
     }
 }
 
@@ -310,8 +312,8 @@ int oppx_offset_indices(int32_t* base, int64_t n_records, int rec_ints, int firs
     return OPPX_OK;
 }
 
-int oppx_copy_batch(int n, const oppx_copy_job* jobs, void* stream) {
-    OPPX_ARG_CHECK(n >= 0 && (n == 0 || jobs), "oppx_copy_batch: bad job list");
+int oppx_copy_batch(int n, const oppx_copy_job* jobs, int max_blocks, void* stream) {
+    OPPX_ARG_CHECK(n >= 0 && max_blocks >= 0 && (n == 0 || jobs), "oppx_copy_batch: bad job list");
     for (int j = 0; j < n; j++) {
         const oppx_copy_job& J = jobs[j];
         OPPX_ARG_CHECK(J.bytes >= 0 && J.rows >= 0, "oppx_copy_batch: negative size");
@@ -327,13 +329,14 @@ int oppx_copy_batch(int n, const oppx_copy_job* jobs, void* stream) {
     }
     CopyTable T;
     T.n = 0;
-    int64_t blocks = 0;
+    int64_t chunks = 0;
     const auto launch = [&]() -> int {
         if (T.n == 0) return OPPX_OK;
-        copy_segs_kernel<<<(unsigned)blocks, kSegBlock, 0, as_stream(stream)>>>(T);
+        const int64_t g = max_blocks && max_blocks < chunks ? max_blocks : chunks;
+        copy_segs_kernel<<<(unsigned)g, kSegBlock, 0, as_stream(stream)>>>(T, (uint32_t)chunks);
         OPPX_LAUNCH_CHECK("copy_batch");
         T.n = 0;
-        blocks = 0;
+        chunks = 0;
         return OPPX_OK;
     };
     for (int j = 0; j < n; j++) {
@@ -355,14 +358,14 @@ int oppx_copy_batch(int n, const oppx_copy_job* jobs, void* stream) {
             S.count = (uint8_t)J.count;
             int64_t need = (S.units + kSegBlock * kSegUnits - 1) / (kSegBlock * kSegUnits);
             if (need == 0) need = 1;
-            if (T.n == kSegs || blocks + need > kMaxGrid) {
+            if (T.n == kSegs || chunks + need > kMaxGrid) {
                 const int rc = launch();
                 if (rc != OPPX_OK) return rc;
             }
             OPPX_ARG_CHECK(need <= kMaxGrid, "oppx_copy_batch: row too long");
-            S.block0 = (uint32_t)blocks;
+            S.chunk0 = (uint32_t)chunks;
             T.s[T.n++] = S;
-            blocks += need;
+            chunks += need;
         }
     }
     return launch();

@@ -111,7 +111,7 @@ _SIGS = {
     "oppx_memset_zero": (c_int, [c_void_p, c_size_t, c_void_p]),
     "oppx_stream_sync": (c_int, [c_void_p]),
     "oppx_offset_indices": (c_int, [c_void_p, c_int64, c_int, c_int, c_int, c_int32, c_void_p]),
-    "oppx_copy_batch": (c_int, [c_int, c_void_p, c_void_p]),
+    "oppx_copy_batch": (c_int, [c_int, c_void_p, c_int, c_void_p]),
     "oppx_fill_pattern": (c_int, [c_void_p, c_int64, c_int, c_int, c_void_p, c_int64, c_void_p]),
     "oppx_aos_to_soa": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_int64, c_int, c_void_p]),
     "oppx_soa_to_aos": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_int64, c_int, c_void_p]),
@@ -256,10 +256,10 @@ def copy_job(dst: int, src: int, nbytes: int, rows=1, dst_stride=0, src_stride=0
     return dst, src, nbytes, rows, dst_stride, src_stride, fill, add, *rec
 
 
-def copy_batch(jobs, stream):
-    """Runs copy_job rows on `stream` (one launch for every 32 rows of memory)."""
+def copy_batch(jobs, stream, max_blocks=0):
+    """Runs copy_job rows on `stream` (one launch for every 32 rows of memory, of at most max_blocks workgroups)."""
     a = np.array(jobs, dtype=COPY_JOB)
-    check(lib().oppx_copy_batch(len(a), a.ctypes.data, stream), "copy_batch")
+    check(lib().oppx_copy_batch(len(a), a.ctypes.data, max_blocks, stream), "copy_batch")
 
 
 def raw_stream(dev) -> int:

@@ -11,22 +11,22 @@ pytestmark = pytest.mark.gpu
 MAX = oppx.MAX_CELL_INDEX
 
 
-def run(jobs):
-    oppx.copy_batch(jobs, torch.cuda.current_stream().cuda_stream)
+def run(jobs, max_blocks=0):
+    oppx.copy_batch(jobs, torch.cuda.current_stream().cuda_stream, max_blocks)
     torch.cuda.synchronize()
 
 
 @pytest.mark.parametrize("words", [1, 2, 3, 4, 5, 7, 2047, 2048, 2049, 4096, 70_001])
 @pytest.mark.parametrize("to,frm", [(0, 0), (2, 2), (4, 2), (1, 1), (3, 0), (0, 1)])
-@pytest.mark.parametrize("rows", [1, 3, 40])
-def test_gpu_copy_batch_rows(words, to, frm, rows):
+@pytest.mark.parametrize("rows,blocks", [(1, 0), (3, 5), (40, 0), (40, 1)])
+def test_gpu_copy_batch_rows(words, to, frm, rows, blocks):
     if rows * words > 300_000:
         rows = 4
     rng = np.random.default_rng(words + 7 * to + frm)
     ds, ss = words + to + 5, words + frm + 2
     src = rng.integers(-2**31, 2**31, rows * ss + 8, dtype=np.int64).astype(np.int32)
     a, b = torch.from_numpy(src).cuda(), torch.full((rows * ds + 8,), 77, dtype=torch.int32, device="cuda")
-    run([oppx.copy_job(b.data_ptr() + 4 * to, a.data_ptr() + 4 * frm, 4 * words, rows, 4 * ds, 4 * ss)])
+    run([oppx.copy_job(b.data_ptr() + 4 * to, a.data_ptr() + 4 * frm, 4 * words, rows, 4 * ds, 4 * ss)], blocks)
     want = np.full(rows * ds + 8, 77, np.int32)
     for r in range(rows):
         want[to + r * ds:to + r * ds + words] = src[frm + r * ss:frm + r * ss + words]
