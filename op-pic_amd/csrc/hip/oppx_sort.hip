@@ -426,8 +426,18 @@ __global__ void __launch_bounds__(kB) sort_rows(uint32_t* __restrict__ hist, con
 
 constexpr int kGatherRows = 4;   // particles a thread moves of its column
 constexpr int kGatherCols = 64;  // most columns side by side in the grid
+constexpr int64_t kCacheBytes = 256ll << 20;
+constexpr uint32_t kGatherTiles = 512;        // tiles of a chunk
+constexpr uint32_t kGatherBlocks = 1u << 18;  // workgroups of a launch
 
-template <typename T>
+// An XCD's share of the tiles goes column by column in chunks of this many tiles: all of them where the results fit the
+// cache (and then at most 2^16 workgroups move them, a 4-byte word or more a lane).
+template <bool STREAM>
+__host__ __device__ inline uint32_t gather_chunk(uint32_t share) {
+    return share < 1 ? 1 : (!STREAM || share < kGatherTiles ? share : kGatherTiles);
+}
+
+template <typename T, bool STREAM>
 __device__ __forceinline__ void gather_column(const void* in, void* out, int64_t first, const uint32_t (&from)[kGatherRows],
                                               const bool (&ok)[kGatherRows], int64_t j) {
     const T* s = reinterpret_cast<const T*>(in) + first;
@@ -438,54 +448,80 @@ __device__ __forceinline__ void gather_column(const void* in, void* out, int64_t
         if (ok[r]) v[r] = s[from[r]];
 #pragma unroll
     for (int r = 0; r < kGatherRows; r++)
-        if (ok[r]) d[j + r * kB] = v[r];
+        if (ok[r]) {
+            if (STREAM) __builtin_nontemporal_store(v[r], d + j + r * kB);
+            else d[j + r * kB] = v[r];
+        }
 }
 
 // Bound by the lines it reads: cells of neighbouring planes take particles out of the same lines, and moving whole
 // particles an XCD's L2 lost a line before its last reader came (3 M particles on 40^3 cubes: 75,000 particles between
-// two planes, 6.3 MB of their dats against 4 MB of L2). So the grid runs through one column (a component of a dat)
-// after the other, where the same window is 0.6 MB; the permutation is read once per column instead of once. The
-// gather of pos, vel, lc and p2c, us: 3 M particles two steps from cell order 235 -> 183 (two columns at a time 195, three
-// 203; 2 or 8 particles a thread 193, 190), 24 M on a Morton mesh 1700 -> 1420, 1 M 55 -> 44. Streaming stores: 1390
-// at 24 M but 191 at 3 M, where the deposit that follows finds its input in the caches.
+// two planes, 6.3 MB of their dats against 4 MB of L2). So an XCD runs through its tiles one column (a component of a
+// dat) after the other, where the same window is 0.6 MB, in chunks of 512 tiles, half a million particles, whose part
+// of the permutation is still in L2 for the next column. Whole particles before / one column of the whole set after the
+// other / chunks, pos, vel, lc and p2c, us: displaced by up to 100,000 places 1 M 118 / 64 / 64, 3 M 363 / 244 / 244,
+// 24 M 2,912 / 2,102 / 2,010, 80 M 9,746 / 6,966 / 7,320; in random order 3 M 639 / 540 / 541, 24 M 6,355 / 5,090 /
+// 5,090, 80 M 22,960 / 17,490 / 22,870; nearly in place already, where every line is read once anyway, 3 M 94 / 98 / 98,
+// 24 M 710 / 865 / 731, 80 M 2,324 / 2,856 / 2,463. Chunks of 16 to 128 tiles lose the window (24 M within 3 M places
+// 4,180 at 512, 6,300 at 32). At most 2^18 workgroups: with 16 of 100 M particles live the rest are launched for nothing (763 us with all, 512 so), while
+// with 2^16 the blocks of a full set drift apart (24 M 2,247).
+template <bool STREAM>
 __global__ void __launch_bounds__(kB) sort_gather(const uint32_t* __restrict__ perm, const int32_t* __restrict__ live,
-                                                  int64_t n_max, GatherTable T, int cols, int32_t* __restrict__ perm_out,
+                                                  int64_t n_max, GatherTable T, int cols, int side, int32_t* __restrict__ perm_out,
                                                   Finish F) {
     const int64_t n = live_n(live, n_max);
-    if (blockIdx.y == 0) finish_sort(F);
-    // each XCD takes one contiguous eighth of every column: a permuted line is then read into one L2 instead of eight
-    const uint32_t nlive = live_blocks(n, kB * kGatherRows, gridDim.x);
-    if (blockIdx.x >= nlive) return;
-    const int64_t j = (int64_t)xcd_block(blockIdx.x, nlive) * (kB * kGatherRows) + threadIdx.x;
-    uint32_t from[kGatherRows];
-    bool ok[kGatherRows];
+    finish_sort(F);
+    // each XCD takes one contiguous eighth of the tiles, a chunk of them at a time, column by column
+    const uint32_t tiles = (uint32_t)((n + kB * kGatherRows - 1) / (kB * kGatherRows));
+    const uint32_t share = (tiles + kXcds - 1) / kXcds;
+    const uint32_t ch = gather_chunk<STREAM>(share), per = ch * (uint32_t)side, steps = (share + ch - 1) / ch * per;
+    for (uint32_t k = blockIdx.x / kXcds; k < steps; k += STREAM ? gridDim.x / kXcds : steps) {
+        const uint32_t before = STREAM ? k / per : 0u, in = k - before * per, col = in / ch;
+        const uint32_t tile = before * ch + in - col * ch;
+        if (STREAM && tile >= share) continue;
+        const int64_t j = (int64_t)((blockIdx.x % kXcds) * share + tile) * (kB * kGatherRows) + threadIdx.x;
+        uint32_t from[kGatherRows];
+        bool ok[kGatherRows];
 #pragma unroll
-    for (int r = 0; r < kGatherRows; r++) {
-        const int64_t i = j + r * kB;
-        ok[r] = i < n;
-        from[r] = ok[r] ? perm[i] : 0u;
-        ok[r] = ok[r] && from[r] < T.stride;  // never read outside the dats
-    }
-    for (int c = blockIdx.y; c < cols; c += gridDim.y) {
-        int q = 0, d = c;
-        while (d >= T.dim[q]) d -= T.dim[q++];
-        if (T.eb[q] == 8) gather_column<double>(T.in[q], T.out[q], d * T.stride, from, ok, j);
-        else gather_column<int32_t>(T.in[q], T.out[q], d * T.stride, from, ok, j);
-    }
-    if (perm_out && blockIdx.y == 0) {
+        for (int r = 0; r < kGatherRows; r++) {
+            const int64_t i = j + r * kB;
+            ok[r] = i < n;
+            from[r] = ok[r] ? perm[i] : 0u;
+            ok[r] = ok[r] && from[r] < T.stride;  // never read outside the dats
+        }
+        for (int c = (int)col; c < cols; c += side) {
+            int q = 0, d = c;
+            while (d >= T.dim[q]) d -= T.dim[q++];
+            if (T.eb[q] == 8) gather_column<double, STREAM>(T.in[q], T.out[q], d * T.stride, from, ok, j);
+            else gather_column<int32_t, STREAM>(T.in[q], T.out[q], d * T.stride, from, ok, j);
+        }
+        if (perm_out && col == 0) {
 #pragma unroll
-        for (int r = 0; r < kGatherRows; r++)
-            if (ok[r]) perm_out[j + r * kB] = (int32_t)from[r];
+            for (int r = 0; r < kGatherRows; r++)
+                if (ok[r]) perm_out[j + r * kB] = (int32_t)from[r];
+        }
     }
 }
 
 void launch_gather(const uint32_t* perm, const int32_t* live, int64_t n_max, const GatherTable& T, int32_t* perm_out,
                    const Finish& finish, hipStream_t s) {
     int cols = 0;
-    for (int q = 0; q < T.n; q++) cols += T.dim[q];
-    const unsigned y = cols < 1 ? 1 : (cols < kGatherCols ? cols : kGatherCols);
-    sort_gather<<<dim3(xcd_grid(grid_for(n_max, kB * kGatherRows)), y), kB, 0, s>>>(perm, live, n_max, T, cols, perm_out,
-                                                                                    finish);
+    int64_t record = 0;
+    for (int q = 0; q < T.n; q++) {
+        cols += T.dim[q];
+        record += (int64_t)T.dim[q] * T.eb[q];
+    }
+    const int side = cols < 1 ? 1 : (cols < kGatherCols ? cols : kGatherCols);
+    const uint32_t share = (grid_for(n_max, kB * kGatherRows) + kXcds - 1) / kXcds;
+    const bool stream = n_max * record > kCacheBytes;
+    const uint32_t ch = stream ? gather_chunk<true>(share) : gather_chunk<false>(share);
+    uint32_t g = (share + ch - 1) / ch * ch * (uint32_t)side * kXcds;
+    if (stream && g > kGatherBlocks) g = kGatherBlocks;
+    // Results past the 256 MB cache are stored streaming, which keeps the L2 for the lines being gathered (24 M a lazily
+    // sorted step later 2,010 -> 1,940 us); in smaller ones the kernels that follow find their input there (serving
+    // steps of 500,000 particles 150 us, 163 with streaming stores).
+    if (stream) sort_gather<true><<<g, kB, 0, s>>>(perm, live, n_max, T, cols, side, perm_out, finish);
+    else sort_gather<false><<<g, kB, 0, s>>>(perm, live, n_max, T, cols, side, perm_out, finish);
 }
 
 __global__ void lower_bound_kernel(const int32_t* __restrict__ p2c, const oppx_move_counters* ctr, int64_t n_max,
