@@ -111,10 +111,10 @@ __device__ __forceinline__ double row_add(double x) {
 }
 
 // Adds the twelve values of the lanes in `mask` (wave-uniform, not empty), whose particles all deposit into `cell`
-// (wave-uniform), to the cell's entry. Called by whole waves. Each exchange halves the values a lane carries: twelve to six across the wave's
-// halves, six to three across the rows of 16, then three sums inside the rows -- 63 vector instructions where summing
-// every value over the whole wave by shuffles took 144 LDS-crossbar moves. Row r then holds values 3 r .. 3 r + 2,
-// and twelve lanes add one each.
+// (wave-uniform), to the cell's entry. Called by whole waves. Each exchange halves the values a lane carries: twelve
+// to six across the wave's halves, six to three across the rows of 16, then three sums inside the rows -- 63 vector
+// instructions where summing every value over the whole wave by shuffles took 144 LDS-crossbar moves. Row r then
+// holds values 3 r .. 3 r + 2, and twelve lanes add one each.
 __device__ __forceinline__ void cab_wave_add(CabTable& T, double* __restrict__ acc, int cell, unsigned long long mask, int lane,
                                              const double* v) {
     const bool in = (mask >> lane) & 1ull;

@@ -491,7 +491,8 @@ struct WorkList {
 };
 
 template <int BS, bool PUSH, bool DH, bool DEPOSIT, bool BATCH, bool GATHER, bool DENSE>
-__global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(7))) fempic_first_kernel(StepArgs P, uint32_t nblocks, int inline_hops, WorkList W) {
+__global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(7)))
+fempic_first_kernel(StepArgs P, uint32_t nblocks, int inline_hops, WorkList W) {
     int64_t n = P.ctr->size;
     n = n < 0 ? 0 : (n > P.n_max ? P.n_max : n);
     // workgroups past the blocks of live particles (the grid is sized by the host's bound) leave at
@@ -1525,8 +1526,8 @@ bool launch_two_pass(const StepArgs& P, int64_t n_max, void* work, size_t work_b
     }
     if (alone) return true;
     // A first pass that walks 16 evaluations itself hands over next to nothing: 256 records a walk block, at most
-    // 64 blocks (each adds to the one counters record; 94,000 records: 9.0 us, with 256 blocks 13.4). Below that the walk spreads over the resident grid. With dense
-    // deposits 8 records, 2048 particles, a block, one block a CU.
+    // 64 blocks (each adds to the one counters record; 94,000 records: 9.0 us, with 256 blocks 13.4). Below that the walk
+    // spreads over the resident grid. With dense deposits 8 records, 2048 particles, a block, one block a CU.
     const bool rare = g_tuning.inline_hops >= 16;
     const int per = rare && !dense ? kBlock : 8;
     const void* plain = reinterpret_cast<const void*>(fempic_walk_kernel<DEPOSIT, false>);

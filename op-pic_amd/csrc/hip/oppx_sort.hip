@@ -97,10 +97,10 @@ __device__ __forceinline__ uint32_t cell_key(int32_t c, uint32_t n_cells) {
 // (independent loads in flight). Counting needs no ranks: a wave whose live lanes share one digit adds
 // once (nearly sorted keys), any other wave adds per lane.
 template <int ITEMS, bool FIRST, bool FEW>
-__global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(8))) sort_hist(const uint32_t* __restrict__ keys, const int32_t* __restrict__ p2c,
-                                                uint32_t n_cells, const int32_t* __restrict__ live, int64_t n_max,
-                                                int shift, uint32_t* __restrict__ hist,
-                                                uint32_t* __restrict__ rem_block) {
+__global__ void __launch_bounds__(kB) __attribute__((amdgpu_waves_per_eu(8)))
+sort_hist(const uint32_t* __restrict__ keys, const int32_t* __restrict__ p2c, uint32_t n_cells,
+          const int32_t* __restrict__ live, int64_t n_max, int shift, uint32_t* __restrict__ hist,
+          uint32_t* __restrict__ rem_block) {
     __shared__ uint32_t s_h[kBins];
     const int64_t n = live_n(live, n_max);
     const int lane = threadIdx.x & (kWave - 1);
@@ -455,20 +455,21 @@ __device__ __forceinline__ void gather_column(const void* in, void* out, int64_t
 }
 
 // Bound by the lines it reads: cells of neighbouring planes take particles out of the same lines, and moving whole
-// particles an XCD's L2 lost a line before its last reader came (3 M particles on 40^3 cubes: 75,000 particles between
-// two planes, 6.3 MB of their dats against 4 MB of L2). So an XCD runs through its tiles one column (a component of a
-// dat) after the other, where the same window is 0.6 MB, in chunks of 512 tiles, half a million particles, whose part
-// of the permutation is still in L2 for the next column. Whole particles before / one column of the whole set after the
-// other / chunks, pos, vel, lc and p2c, us: displaced by up to 100,000 places 1 M 118 / 64 / 64, 3 M 363 / 244 / 244,
-// 24 M 2,912 / 2,102 / 2,010, 80 M 9,746 / 6,966 / 7,320; in random order 3 M 639 / 540 / 541, 24 M 6,355 / 5,090 /
-// 5,090, 80 M 22,960 / 17,490 / 22,870; nearly in place already, where every line is read once anyway, 3 M 94 / 98 / 98,
-// 24 M 710 / 865 / 731, 80 M 2,324 / 2,856 / 2,463. Chunks of 16 to 128 tiles lose the window (24 M within 3 M places
-// 4,180 at 512, 6,300 at 32). At most 2^18 workgroups: with 16 of 100 M particles live the rest are launched for nothing (763 us with all, 512 so), while
-// with 2^16 the blocks of a full set drift apart (24 M 2,247).
+// particles an XCD's L2 lost a line before its last reader came (3 M particles on 40^3 cubes: 75,000 particles
+// between two planes, 6.3 MB of their dats against 4 MB of L2). So an XCD runs through its tiles one column (a
+// component of a dat) after the other, where the same window is 0.6 MB, in chunks of 512 tiles, half a million
+// particles, whose part of the permutation is still in L2 for the next column. Whole particles before / one column of
+// the whole set after the other / chunks, pos, vel, lc and p2c, us: displaced by up to 100,000 places 1 M 118 / 64 /
+// 64, 3 M 363 / 244 / 244, 24 M 2,912 / 2,102 / 2,010, 80 M 9,746 / 6,966 / 7,320; in random order 3 M 639 / 540 /
+// 541, 24 M 6,355 / 5,090 / 5,090, 80 M 22,960 / 17,490 / 22,870; nearly in place already, where every line is read
+// once anyway, 3 M 94 / 98 / 98, 24 M 710 / 865 / 731, 80 M 2,324 / 2,856 / 2,463. Chunks of 16 to 128 tiles lose the
+// window (24 M within 3 M places 4,180 at 512, 6,300 at 32). At most 2^18 workgroups: with 16 of 100 M particles live
+// the rest are launched for nothing (763 us with all, 512 so), while with 2^16 the blocks of a full set drift apart
+// (24 M 2,247).
 template <bool STREAM>
 __global__ void __launch_bounds__(kB) sort_gather(const uint32_t* __restrict__ perm, const int32_t* __restrict__ live,
-                                                  int64_t n_max, GatherTable T, int cols, int side, int32_t* __restrict__ perm_out,
-                                                  Finish F) {
+                                                  int64_t n_max, GatherTable T, int cols, int side,
+                                                  int32_t* __restrict__ perm_out, Finish F) {
     const int64_t n = live_n(live, n_max);
     finish_sort(F);
     // each XCD takes one contiguous eighth of the tiles, a chunk of them at a time, column by column
@@ -547,9 +548,10 @@ __global__ void sort_empty(oppx_move_counters* ctr, int drop) {
 }
 
 // Tiles up to which a sort runs without its row scans, one launch less a pass: every scatter block then reads all the
-// tiles' counts, 1 KB each. us, two digit passes of a lazy sort in a graph, with the scans and without: 1,000 particles
-// 21.7 and 16.4, 10,000 23.5 and 18.6, 30,000 24.3 and 19.3, 60,000 (59 tiles) 25.3 and 22.8, 120,000 25.0 and 28.5 (with 16
-// counts in flight 15.5 / 17.8 / 20.3 / 24.9, with 64 18.0 / 20.1 / 20.6 / 21.8 at the first four). Not where one launch does it all: it would set the live count while its other blocks read it.
+// tiles' counts, 1 KB each. us, two digit passes of a lazy sort in a graph, with the scans and without: 1,000
+// particles 21.7 and 16.4, 10,000 23.5 and 18.6, 30,000 24.3 and 19.3, 60,000 (59 tiles) 25.3 and 22.8, 120,000 25.0
+// and 28.5 (with 16 counts in flight 15.5 / 17.8 / 20.3 / 24.9, with 64 18.0 / 20.1 / 20.6 / 21.8 at the first four).
+// Not where one launch does it all: it would set the live count while its other blocks read it.
 constexpr int64_t kFewTiles = 64;
 struct SortScratch {
     uint32_t *ka, *va, *kb, *vb, *hist, *row_total, *rem_block;
@@ -679,8 +681,9 @@ int oppx_sort_by_cell(int64_t n_max, int64_t stride, oppx_move_counters* counter
 #undef OPPX_HIST
 #undef OPPX_HIST_W
                 OPPX_LAUNCH_CHECK("sort_hist");
-                if (!few) sort_rows<<<kBins + (first ? 1 : 0), kB, 0, s>>>(sc.hist, live, n_max, (int64_t)kB * items, sc.row_total,
-                                                                 sc.rem_block, hist_grid, sc.state);
+                if (!few)
+                    sort_rows<<<kBins + (first ? 1 : 0), kB, 0, s>>>(sc.hist, live, n_max, (int64_t)kB * items,
+                                                                     sc.row_total, sc.rem_block, hist_grid, sc.state);
                 OPPX_LAUNCH_CHECK("sort_rows");
 #define OPPX_SCATTER(I, LST, F, FW)                                                                 \
     do {                                                                                              \
