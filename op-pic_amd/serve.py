@@ -319,6 +319,8 @@ class FempicArena:
         slots = list(slots)
         if not slots:
             return PendingResults([], None)
+        if len(set(slots)) != len(slots):
+            raise KeyError("retire: a slot is listed twice")
         keys = []
         for slot in slots:
             tpl, cb, nb, ob = self.res[slot]
@@ -329,10 +331,12 @@ class FempicArena:
                                  bounds.data_ptr(), s), "lower_bound")
         b = bounds.cpu().numpy()  # the step is complete from here on
         main = torch.cuda.current_stream(self.dev)
-        self.copy_stream.wait_stream(main)
+        # Everything that can fail (the pinned arrays, the launches) comes before the arena gives anything up: a
+        # request whose ranges were free again while its particles were not yet marked removed would be stepped as part
+        # of the next one admitted there.
         staged, now, beside, after = [], [], [], []
         for j, slot in enumerate(slots):
-            tpl, cb, nb, ob = self.res.pop(slot)
+            tpl, cb, nb, ob = self.res[slot]
             lo, hi = int(b[2 * j]), int(b[2 * j + 1])
             k, nn = hi - lo, tpl.n_nodes
             pin = lambda shape, dt: torch.empty(shape, dtype=dt, pin_memory=True)
@@ -343,27 +347,31 @@ class FempicArena:
             beside += [copy_job(out[name].data_ptr(), t.data_ptr() + 8 * lo, 8 * k, t.shape[0], 8 * k, 8 * self.cap)
                        for name, t in (("pos", self.pos), ("vel", self.vel), ("lc", self.lc))]
             staged.append((out, k, cb))
-            self.dropping += k
             after += [copy_job(self.p2c.data_ptr() + 4 * lo, 0, 4 * k, fill=MAX_CELL_INDEX * 0x100000001),
                       # leaves the particle set at the next sort; its node rows are empty
                       copy_job(self.node_start.data_ptr() + 4 * nb, 0, 4 * nn),
                       copy_job(self.node_end.data_ptr() + 4 * nb, 0, 4 * nn)]
+        try:
+            self.copy_stream.wait_stream(main)
+            copy_batch(now, s, self.link_blocks)
+            copy_batch(beside, self.copy_stream.cuda_stream, self.link_blocks)
+            copy_batch(after, s)
+            done = (torch.cuda.Event(), torch.cuda.Event())
+            done[0].record(main)
+            done[1].record(self.copy_stream)
+        except BaseException:  # nothing may still write the pinned arrays once they go back to the allocator
+            torch.cuda.synchronize(self.dev)
+            raise
+        pending = PendingResults(staged, done)
+        for slot, (_, k, _) in zip(slots, staged):
+            tpl, cb, nb, ob = self.res.pop(slot)
+            self.dropping += k
             self.cells.release(cb)
             self.nodes.release(nb)
             if ob >= 0:
                 self.ovl.release(ob)
             self.slots_free.append(slot)
-        try:
-            copy_batch(now, s, self.link_blocks)
-            copy_batch(beside, self.copy_stream.cuda_stream, self.link_blocks)
-            copy_batch(after, s)
-        except BaseException:  # nothing may still write the pinned arrays once they go back to the allocator
-            torch.cuda.synchronize(self.dev)
-            raise
-        done = (torch.cuda.Event(), torch.cuda.Event())
-        done[0].record(main)
-        done[1].record(self.copy_stream)
-        return PendingResults(staged, done)
+        return pending
 
     @staticmethod
     def for_budget(arena_bytes: float, device="cuda", max_insts: int = 4096) -> "FempicArena":
