@@ -181,10 +181,13 @@ class FempicArena:
         self.slots_free = list(range(max_insts - 1, -1, -1))
         self.res = {}  # slot -> (template, cb, nb, ob)
         self.dropping = 0  # particles of retired requests still in the set (marked removed) until the next sort
-        # results of retired requests go to the host on their own stream, beside the next step: few blocks fill the link,
-        # and all the blocks of a large result would take the step's place on the device until the link has drained. A
-        # stream of 443 requests, some of 50 M particles: p99 step 62-67 ms with all blocks, 34 with 32, 38 with 64, 43
-        # with 256; 20 MB of small results 610 us with all, 650 with 32
+        # results of retired requests go to the host on their own stream, beside the next step: rows from engine_bytes on
+        # through the copy engine, which leaves the device to the step, shorter ones together in one kernel, where a copy
+        # each would cost its launch, on as many blocks as fill the link. A stream of 443 requests, some of 50 M particles:
+        # p99 step 36 ms and 2.7e9 particles/s with every row in the kernel, 16.5 ms and 3.0e9 so (17 ms from 256 KiB or
+        # 8 MiB on, 19 from 64 MiB); before there was a kernel for it, strided copies through a device temporary, 71 ms and
+        # 2.5e9 in the same run. 20 MB of small results 650 us on 32 blocks, 610 on all.
+        self.engine_bytes = 1 << 20
         self.link_blocks = 32
         self.copy_stream = torch.cuda.Stream(device=self.dev)
         self.cap, self.size = P, 0
@@ -304,6 +307,21 @@ class FempicArena:
         self.size = self.published = int(self.counters[0].item())  # the live count after the finalize (host sync)
         self.dropping = 0  # the finalize dropped the retired particles
 
+    def _to_host(self, rows, stream):
+        """(pinned array, device array, first, count): `count` elements from `first` on of every row, on `stream`.
+        Short rows go in one launch, long ones one by one through the copy engine."""
+        jobs = []
+        for dst, src, first, count in rows:
+            el = src.element_size()
+            if count * el < self.engine_bytes:
+                jobs.append(copy_job(dst.data_ptr(), src.data_ptr() + el * first, el * count, src.shape[0], el * count,
+                                     el * src.stride(0)))
+                continue
+            with self.torch.cuda.stream(stream):
+                for to, row in zip(dst, src):
+                    to.copy_(row[first:first + count], non_blocking=True)
+        copy_batch(jobs, stream.cuda_stream, self.link_blocks)
+
     def retire(self, slots) -> list:
         """Hand back requests' states (each contiguous after the sort) and free their ranges."""
         return self.retire_async(slots).wait()
@@ -342,10 +360,9 @@ class FempicArena:
             pin = lambda shape, dt: torch.empty(shape, dtype=dt, pin_memory=True)
             out = dict(pos=pin((3, k), torch.float64), vel=pin((3, k), torch.float64), lc=pin((4, k), torch.float64),
                        p2c=pin((k,), torch.int32), charge_f32=pin((nn,), torch.float32))
-            now += [copy_job(out["p2c"].data_ptr(), self.p2c.data_ptr() + 4 * lo, 4 * k),
-                    copy_job(out["charge_f32"].data_ptr(), self.charge_f32.data_ptr() + 4 * nb, 4 * nn)]
-            beside += [copy_job(out[name].data_ptr(), t.data_ptr() + 8 * lo, 8 * k, t.shape[0], 8 * k, 8 * self.cap)
-                       for name, t in (("pos", self.pos), ("vel", self.vel), ("lc", self.lc))]
+            now.append((out["charge_f32"][None], self.charge_f32[None], nb, nn))
+            now.append((out["p2c"][None], self.p2c[None], lo, k))
+            beside += [(out["pos"], self.pos, lo, k), (out["vel"], self.vel, lo, k), (out["lc"], self.lc, lo, k)]
             staged.append((out, k, cb))
             after += [copy_job(self.p2c.data_ptr() + 4 * lo, 0, 4 * k, fill=MAX_CELL_INDEX * 0x100000001),
                       # leaves the particle set at the next sort; its node rows are empty
@@ -353,8 +370,8 @@ class FempicArena:
                       copy_job(self.node_end.data_ptr() + 4 * nb, 0, 4 * nn)]
         try:
             self.copy_stream.wait_stream(main)
-            copy_batch(now, s, self.link_blocks)
-            copy_batch(beside, self.copy_stream.cuda_stream, self.link_blocks)
+            self._to_host(now, main)
+            self._to_host(beside, self.copy_stream)
             copy_batch(after, s)
             done = (torch.cuda.Event(), torch.cuda.Event())
             done[0].record(main)
