@@ -102,7 +102,8 @@ __global__ void offset_indices_kernel(int32_t* __restrict__ base, int64_t n, int
 constexpr int kSegs = 32;      // row segments a launch takes (their table is a kernel argument)
 constexpr int kSegBlock = 256;
 constexpr int kSegUnits = 2;   // units a thread has in flight
-constexpr int64_t kMaxGrid = 1 << 30;
+constexpr int64_t kMaxChunks = 1 << 30;  // of a launch (a 32-bit index)
+constexpr int64_t kMaxGrid = 1 << 22;    // its workgroups, which stride over the chunks: a grid of 2^32 threads is refused
 
 // One contiguous piece of memory: `units` units of 1 << shift bytes and the words behind them.
 struct CopySeg {
@@ -332,7 +333,8 @@ int oppx_copy_batch(int n, const oppx_copy_job* jobs, int max_blocks, void* stre
     int64_t chunks = 0;
     const auto launch = [&]() -> int {
         if (T.n == 0) return OPPX_OK;
-        const int64_t g = max_blocks && max_blocks < chunks ? max_blocks : chunks;
+        int64_t g = chunks < kMaxGrid ? chunks : kMaxGrid;
+        if (max_blocks && max_blocks < g) g = max_blocks;
         copy_segs_kernel<<<(unsigned)g, kSegBlock, 0, as_stream(stream)>>>(T, (uint32_t)chunks);
         OPPX_LAUNCH_CHECK("copy_batch");
         T.n = 0;
@@ -358,11 +360,11 @@ int oppx_copy_batch(int n, const oppx_copy_job* jobs, int max_blocks, void* stre
             S.count = (uint8_t)J.count;
             int64_t need = (S.units + kSegBlock * kSegUnits - 1) / (kSegBlock * kSegUnits);
             if (need == 0) need = 1;
-            if (T.n == kSegs || chunks + need > kMaxGrid) {
+            if (T.n == kSegs || chunks + need > kMaxChunks) {
                 const int rc = launch();
                 if (rc != OPPX_OK) return rc;
             }
-            OPPX_ARG_CHECK(need <= kMaxGrid, "oppx_copy_batch: row too long");
+            OPPX_ARG_CHECK(need <= kMaxChunks, "oppx_copy_batch: row too long");
             S.chunk0 = (uint32_t)chunks;
             T.s[T.n++] = S;
             chunks += need;
