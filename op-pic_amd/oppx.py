@@ -584,7 +584,8 @@ class FempicDevice:
                 src = src.contiguous()
                 jobs.append(copy_job(to.data_ptr(), src.data_ptr() if name in copied else 0,
                                      to.numel() * to.element_size()))
-        copy_batch(jobs, self.stream())
+        with torch.cuda.device(self.dev):  # the launch goes to the current device
+            copy_batch(jobs, self.stream())
         g.pending = g.staged = False
         g._rebind()
         return g
