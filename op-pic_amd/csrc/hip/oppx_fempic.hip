@@ -982,8 +982,9 @@ __global__ void __launch_bounds__(DENSE ? kMaxBlock : kBlock) fempic_walk_kernel
         nfault += t.faults;
     };
     if constexpr (DENSE) {
-        if (blockIdx.x < 2 * kXcds)  // its chunks are many and small: a few blocks add up all the records
-            for (uint32_t q = blockIdx.x * BT + threadIdx.x; q < nlive; q += 2 * kXcds * BT) take(W.rec[q]);
+        const uint32_t adders = gridDim.x < 2u * kXcds ? gridDim.x : 2u * kXcds;
+        if (blockIdx.x < adders)  // its chunks are many and small: a few blocks add up all the records
+            for (uint32_t q = blockIdx.x * BT + threadIdx.x; q < nlive; q += adders * BT) take(W.rec[q]);
     } else {  // the records of the block's chunks, without a barrier between them
         int any = 0;
 #pragma unroll 4
