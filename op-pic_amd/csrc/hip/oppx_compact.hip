@@ -85,22 +85,23 @@ __global__ void __launch_bounds__(kB) hf_count(const uint64_t* __restrict__ bits
 }
 
 // Record v to hole h.
-__device__ __forceinline__ void move_record(const CompTable& T, int64_t v, int64_t h) {
-            for (int c0 = 0; c0 < T.n; c0 += kCopyBatch) {
-                uint64_t x[kCopyBatch];
-    #pragma unroll
-                for (int u = 0; u < kCopyBatch; u++) {
-                    if (c0 + u >= T.n) continue;
-                    if ((T.wide >> (c0 + u)) & 1ull) x[u] = reinterpret_cast<const uint64_t*>(T.base[c0 + u])[v];
-                    else x[u] = reinterpret_cast<const uint32_t*>(T.base[c0 + u])[v];
-                }
-    #pragma unroll
-                for (int u = 0; u < kCopyBatch; u++) {
-                    if (c0 + u >= T.n) continue;
-                    if ((T.wide >> (c0 + u)) & 1ull) reinterpret_cast<uint64_t*>(T.base[c0 + u])[h] = x[u];
-                    else reinterpret_cast<uint32_t*>(T.base[c0 + u])[h] = (uint32_t)x[u];
-                }
-            }
+template <typename Index>
+__device__ __forceinline__ void move_record(const CompTable& T, Index v, Index h) {
+    for (int c0 = 0; c0 < T.n; c0 += kCopyBatch) {
+        uint64_t x[kCopyBatch];
+#pragma unroll
+        for (int u = 0; u < kCopyBatch; u++) {
+            if (c0 + u >= T.n) continue;
+            if ((T.wide >> (c0 + u)) & 1ull) x[u] = reinterpret_cast<const uint64_t*>(T.base[c0 + u])[v];
+            else x[u] = reinterpret_cast<const uint32_t*>(T.base[c0 + u])[v];
+        }
+#pragma unroll
+        for (int u = 0; u < kCopyBatch; u++) {
+            if (c0 + u >= T.n) continue;
+            if ((T.wide >> (c0 + u)) & 1ull) reinterpret_cast<uint64_t*>(T.base[c0 + u])[h] = x[u];
+            else reinterpret_cast<uint32_t*>(T.base[c0 + u])[h] = (uint32_t)x[u];
+        }
+    }
 }
 
 // Every block scans the block counts into LDS itself (group e: blocks [e * per, (e + 1) * per)), then its
@@ -181,16 +182,20 @@ __global__ void __launch_bounds__(kB) hf_fill(const uint64_t* __restrict__ bits,
         if (hw == 0ull) continue;  // inconsistent bitmap: never write outside [0, S)
         const int64_t h = lo * 64 + (__ffsll((long long)hw) - 1);
         if (h < 0 || h >= S) continue;
-        move_record(T, v, h);
+        move_record<int64_t>(T, v, h);
     }
 }
 
-// The whole fill of a small set by one block: words, prefixes and searches in LDS, one launch instead of two. A set of up
-// to 8,192 particles is filled so, whatever share of it was removed: us in a graph, two launches and one, with 3, 10, 30
-// and 60% removed: 4,000 particles 7.1 / 8.1 / 16.5 / 26.7 and 5.2 / 5.6 / 10.1 / 15.7, 8,192 7.8 / 8.6 / 17.4 / 28.5
-// and 5.6 / 6.9 / 15.9 / 27.9. Beyond, one block is too few where many records move: 16,384 with 10% 9.2 and 12.6.
+// The whole fill of a small set by one block, one launch instead of two. Each thread puts the places it looks at into two
+// lists in LDS, the holes below the new size and the live records past it, in the order in which they belong
+// together, so that a record needs no search and the moves are dense however much was removed. us in a graph,
+// with 3, 10, 30, 50, 70 and 90% removed, five launches as it once was / the two of hf_count and hf_fill / this: 2,000
+// particles 10.3 10.5 11.3 12.0 12.3 13.2 / 8.2 8.0 7.9 8.5 8.7 9.9 / 4.5 4.3 4.5 4.4 4.4 4.2; 4,000 10.6 11.5 11.9 12.7
+// 12.5 14.5 / 7.4 8.5 9.0 9.2 9.2 10.8 / 4.8 4.9 5.5 5.8 5.4 4.9; 8,192 11.3 12.2 12.2 12.7 13.0 14.2 / 7.6 8.6 8.7 9.2 9.6
+// 11.0 / 5.4 6.9 9.2 9.3 8.7 6.6 (a search for every record of the tail took 40 at the last). Beyond, one block is too few.
 __global__ void __launch_bounds__(kSmallThreads) hf_small(const uint64_t* __restrict__ bits,
                                                           oppx_move_counters* __restrict__ ctr, CompTable T, int64_t n_max) {
+    __shared__ uint16_t s_hole[32 * kSmallWords], s_live[32 * kSmallWords];  // at most half of the set moves
     __shared__ uint64_t s_bits[kSmallWords];
     __shared__ uint32_t s_pre[kSmallWords], s_wave[kSmallThreads / kWave];
     const int N = (int)live_count(ctr, n_max), W = (int)words_of(N);
@@ -216,31 +221,27 @@ __global__ void __launch_bounds__(kSmallThreads) hf_small(const uint64_t* __rest
     __syncthreads();
     const int R = (int)total, S = N - R;
     const bool some = R > 0 && R <= N;
+    // holes below the new size (R > 0 and not past N, so S is a place in the set)
+    const int moves = some ? (int)s_pre[S >> 6] + __popcll(s_bits[S >> 6] & ((1ull << (S & 63)) - 1ull)) : 0;
     if (threadIdx.x == 0) {
         ctr->removed = R;
-        const uint64_t lowmask = (1ull << (S & 63)) - 1ull;
-        ctr->holes_low = some && S < N ? (int)s_pre[S >> 6] + __popcll(s_bits[S >> 6] & lowmask) : 0;
+        ctr->holes_low = moves;
         if (some) ctr->size = S;
     }
-    if (!some) return;
-    for (int v = S + (int)threadIdx.x; v < N; v += kSmallThreads) {
+    if (moves == 0) return;
+    for (int v = (int)threadIdx.x; v < N; v += kSmallThreads) {
         const uint64_t word = s_bits[v >> 6];
-        const int j = v & 63;
-        if ((word >> j) & 1ull) continue;  // a hole itself
-        const int k = (N - 1 - v) - (R - ((int)s_pre[v >> 6] + __popcll(word & ((1ull << j) - 1ull))));
-        int lo = 0, hi = W - 1;
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if ((int)s_pre[mid] <= k) lo = mid;
-            else hi = mid - 1;
+        const int j = v & 63, below = (int)s_pre[v >> 6] + __popcll(word & ((1ull << j) - 1ull));
+        const bool hole = (word >> j) & 1ull;
+        if (v < S) {
+            if (hole) s_hole[below] = (uint16_t)v;
+        } else if (!hole) {
+            const int k = (N - 1 - v) - (R - below);  // its place among the live records, from the end
+            if (k >= 0) s_live[k] = (uint16_t)v;       // (below 0 only where a bit past N is set)
         }
-        uint64_t hw = s_bits[lo];
-        for (int r = k - (int)s_pre[lo]; r > 0 && hw; r--) hw &= hw - 1ull;
-        if (hw == 0ull) continue;  // inconsistent bitmap: never write outside [0, S)
-        const int h = lo * 64 + (__ffsll((long long)hw) - 1);
-        if (h >= S) continue;
-        move_record(T, v, h);
     }
+    __syncthreads();
+    for (int k = (int)threadIdx.x; k < moves; k += kSmallThreads) move_record<uint32_t>(T, s_live[k], s_hole[k]);
 }
 
 struct Scratch {
@@ -286,8 +287,12 @@ int holefill_impl(int64_t n_max, int64_t stride, oppx_move_counters* counters, c
         OPPX_LAUNCH_CHECK("hf_count");
     }
     const int per = (int)((sc.nb + kMaxGroups - 1) / kMaxGroups);
-    // one block for 8 * kB particles: with a few percent removed, a thread has at most one record to move
-    int64_t g = (n_max + 8 * kB - 1) / (8 * kB);
+    // A thread for every particle, so that at most one record is a thread's to move, whatever share was removed; more than
+    // 1,024 blocks add nothing. us, with 3, 30, 60 and 90% removed, five launches as it once was / a block for 2,048
+    // particles / this: 9,000 particles 11.5 12.6 12.9 14.3 / 8.2 17.5 26.7 40.6 / 7.8 9.0 9.4 10.9, 131,072 14.9 15.5 16.3
+    // 16.9 / 9.8 20.5 30.9 52.5 / 9.9 11.1 11.6 12.9, 1 M 18.8 33.1 41.2 50.6 / 12.3 29.8 41.5 60.4 / 12.3 25.8 33.2 37.9,
+    // 24 M 332 824 1,060 1,444 / 320 826 722 844 / 321 826 722 842.
+    int64_t g = (n_max + kB - 1) / kB;
     g = g < 1 ? 1 : (g > 1024 ? 1024 : g);
     CompTable T{};
     for (int q = 0, d = 0; q < n_dats;) {  // flatten the dats; a full table is launched and started again
