@@ -584,8 +584,11 @@ class FempicDevice:
                 src = src.contiguous()
                 jobs.append(copy_job(to.data_ptr(), src.data_ptr() if name in copied else 0,
                                      to.numel() * to.element_size()))
-        with torch.cuda.device(self.dev):  # the launch goes to the current device
+        if self.dev.index in (None, torch.cuda.current_device()):
             copy_batch(jobs, self.stream())
+        else:  # a launch goes to the current device; the switch takes 5 us, so not where there is nothing to switch
+            with torch.cuda.device(self.dev):
+                copy_batch(jobs, self.stream())
         g.pending = g.staged = False
         g._rebind()
         return g
