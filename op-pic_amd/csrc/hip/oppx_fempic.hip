@@ -1383,9 +1383,13 @@ __global__ void __launch_bounds__(kBlock) gather_records_kernel(int64_t n_max, i
     n = n < 0 ? 0 : (n > n_max ? n_max : n);
     // A permuted record's lines in one L2: each XCD takes runs of `group` tiles, an eighth of them all in smaller sets, 64
     // tiles (16,384 particles) in larger ones, where eight regions far apart cost more than neighbouring XCDs' shared
-    // lines. us, single tiles (as before) / runs of 64 / eighths: 2.4 M particles of 24 instances 61 / 48 / 42, 3 M 66 / 56
-    // / 55, 24 M (x-fastest) 575 / 564 / 560, 24 M (Morton) 522 / 511 / 517, 50 M 1,153 / 1,001 / 1,033, 47 M of 128
-    // instances 1,197 / 1,104 / 1,205, 100 M displaced by up to 100,000 places 2,940 / 2,985 / 3,793.
+    // lines. With 8,192 workgroups a large set's blocks strode over their tiles and drifted apart; with 65,536 most of them
+    // take one tile, and they are few enough for a set of which little is left alive (16 of 113 M in order 299 / 286 / 269
+    // us, 326 with 2^18). us, single tiles on 8,192 workgroups as it once was / these runs on 8,192 / on 65,536: 3 M
+    // displaced by up to 100,000 places 84 / 68 / 58, 8 M 222 / 219 / 200, 24 M 702 / 679 / 615, in order 472 / 458 / 412,
+    // 100 M 2,924 / 2,915 / 2,722, in order 1,963 / 1,892 / 1,798; an ensemble of 256 instances and 102 M particles after
+    // its first step 3,153 / 3,215 / 2,584, 62 M after the fourth 1,773 / 1,772 / 1,515. Runs of 16 or 256 tiles 2,567 and
+    // 2,699 at the last but one, eighths 2,936.
     const uint32_t tiles = (uint32_t)((n + kBlock - 1) / kBlock);
     const uint32_t group = tiles > 65536u ? 64u : (tiles + kXcds - 1) / kXcds;
     const uint32_t slots = group ? (tiles + kXcds * group - 1) / (kXcds * group) * group : 0;  // tiles of an XCD
@@ -1809,7 +1813,7 @@ int oppx_gather_records(int64_t n_max, int64_t stride, oppx_move_counters* count
     OPPX_ARG_CHECK(n_max >= 0 && stride >= n_max, "oppx_gather_records: need 0 <= n_max <= stride");
     if (n_max == 0) return OPPX_OK;
     unsigned g = grid_for(n_max, kBlock);
-    g = xcd_grid(g > 8192 ? 8192 : g);
+    g = xcd_grid(g > 65536 ? 65536 : g);
     gather_records_kernel<<<g, kBlock, 0, as_stream(stream)>>>(n_max, stride, counters, perm, rec, pos, vel,
                                                               &counters->faults);
     OPPX_LAUNCH_CHECK("gather_records");
