@@ -468,18 +468,31 @@ __device__ __forceinline__ void coop_walk(const StepArgs& P, CoopBuf& C, bool mo
                 walk = walk_state(res, h, inline_hops);
                 moving = walk == kWalkOn;
             }
-            // every value read above has been used, so the next batch may overwrite the buffer
+            // The next batch may overwrite the buffer: its loads need C.cell, and LDS reads return in order, so those
+            // above have returned before any of them is issued.
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         }
     }
 }
 
+// Which first passes fetch together: all blocks of 256, and those of 1024 that read through a permutation. The 16 buffers
+// of a block of 1024 take 84 KB, so that one block fits a CU where two with lane-wise loads do (54 registers). In place
+// that costs more than the fetch gains: 113 M particles of 256 instances, the move of a first / second step 7.12 / 7.07 ms
+// with the fetch, 5.83 / 6.11 without (5.86 / 6.16 as it once was), and 7.18 / 6.33 where it stages records; through a
+// permutation, where the reads of the particles themselves are the longer wait, 8.96 with it and 9.56 without.
+template <int BS, bool GATHER>
+constexpr bool kCoop = BS == kBlock || GATHER;
+
 // LDS of a first-pass block: the record staging, the waves' fetch buffers and the deposit table in turn.
-template <int BS>
+template <int BS, bool COOP>
 union FirstLds {
     DepositTable dep;
     double2 stage[3 * BS];
     CoopBuf coop[BS / kWave];
+};
+template <int BS>
+union FirstLds<BS, false> {
+    DepositTable dep;
 };
 
 // What the first pass leaves for the walk pass: one record per block, and the blocks' worklists, `parts`
@@ -491,7 +504,7 @@ struct WorkList {
 };
 
 template <int BS, bool PUSH, bool DH, bool DEPOSIT, bool BATCH, bool GATHER, bool DENSE>
-__global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(7)))
+__global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(BS == kBlock ? 7 : 4)))
 fempic_first_kernel(StepArgs P, uint32_t nblocks, int inline_hops, WorkList W) {
     int64_t n = P.ctr->size;
     n = n < 0 ? 0 : (n > P.n_max ? P.n_max : n);
@@ -504,6 +517,8 @@ fempic_first_kernel(StepArgs P, uint32_t nblocks, int inline_hops, WorkList W) {
     __shared__ unsigned s_order;  // deposits << 12 + new first nodes; from kKeep on: the table stays
     constexpr unsigned kKeep = 1u << 28;
     if (threadIdx.x == 0) s_pending = s_order = 0;  // a barrier comes before their first use
+    constexpr bool COOP = kCoop<BS, GATHER>;
+    if constexpr (!COOP) __syncthreads();  // here, where no load is waited for yet
     const uint32_t b = xcd_block(blockIdx.x, nlive);
     int64_t i = (int64_t)b * BS + threadIdx.x;
     const bool live = i < n;
@@ -536,7 +551,7 @@ fempic_first_kernel(StepArgs P, uint32_t nblocks, int inline_hops, WorkList W) {
     bool removed = false, pending = false, pushed = false, p2c_done = false, lc_done = false;
     int h = 0;
     double l0 = 0.0, l1 = 0.0, l2 = 0.0, l3 = 0.0;
-    __shared__ FirstLds<BS> s_lds;
+    __shared__ FirstLds<BS, COOP> s_lds;
     DepositTable& s_table = s_lds.dep;
 
     // push: the particle's new position and velocity (or, for a particle this pass does not push, the
@@ -607,27 +622,34 @@ fempic_first_kernel(StepArgs P, uint32_t nblocks, int inline_hops, WorkList W) {
             }
         }
     }
-    // records out (block-uniform): every live particle's {x, y, z, vx, vy, vz}. The wave's 64 records pass through
-    // LDS so that each of the three 16-byte stores of a lane lands next to its neighbours' (1 KB contiguous per
-    // instruction)
+    // records out (block-uniform): every live particle's {x, y, z, vx, vy, vz}. Where there is LDS for it the wave's 64
+    // records pass through it so that each of the three 16-byte stores of a lane lands next to its neighbours' (1 KB
+    // contiguous per instruction)
     if (P.rec_out) {
-        const int wave = threadIdx.x / kWave;
-        f64x2* slice = reinterpret_cast<f64x2*>(s_lds.stage) + wave * (3 * kWave);
-        if (live) {
-            slice[3 * lane] = f64x2{x, y};
-            slice[3 * lane + 1] = f64x2{z, vx};
-            slice[3 * lane + 2] = f64x2{vy, vz};
-        }
-        __syncthreads();
-        const int64_t base = (int64_t)b * BS + wave * kWave;  // first particle of the wave
-        const int64_t nw = n - base;                          // live particles of the wave
-        f64x2* dst = reinterpret_cast<f64x2*>(P.rec_out + 6 * base);
-        for (int k = 0; k < 3; k++) {
-            const int q = k * kWave + lane;  // pair q of the wave's 192: record q / 3
-            if (q / 3 < nw) __builtin_nontemporal_store(slice[q], dst + q);
+        if constexpr (COOP) {
+            const int wave = threadIdx.x / kWave;
+            f64x2* slice = reinterpret_cast<f64x2*>(s_lds.stage) + wave * (3 * kWave);
+            if (live) {
+                slice[3 * lane] = f64x2{x, y};
+                slice[3 * lane + 1] = f64x2{z, vx};
+                slice[3 * lane + 2] = f64x2{vy, vz};
+            }
+            __syncthreads();
+            const int64_t base = (int64_t)b * BS + wave * kWave;  // first particle of the wave
+            const int64_t nw = n - base;                          // live particles of the wave
+            f64x2* dst = reinterpret_cast<f64x2*>(P.rec_out + 6 * base);
+            for (int k = 0; k < 3; k++) {
+                const int q = k * kWave + lane;  // pair q of the wave's 192: record q / 3
+                if (q / 3 < nw) __builtin_nontemporal_store(slice[q], dst + q);
+            }
+        } else if (live) {  // ordinary stores: L2 merges a wave's three partial-line writes into whole lines
+            f64x2* r = reinterpret_cast<f64x2*>(P.rec_out + 6 * i);
+            r[0] = f64x2{x, y};
+            r[1] = f64x2{z, vx};
+            r[2] = f64x2{vy, vz};
         }
     }
-    __syncthreads();  // the staging's readers are done, and s_pending is set
+    if constexpr (COOP) __syncthreads();  // the staging's readers are done, and s_pending is set
     {   // the indexes, opaque: addresses formed above are not kept in registers across the walk
         uint32_t at = (uint32_t)i;
         asm volatile("" : "+v"(at));
@@ -649,7 +671,16 @@ fempic_first_kernel(StepArgs P, uint32_t nblocks, int inline_hops, WorkList W) {
         }
         moving = !removed && !fault;
     }
-    coop_walk(P, s_lds.coop[threadIdx.x / kWave], moving, lane, x, y, z, cell, l0, l1, l2, l3, h, walk, inline_hops);
+    if constexpr (COOP) {
+        coop_walk(P, s_lds.coop[threadIdx.x / kWave], moving, lane, x, y, z, cell, l0, l1, l2, l3, h, walk, inline_hops);
+    } else {
+        while (moving) {
+            const int r = hop_eval(P, x, y, z, cell, l0, l1, l2, l3);
+            h++;
+            walk = walk_state(r, h, inline_hops);
+            moving = walk == kWalkOn;
+        }
+    }
     removed = removed || walk == kWalkOut;
     fault = fault || walk == kWalkBad;
     pending = walk == kWalkHandOff;
