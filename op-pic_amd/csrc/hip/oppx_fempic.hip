@@ -106,6 +106,7 @@ struct BlockStat {
     int pending;  // worklist entries of the block; kScattered: none, and the walk pass deposits its particles
 };
 constexpr int kScattered = -1;
+constexpr uint32_t kAdders = 2 * kXcds;  // workgroups of a dense walk pass that add the records up: it has at least these
 
 // The block's totals, valid in thread 0 (ends with the other threads free to leave).
 __device__ __forceinline__ BlockStat block_totals(long long hsum, int hmax, int nrem, int nfault) {
@@ -987,7 +988,10 @@ __global__ void __launch_bounds__(kQuadBlock) fempic_quad_kernel(StepArgs P, uin
 // whole charge array in LDS, adds to it there, and adds it to the global one at its end, consecutive lanes to
 // consecutive nodes. Scattered adds to global memory go at 20 a nanosecond over the chip, such a sweep at 100, and LDS
 // takes 16,384 scattered adds a CU in 8 us: 1 M particles in no order on 9,261 nodes,
-// a fused pass 234 -> 114 us; 6 M on 15,625: 1,046 -> 632 us; 1 M in cell order (no block scattered) 70 -> 73 us.
+// a fused pass 236 -> 112 us; 6 M on 15,625: 1,083 -> 627 us. In cell order no block is scattered, and a block that finds
+// nothing in its first chunk looks at the records of all the others at once: a pass over 1 M on 2,197 nodes 66 (one chunk after
+// the other 66, without the form 64, a pass of before it 68), 6 M on 2,197 295 (299, 292, 295), 20 M on 15,625 943 (975, 950,
+// 950). A look ahead of every first chunk cost unordered sets 0.8 us a pass.
 template <bool DEPOSIT, bool DENSE>
 __global__ void __launch_bounds__(DENSE ? kMaxBlock : kBlock) fempic_walk_kernel(StepArgs P, WorkList W, uint32_t nblocks,
                                                                                  int per) {
@@ -1006,6 +1010,7 @@ __global__ void __launch_bounds__(DENSE ? kMaxBlock : kBlock) fempic_walk_kernel
     long long hsum = 0;
     int hmax = 0, nrem = 0, nfault = 0;
     bool used = false;  // s_dense holds something (uniform over the block)
+    bool looked = false;
     auto take = [&](const BlockStat& t) {
         hsum += (long long)t.hops;
         hmax = hmax > t.max_hops ? hmax : t.max_hops;
@@ -1013,9 +1018,8 @@ __global__ void __launch_bounds__(DENSE ? kMaxBlock : kBlock) fempic_walk_kernel
         nfault += t.faults;
     };
     if constexpr (DENSE) {
-        const uint32_t adders = gridDim.x < 2u * kXcds ? gridDim.x : 2u * kXcds;
-        if (blockIdx.x < adders)  // its chunks are many and small: a few blocks add up all the records
-            for (uint32_t q = blockIdx.x * BT + threadIdx.x; q < nlive; q += adders * BT) take(W.rec[q]);
+        if (blockIdx.x < kAdders)  // its chunks are many and small: a few blocks add up all the records
+            for (uint32_t q = blockIdx.x * BT + threadIdx.x; q < nlive; q += kAdders * BT) take(W.rec[q]);
     } else {  // the records of the block's chunks, without a barrier between them
         int any = 0;
 #pragma unroll 4
@@ -1034,7 +1038,19 @@ __global__ void __launch_bounds__(DENSE ? kMaxBlock : kBlock) fempic_walk_kernel
         const uint32_t first = x + kXcds * c * (uint32_t)per;  // first-pass blocks first, first + 8, ...
         BlockStat t{0ull, 0, 0, 0, 0};
         if ((int)threadIdx.x < per && c * (uint32_t)per + threadIdx.x < mine) t = W.rec[first + kXcds * threadIdx.x];
-        if (!__syncthreads_or(t.pending)) continue;
+        if (!__syncthreads_or(t.pending)) {
+            if (DENSE && !looked) {  // particles in order, most likely: the chunks to come at one look
+                looked = true;
+                int any = 0;
+                for (uint32_t e = threadIdx.x;; e += BT) {
+                    const uint32_t k = (c + (1 + e / (uint32_t)per) * (gridDim.x / kXcds)) * (uint32_t)per + e % (uint32_t)per;
+                    if (k >= mine) break;  // (k grows with e)
+                    any |= W.rec[x + kXcds * k].pending;
+                }
+                if (!__syncthreads_or(any)) break;
+            }
+            continue;
+        }
         if constexpr (DENSE) {
             s_off[threadIdx.x] = t.pending;
             if (__syncthreads_or(t.pending == kScattered)) {
@@ -1570,7 +1586,8 @@ bool launch_two_pass(const StepArgs& P, int64_t n_max, void* work, size_t work_b
     const unsigned cap = dense ? 256u : (rare ? 64u : resident_blocks(plain, kBlock));
     unsigned wg = ((g + kXcds - 1) / kXcds + per - 1) / per * kXcds;  // every chunk of every XCD
     if (wg > cap) wg = cap / kXcds * kXcds;
-    if (wg < (unsigned)kXcds) wg = kXcds;
+    const unsigned least = dense ? kAdders : (unsigned)kXcds;
+    if (wg < least) wg = least;
     if constexpr (DEPOSIT) {
         if (dense) {
             const size_t bytes = (size_t)P.n_nodes * sizeof(double);
