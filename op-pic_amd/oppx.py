@@ -584,7 +584,7 @@ class FempicDevice:
                 src = src.contiguous()
                 jobs.append(copy_job(to.data_ptr(), src.data_ptr() if name in copied else 0,
                                      to.numel() * to.element_size()))
-        if self.dev.index in (None, torch.cuda.current_device()):
+        if self.dev.index is None or self.dev.index == torch.cuda.current_device():
             copy_batch(jobs, self.stream())
         else:  # a launch goes to the current device; the switch takes 5 us, so not where there is nothing to switch
             with torch.cuda.device(self.dev):
