@@ -103,9 +103,10 @@ typedef struct oppx_move_counters {
  * `sort_items` (4, 8, 16 or 32) is the elements per thread of the radix sort passes (a block sorts
  * 256 * sort_items keys; sets of fewer than 12 million particles take at most 8, below 2^20 at most
  * 4); `inline_hops` >= 1 selects the two-pass move (walk evaluations done in the first,
- * one-lane-per-particle pass before a particle goes to the worklist walk; a set of at most 256 blocks of
- * that pass walks to the end in it from 16 on), 0 the cooperative tile walk. Process-wide; chosen by the autotuner (op-pic_amd/autotune.py) or
- * oppx_set_tuning. Results do not depend on it. */
+ * one-lane-per-particle pass before a particle goes to the worklist walk; from 16 on a set of at most 256
+ * blocks of that pass, or of 768 blocks of 256, walks to the end in it), 0 the cooperative tile walk.
+ * Process-wide; chosen by the autotuner (op-pic_amd/autotune.py) or oppx_set_tuning. Results do not depend
+ * on it. */
 typedef struct oppx_tuning {
     int32_t tile;
     int32_t refill_min;

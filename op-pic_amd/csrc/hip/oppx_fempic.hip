@@ -476,14 +476,6 @@ __device__ __forceinline__ void coop_walk(const StepArgs& P, CoopBuf& C, bool mo
     }
 }
 
-// Which first passes fetch together: all blocks of 256, and those of 1024 that read through a permutation. The 16 buffers
-// of a block of 1024 take 84 KB, so that one block fits a CU where two with lane-wise loads do (54 registers). In place
-// that costs more than the fetch gains: 113 M particles of 256 instances, the move of a first / second step 7.12 / 7.07 ms
-// with the fetch, 5.83 / 6.11 without (5.86 / 6.16 as it once was), and 7.18 / 6.33 where it stages records; through a
-// permutation, where the reads of the particles themselves are the longer wait, 8.96 with it and 9.56 without.
-template <int BS, bool GATHER>
-constexpr bool kCoop = BS == kBlock || GATHER;
-
 // LDS of a first-pass block: the record staging, the waves' fetch buffers and the deposit table in turn.
 template <int BS, bool COOP>
 union FirstLds {
@@ -504,8 +496,8 @@ struct WorkList {
     int parts;
 };
 
-template <int BS, bool PUSH, bool DH, bool DEPOSIT, bool BATCH, bool GATHER, bool DENSE>
-__global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(BS == kBlock ? 7 : 4)))
+template <int BS, bool PUSH, bool DH, bool DEPOSIT, bool BATCH, bool GATHER, bool DENSE, bool COOP>
+__global__ void __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(COOP && BS == kBlock ? 7 : 4)))
 fempic_first_kernel(StepArgs P, uint32_t nblocks, int inline_hops, WorkList W) {
     int64_t n = P.ctr->size;
     n = n < 0 ? 0 : (n > P.n_max ? P.n_max : n);
@@ -518,7 +510,6 @@ fempic_first_kernel(StepArgs P, uint32_t nblocks, int inline_hops, WorkList W) {
     __shared__ unsigned s_order;  // deposits << 12 + new first nodes; from kKeep on: the table stays
     constexpr unsigned kKeep = 1u << 28;
     if (threadIdx.x == 0) s_pending = s_order = 0;  // a barrier comes before their first use
-    constexpr bool COOP = kCoop<BS, GATHER>;
     if constexpr (!COOP) __syncthreads();  // here, where no load is waited for yet
     const uint32_t b = xcd_block(blockIdx.x, nlive);
     int64_t i = (int64_t)b * BS + threadIdx.x;
@@ -1536,6 +1527,7 @@ void fold_slots(const StepArgs& P, hipStream_t s) {
     if (P.slots) slots_reduce_kernel<<<1, kSlots, 0, s>>>(P.slots, P.ctr);
 }
 
+constexpr int kLaneBlocks = 768;  // first-pass blocks up to which their lanes load cell records by themselves
 constexpr int kFewBlocks = 256;  // first-pass blocks up to which there is no walk pass
 
 // Two-pass move (first-hop pass + worklist walk) when the work buffer is large enough and the
@@ -1550,13 +1542,22 @@ bool launch_two_pass(const StepArgs& P, int64_t n_max, void* work, size_t work_b
     // the second read of lc and p2c. A copy fits a CU's LDS beside the rest up to 16,384 nodes.
     const bool dense = DEPOSIT && g_tuning.lanes == 1 && g_tuning.first_block == kBlock && P.n_nodes > 0 &&
                        P.n_nodes <= kDenseNodes && n_max >= 32 * P.n_nodes && n_max >= (1 << 18);
-    // A few blocks walk everything themselves and add their totals to the counters, one after the other in some 10 ns
-    // each: no walk pass, whose launch the smallest sets wait for. A fused step, us, with it and without: 1,000 particles
-    // 21.4 and 18.4, 4,000 22.8 and 19.3, 16,000 28.9 and 25.6, 32,000 35.3 and 31.8, 65,000 36.4 and 34.4, 130,000 (508
-    // blocks) 41 and 41. Not where the pass also clears the counters: its blocks' adds would race that.
+    // A few blocks walk everything themselves and add their totals to the counters, one after the other in some 10 ns each: no
+    // walk pass, whose launch the smallest sets wait for. A fused step, us, with it and without: 1,000 particles 21.4 and
+    // 18.4, 4,000 22.8 and 19.3, 16,000 28.9 and 25.6, 32,000 35.3 and 31.8, 65,000 36.4 and 34.4, 130,000 (508 blocks) 41 and
+    // 41. Where the pass also clears the counters its blocks' adds would race that, and the walk pass adds up their records.
     const int per_block = g_tuning.lanes == 4 ? kQuadParts : (g_tuning.first_block == kMaxBlock ? kMaxBlock : kBlock);
-    const bool alone = !P.reset && !dense && g_tuning.inline_hops >= 16 && n_max <= (int64_t)kFewBlocks * per_block;
-    const int inline_hops = alone ? OPPX_MAX_HOPS : g_tuning.inline_hops;
+    const bool far = !dense && g_tuning.inline_hops >= 16;
+    const bool few = far && n_max <= (int64_t)kFewBlocks * per_block, alone = few && !P.reset;
+    // Up to 768 blocks walk lane by lane: they wait for one evaluation after the other, 0.45 us each, where the cooperative
+    // fetch takes 0.95 and pays only once the loads of many waves queue. A pass without an overlay, us, cooperative / lane
+    // by lane / as it once was: 80,000 particles, walks of 2.6 evaluations at the mean 21.8 / 16.9 / 23.4, of 5.8 38 / 27 /
+    // 33, of 9.6 70 / 49 / 57; 160,000 of 5.8 42 / 35 / 42, of 9.6 78 / 61 / 69; 250,000 of 2.6 28.5 / 26.5 / 31.5, but in no
+    // order 75 / 79 / 92; 65,000 of which 0.1% walk 200 evaluations 128 / 84 / 96. (In larger sets such few long walks cost 10
+    // to 25% over lane-wise loads, and so do particles in no order on meshes past the L2s, 3 to 11%; blocks of 1024, in
+    // place, are the lane-wise form there.)
+    const bool lanewise = few || (far && per_block == kBlock && n_max <= (int64_t)kLaneBlocks * kBlock);
+    const int inline_hops = lanewise ? OPPX_MAX_HOPS : g_tuning.inline_hops;
     if (alone) W.rec = nullptr;
     unsigned g;
     if (g_tuning.lanes == 4) {
@@ -1564,17 +1565,34 @@ bool launch_two_pass(const StepArgs& P, int64_t n_max, void* work, size_t work_b
         g = grid_for(n_max, kQuadParts);
         fempic_quad_kernel<PUSH, DH, DEPOSIT, BATCH, GATHER><<<g, kQuadBlock, 0, s>>>(P, g, inline_hops, W);
     } else if (g_tuning.first_block == kMaxBlock) {
+        // Of the blocks of 1024 those that read through a permutation fetch together. The 16 buffers of such a block take 84
+        // KB, so that one fits a CU where two with lane-wise loads do (54 registers). In place that costs more than the
+        // fetch gains: 113 M particles of 256 instances, the move of a first / second step 7.14 / 7.07 ms with the fetch, 5.85 /
+        // 6.12 without, and 7.16 / 6.33 where it stages records; through a permutation, where the reads of the particles
+        // themselves are the longer wait, 8.98 with it and 9.58 without.
         W.parts = kMaxBlock;
         g = grid_for(n_max, kMaxBlock);
-        fempic_first_kernel<kMaxBlock, PUSH, DH, DEPOSIT, BATCH, GATHER, false>
-            <<<g, kMaxBlock, 0, s>>>(P, g, inline_hops, W);
+        if constexpr (GATHER) {
+            if (lanewise) fempic_first_kernel<kMaxBlock, PUSH, DH, DEPOSIT, BATCH, true, false, false>
+                              <<<g, kMaxBlock, 0, s>>>(P, g, inline_hops, W);
+            else fempic_first_kernel<kMaxBlock, PUSH, DH, DEPOSIT, BATCH, true, false, true>
+                     <<<g, kMaxBlock, 0, s>>>(P, g, inline_hops, W);
+        } else {
+            fempic_first_kernel<kMaxBlock, PUSH, DH, DEPOSIT, BATCH, false, false, false>
+                <<<g, kMaxBlock, 0, s>>>(P, g, inline_hops, W);
+        }
     } else {
         g = grid_for(n_max, kBlock);
-        auto first = fempic_first_kernel<kBlock, PUSH, DH, DEPOSIT, BATCH, GATHER, false>;
-        if constexpr (DEPOSIT) {
-            if (dense) first = fempic_first_kernel<kBlock, PUSH, DH, true, BATCH, GATHER, true>;
+        if (lanewise) {
+            fempic_first_kernel<kBlock, PUSH, DH, DEPOSIT, BATCH, GATHER, false, false>
+                <<<g, kBlock, 0, s>>>(P, g, inline_hops, W);
+        } else {
+            auto first = fempic_first_kernel<kBlock, PUSH, DH, DEPOSIT, BATCH, GATHER, false, true>;
+            if constexpr (DEPOSIT) {
+                if (dense) first = fempic_first_kernel<kBlock, PUSH, DH, true, BATCH, GATHER, true, true>;
+            }
+            first<<<g, kBlock, 0, s>>>(P, g, inline_hops, W);
         }
-        first<<<g, kBlock, 0, s>>>(P, g, inline_hops, W);
     }
     if (alone) return true;
     // A first pass that walks 16 evaluations itself hands over next to nothing: 256 records a walk block, at most
