@@ -106,7 +106,6 @@ struct BlockStat {
     int pending;  // worklist entries of the block; kScattered: none, and the walk pass deposits its particles
 };
 constexpr int kScattered = -1;
-constexpr uint32_t kAdders = 2 * kXcds;  // workgroups of a dense walk pass that add the records up: it has at least these
 
 // The block's totals, valid in thread 0 (ends with the other threads free to leave).
 __device__ __forceinline__ BlockStat block_totals(long long hsum, int hmax, int nrem, int nfault) {
@@ -971,10 +970,9 @@ __global__ void __launch_bounds__(kQuadBlock) fempic_quad_kernel(StepArgs P, uin
     }
 }
 
-// The walk pass: adds up the first pass's block records and walks its worklists to completion. A block takes
-// `per` first-pass blocks at a time, all of one XCD (first-pass block p ran on XCD p % 8), and walks their
-// entries as one dense list: 256 where the first pass walks (nearly) everything itself and the records are
-// all there is to read, few where it hands over many entries and the grid should spread them.
+// The walk pass: its first `adders` blocks add up the first pass's block records, and every block walks worklists of them to
+// completion. A block takes `per` first-pass blocks at a time, all of one XCD (first-pass block p ran on XCD p % 8), and
+// walks their entries as one dense list.
 // DENSE: it also deposits the particles of the first-pass blocks that found theirs scattered. A block then holds the
 // whole charge array in LDS, adds to it there, and adds it to the global one at its end, consecutive lanes to
 // consecutive nodes. Scattered adds to global memory go at 20 a nanosecond over the chip, such a sweep at 100, and LDS
@@ -985,7 +983,7 @@ __global__ void __launch_bounds__(kQuadBlock) fempic_quad_kernel(StepArgs P, uin
 // 950). A look ahead of every first chunk cost unordered sets 0.8 us a pass.
 template <bool DEPOSIT, bool DENSE>
 __global__ void __launch_bounds__(DENSE ? kMaxBlock : kBlock) fempic_walk_kernel(StepArgs P, WorkList W, uint32_t nblocks,
-                                                                                 int per) {
+                                                                                 int per, uint32_t adders) {
     constexpr int BT = DENSE ? kMaxBlock : kBlock;
     extern __shared__ double s_dense[];
     int64_t n = P.ctr->size;
@@ -1008,20 +1006,17 @@ __global__ void __launch_bounds__(DENSE ? kMaxBlock : kBlock) fempic_walk_kernel
         nrem += t.removed;
         nfault += t.faults;
     };
-    if constexpr (DENSE) {
-        if (blockIdx.x < kAdders)  // its chunks are many and small: a few blocks add up all the records
-            for (uint32_t q = blockIdx.x * BT + threadIdx.x; q < nlive; q += kAdders * BT) take(W.rec[q]);
-    } else {  // the records of the block's chunks, without a barrier between them
+    if (blockIdx.x < adders)
+        for (uint32_t q = blockIdx.x * BT + threadIdx.x; q < nlive; q += adders * BT) take(W.rec[q]);
+    if constexpr (!DENSE) {  // the records of the block's chunks, without a barrier between them
         int any = 0;
 #pragma unroll 4
         for (uint32_t c = blockIdx.x / kXcds; c < chunks; c += gridDim.x / kXcds) {
             if ((int)threadIdx.x >= per || c * (uint32_t)per + threadIdx.x >= mine) continue;
-            const BlockStat t = W.rec[x + kXcds * (c * (uint32_t)per + threadIdx.x)];
-            take(t);
-            any |= t.pending;
+            any |= W.rec[x + kXcds * (c * (uint32_t)per + threadIdx.x)].pending;
         }
         if (!__syncthreads_or(any)) {  // the usual case: nothing was handed over
-            block_stats(P, hsum, hmax, nrem, nfault);
+            if (blockIdx.x < adders) block_stats(P, hsum, hmax, nrem, nfault);
             return;
         }
     }
@@ -1595,27 +1590,30 @@ bool launch_two_pass(const StepArgs& P, int64_t n_max, void* work, size_t work_b
         }
     }
     if (alone) return true;
-    // A first pass that walks 16 evaluations itself hands over next to nothing: 256 records a walk block, at most
-    // 64 blocks (each adds to the one counters record; 94,000 records: 9.0 us, with 256 blocks 13.4). Below that the walk
-    // spreads over the resident grid. With dense deposits 8 records, 2048 particles, a block, one block a CU.
-    const bool rare = g_tuning.inline_hops >= 16;
-    const int per = rare && !dense ? kBlock : 8;
+    // The walk pass. Its first `adders` blocks add all the records up (each adds to the one counters record: 94,000 records 9.0
+    // us on 64 blocks, 13.4 on 256). The records are also dealt out evenly, for their worklists, over 512 blocks, as many as
+    // keep long walks from queueing behind each other (200,000 particles walking 96 evaluations each: 723 us, on 256 blocks
+    // 855, with 256 records a block and so 8 blocks 9,860; 1,024 and 2,048 no better), or over the resident grid where the
+    // first pass hands over walks of fewer than 16. With dense deposits 8 records, 2048 particles, a block at a time, one block
+    // a CU.
+    const uint32_t each = (g + kXcds - 1) / kXcds;  // first-pass blocks of an XCD
     const void* plain = reinterpret_cast<const void*>(fempic_walk_kernel<DEPOSIT, false>);
-    const unsigned cap = dense ? 256u : (rare ? 64u : resident_blocks(plain, kBlock));
-    unsigned wg = ((g + kXcds - 1) / kXcds + per - 1) / per * kXcds;  // every chunk of every XCD
+    const unsigned cap = dense ? 256u : (g_tuning.inline_hops >= 16 ? 512u : resident_blocks(plain, kBlock));
+    uint32_t per = dense ? 8u : (each * kXcds + cap - 1) / cap;
+    if (per > (uint32_t)kBlock) per = kBlock;
+    unsigned wg = (each + per - 1) / per * kXcds;  // every chunk of every XCD
     if (wg > cap) wg = cap / kXcds * kXcds;
-    const unsigned least = dense ? kAdders : (unsigned)kXcds;
-    if (wg < least) wg = least;
+    const uint32_t most = dense ? 2u * kXcds : 64u, adders = wg < most ? wg : most;
     if constexpr (DEPOSIT) {
         if (dense) {
             const size_t bytes = (size_t)P.n_nodes * sizeof(double);
             (void)hipFuncSetAttribute(reinterpret_cast<const void*>(fempic_walk_kernel<true, true>),
                                       hipFuncAttributeMaxDynamicSharedMemorySize, kDenseNodes * (int)sizeof(double));
-            fempic_walk_kernel<true, true><<<wg, kMaxBlock, bytes, s>>>(P, W, g, per);
+            fempic_walk_kernel<true, true><<<wg, kMaxBlock, bytes, s>>>(P, W, g, (int)per, adders);
             return true;
         }
     }
-    fempic_walk_kernel<DEPOSIT, false><<<wg, kBlock, 0, s>>>(P, W, g, per);
+    fempic_walk_kernel<DEPOSIT, false><<<wg, kBlock, 0, s>>>(P, W, g, (int)per, adders);
     return true;
 }
 
