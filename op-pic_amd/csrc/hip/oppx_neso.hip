@@ -12,7 +12,7 @@
 namespace oppx {
 namespace {
 
-// Threads per block. Every block adds to the one counters record at its end, and adds to one address from several
+// Threads per block at most. Every block adds to the one counters record at its end, and adds to one address from several
 // XCDs take some 10-20 ns each, one after the other: 2,048 blocks of 256 threads spent 20-40 us on that. Blocks of
 // 1024 make it 512: 1.5 M particles on the grid 61 -> 31 us, gathered 89 -> 64 us, 0.1 M gathered 18 -> 12.5 us.
 constexpr int kBlock = 1024;
@@ -144,19 +144,19 @@ __device__ __forceinline__ void neso_end(const NesoArgs& P, int64_t i, const Nes
 }
 
 // Resident grid, grid-stride over the particles, PER particles per lane per iteration, all loaded before any is
-// walked, so each lane keeps that many particles' loads in flight. Two where the walk computes its records (50
+// walked, so each lane keeps that many particles' loads in flight. Two where the walk computes its records in blocks of 1024 (50
 // VGPRs, two blocks per CU; four take 76 and one block: 32 M particles 549 and 685 us), one where it gathers them:
 // there the waves in flight are what hides a walk's chain of dependent reads (16 M particles on 1024 x 1024 cells
 // 1,021 us; two walks a lane advancing together 1,149, four 1,379).
-template <bool GRID>
-__global__ void __launch_bounds__(kBlock) neso_step_kernel(NesoArgs P, int flags) {
-    constexpr int PER = GRID ? 2 : 1;
+template <bool GRID, int BT>
+__global__ void __launch_bounds__(BT) neso_step_kernel(NesoArgs P, int flags) {
+    constexpr int PER = GRID && BT == kBlock ? 2 : 1;
     int64_t n = P.ctr->size;
     n = n < 0 ? 0 : (n > P.n_max ? P.n_max : n);
     long long hsum = 0;
     int hmax = 0, nfault = 0;
-    const int64_t stride = (int64_t)gridDim.x * kBlock;
-    for (int64_t i0 = (int64_t)blockIdx.x * kBlock + threadIdx.x; i0 < n; i0 += PER * stride) {
+    const int64_t stride = (int64_t)gridDim.x * BT;
+    for (int64_t i0 = (int64_t)blockIdx.x * BT + threadIdx.x; i0 < n; i0 += PER * stride) {
         NesoPart part[PER];
 #pragma unroll
         for (int u = 0; u < PER; u++) {
@@ -188,8 +188,8 @@ __global__ void __launch_bounds__(kBlock) neso_step_kernel(NesoArgs P, int flags
             nfault += w.fault ? 1 : 0;
         }
     }
-    __shared__ long long s_sum[kBlock / kWave];
-    __shared__ int s_max[kBlock / kWave], s_flt[kBlock / kWave];
+    __shared__ long long s_sum[BT / kWave];
+    __shared__ int s_max[BT / kWave], s_flt[BT / kWave];
     const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
     const long long hs = wave_sum_i64(hsum);
     const int hm = wave_max_i32(hmax), nf = wave_sum_i32(nfault);
@@ -198,9 +198,8 @@ __global__ void __launch_bounds__(kBlock) neso_step_kernel(NesoArgs P, int flags
     if (threadIdx.x == 0) {
         long long t = 0;
         int m = 0, f = 0;
-        for (int q = 0; q < kBlock / kWave; q++) { t += s_sum[q]; m = m > s_max[q] ? m : s_max[q]; f += s_flt[q]; }
+        for (int q = 0; q < BT / kWave; q++) { t += s_sum[q]; m = m > s_max[q] ? m : s_max[q]; f += s_flt[q]; }
         if (t) atomicAdd((unsigned long long*)&P.ctr->total_hops, (unsigned long long)t);
-        // the maximum only grows: a block whose own does not pass what it reads has nothing to add
         if (m) atomicMax(&P.ctr->max_hops, m);
         if (f) atomicAdd(&P.ctr->faults, f);
     }
@@ -280,11 +279,21 @@ int neso_step_impl(int64_t n_max, const oppx_neso_parts* parts, const oppx_quad_
     P.gnx = gnx;
     P.gny = gny;
     P.inv_gnx = grid ? 1.0 / gnx : 0.0;
-    auto kern = grid ? neso_step_kernel<true> : neso_step_kernel<false>;
-    unsigned g = resident_blocks(reinterpret_cast<const void*>(kern), kBlock);
-    const unsigned need = grid_for(n_max, kBlock);
+    // Smaller sets take smaller blocks, for a block of 1024 with one or two particles a thread leaves the CUs beside it idle.
+    // A step, us, blocks of 256 / 512 / 1024, records computed, then gathered from 490,000 cells at 4 cells a step: 1,000
+    // particles 8.3 8.5 9.8, 10.0 10.6 13.5; 10,000 8.3 8.7 10.2, 10.2 10.9 14.6; 23,000 9.7 9.2 10.6, 11.4 11.2 15.0; 50,000
+    // 12.1 10.3 11.0, 13.8 12.2 15.2; 100,000 17.1 12.7 12.2, 19.0 15.1 16.4. From 6 M particles on the grid is twice the
+    // resident blocks, four times where records are gathered, so that the last wave is a smaller share: 8.2 M in half-cell
+    // steps, resident / so 109 / 102, gathered 171 / 163, 32 M 391 / 374, 616 / 605; but 3 M 43 / 47, 67 / 74.
+    const int bt = n_max < 16'384 ? 256 : (n_max < 65'536 ? 512 : kBlock);
+    auto kern = bt == 256 ? (grid ? neso_step_kernel<true, 256> : neso_step_kernel<false, 256>)
+                          : bt == 512 ? (grid ? neso_step_kernel<true, 512> : neso_step_kernel<false, 512>)
+                                      : (grid ? neso_step_kernel<true, kBlock> : neso_step_kernel<false, kBlock>);
+    unsigned g = resident_blocks(reinterpret_cast<const void*>(kern), bt);
+    if (n_max >= 6'000'000) g *= grid ? 2 : 4;
+    const unsigned need = grid_for(n_max, bt);
     if (g > need) g = need;
-    kern<<<g, kBlock, 0, s>>>(P, flags);
+    kern<<<g, bt, 0, s>>>(P, flags);
     OPPX_LAUNCH_CHECK("neso_step");
     return OPPX_OK;
 }
