@@ -181,13 +181,14 @@ class FempicArena:
         self.slots_free = list(range(max_insts - 1, -1, -1))
         self.res = {}  # slot -> (template, cb, nb, ob)
         self.dropping = 0  # particles of retired requests still in the set (marked removed) until the next sort
-        # results of retired requests go to the host on their own stream, beside the next step: rows from engine_bytes on
-        # through the copy engine, which leaves the device to the step, shorter ones together in one kernel, where a copy
-        # each would cost its launch, on as many blocks as fill the link. A stream of 443 requests, some of 50 M particles:
-        # p99 step 36 ms and 2.7e9 particles/s with every row in the kernel, 16.5 ms and 3.0e9 so (17 ms from 256 KiB or
-        # 8 MiB on, 19 from 64 MiB); before there was a kernel for it, strided copies through a device temporary, 71 ms and
-        # 2.5e9 in the same run. 20 MB of small results 650 us on 32 blocks, 610 on all.
-        self.engine_bytes = 1 << 20
+        # results of retired requests go to the host on their own stream, beside the next step: rows from long_row_bytes on
+        # by the runtime's copy, one by one, shorter ones together in one kernel, where a copy each would cost its launch,
+        # on as many blocks as fill the link. A stream of 443 requests, some of 50 M particles: p99 step 36 ms and 2.7e9
+        # particles/s with every row in the kernel, which stays beside the step until the link has drained, 16.5 ms and
+        # 3.0e9 so (17 ms from 256 KiB or 8 MiB on, 19 from 64 MiB); before there was a kernel for it, strided copies
+        # through a device temporary, 71 ms and 2.5e9 in the same run. 20 MB of small results 650 us on 32 blocks, 610 on
+        # all.
+        self.long_row_bytes = 1 << 20
         self.link_blocks = 32
         self.copy_stream = torch.cuda.Stream(device=self.dev)
         self.cap, self.size = P, 0
@@ -309,11 +310,11 @@ class FempicArena:
 
     def _to_host(self, rows, stream):
         """(pinned array, device array, first, count): `count` elements from `first` on of every row, on `stream`.
-        Short rows go in one launch, long ones one by one through the copy engine."""
+        Short rows go in one launch, long ones one by one by the runtime's copy."""
         jobs = []
         for dst, src, first, count in rows:
             el = src.element_size()
-            if count * el < self.engine_bytes:
+            if count * el < self.long_row_bytes:
                 jobs.append(copy_job(dst.data_ptr(), src.data_ptr() + el * first, el * count, src.shape[0], el * count,
                                      el * src.stride(0)))
                 continue

@@ -1,4 +1,4 @@
-"""Both ways of a retired request's results to the host, the copy engine for long rows and one kernel for short ones: the
+"""Both ways of a retired request's results to the host, the runtime's copy for long rows and one kernel for short ones: the
 same bits whichever row takes which.
 
 Bar: results bit-exact against the same request stepped alone."""
@@ -13,12 +13,12 @@ pytestmark = pytest.mark.gpu
 STEPS = 2
 
 
-@pytest.mark.parametrize("engine_bytes", [0, 4000, 30_000, 1 << 62])  # all, most, some and no rows by the engine
-def test_long_and_short_rows_arrive_alike(engine_bytes):
+@pytest.mark.parametrize("long_row_bytes", [0, 4000, 30_000, 1 << 62])  # all, most, some and no rows by the runtime
+def test_long_and_short_rows_arrive_alike(long_row_bytes):
     tpls = make_templates([(3, 4000), (4, 9000), (2, 700), (2, 1)], seed=67)
     arena = serve.FempicArena(max_cells=5000, max_nodes=2000, max_particles=40000, max_overlay=10000, max_insts=4)
-    assert arena.engine_bytes == 1 << 20
-    arena.engine_bytes = engine_bytes
+    assert arena.long_row_bytes == 1 << 20
+    arena.long_row_bytes = long_row_bytes
     slots = [arena.admit(t) for t in tpls]
     for _ in range(STEPS):
         arena.step()
